@@ -47,7 +47,7 @@ namespace {
 using namespace dsp_mfma;
 
 constexpr int kLog2Unit = 4;   // 16 keys per work unit
-constexpr int kOcc = 3;        // waves per SIMD the kernel is compiled for
+constexpr int kOcc = 3;        // waves per SIMD the kernel is compiled for (two at D 256)
 constexpr int kMinUnits = 4;   // a worker gets at least this many units (64 keys)
 constexpr int kMaxBatch = 512; // every wave scans ctx_lens: the balanced split stops here
 
@@ -124,8 +124,11 @@ __device__ __forceinline__ int64_t active_workers(int64_t C, int num_workers) {
 // a worker is a workgroup of HG waves, wave i taking KV head HG*group + i of every piece,
 // so the waves of a workgroup read the same keys' rows side by side (HG x 256 bytes of
 // each 2 KiB slot row at D 128: the pool's DRAM pages are then read HG slices at a time).
-template <typename Tag, int D, bool kOff32, int HG>
-__global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(kOcc))) void decode_balanced_kernel(
+// kSplitP: the shapes that the generic kernel serves otherwise (D 256 and G > 8), whose
+// probabilities are fp32: they enter P.V as two 16-bit operands (pack8); and keys of a block id
+// outside the cache are masked, as they are there.
+template <typename Tag, int D, bool kOff32, int HG, bool kSplitP>
+__global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128 ? 2 : kOcc))) void decode_balanced_kernel(
     const uint16_t* __restrict__ q, int64_t qsb, int64_t qsh, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
     const int32_t* __restrict__ bt, int64_t bt_stride, int32_t log2_bs,
@@ -235,6 +238,18 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(kOcc)))
       cb1 = j + 1 < 64 ? __builtin_amdgcn_readlane(win, j + 1)
                        : __builtin_amdgcn_readlane(win2, j + 1 - 64);
     };
+    // kSplitP: the keys of the chunk's two 16-key halves below which block ids are valid (a
+    // half lies in one block; its slots inside the cache are a prefix of it).  Scalars.
+    int vlim[2] = {0, 0};
+    auto valid_limits = [&](int t0) {
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        const int key0 = t0 + 16 * st;
+        const int32_t blk = ((key0 >> log2_bs) != (t0 >> log2_bs)) ? cb1 : cb0;
+        const int64_t room = num_slots - int64_t(blk) * (bmask + 1) - (key0 & bmask);
+        vlim[st] = blk < 0 || room <= 0 ? 0 : key0 + static_cast<int>(room < 16 ? room : 16);
+      }
+    };
     // Element offset of `key` of the chunk starting at t0 in one layer's cache (head
     // included), -1 when its block id is out of range.
     auto elem_of = [&](int t0, int key) -> int64_t {
@@ -300,6 +315,7 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(kOcc)))
     // K before V, as inside the loop: the loop head then waits for K only (vmcnt(VINS)),
     // with this chunk's V still in flight, on entry and on every later iteration alike.
     chunk_blocks(kb);
+    if constexpr (kSplitP) valid_limits(kb);
     load_k(kb);
     load_v(kb);
     for (int t0 = kb; t0 < ke; t0 += 32) {
@@ -312,9 +328,11 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(kOcc)))
 #pragma unroll
         for (int kk = 0; kk < NKK; ++kk) sc[st] = mfma32<Tag>(kop[st][kk], qop[kk], sc[st]);
       }
+      const int cur[2] = {kSplitP ? min(lim, vlim[0]) : lim, kSplitP ? min(lim, vlim[1]) : lim};
       if (prefetch) {
         advance(tn);
         chunk_blocks(tn);
+        if constexpr (kSplitP) valid_limits(tn);
         load_k(tn);
       }
       // Scale and mask; lane holds keys t0 + 16*st + 4*grp + j of packed row n.
@@ -325,7 +343,7 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(kOcc)))
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int key = t0 + 16 * st + 4 * grp + j;
-          s[st][j] = (row_ok && key < lim) ? sc[st][j] * scale_log2 : -INFINITY;
+          s[st][j] = (row_ok && key < cur[st]) ? sc[st][j] * scale_log2 : -INFINITY;
           mx = fmaxf(mx, s[st][j]);
         }
       }
@@ -336,19 +354,19 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(kOcc)))
       const float alpha = dsp_exp2(m - m_use);
       m = m_new;
       float psum = 0.f;
-      uint16_t pb[8];
+      float p8[8];
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const float p = dsp_exp2(s[st][j] - m_use);
           psum += p;
-          pb[4 * st + j] = narrow<Tag>(p);
+          p8[4 * st + j] = p;
         }
       }
       lpart = lpart * alpha + psum;
-      const dsp_u32x4 pop = dsp_u32x4{pack2(pb[0], pb[1]), pack2(pb[2], pb[3]),
-                                      pack2(pb[4], pb[5]), pack2(pb[6], pb[7])};
+      dsp_u32x4 pop, plo;
+      pack8<Tag, kSplitP>(p8, pop, plo);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) acc[nt] *= alpha;
 
@@ -378,6 +396,7 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(kOcc)))
         const dsp_u32x4 vop = dsp_u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]),
                                         pack2(v[6], v[7])};
         acc[nt] = mfma32<Tag>(vop, pop, acc[nt]);
+        if constexpr (kSplitP) acc[nt] = mfma32<Tag>(vop, plo, acc[nt]);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -446,7 +465,7 @@ __global__ __launch_bounds__(256) void decode_balanced_combine_kernel(
     const int32_t* __restrict__ ctx_lens, const int32_t* __restrict__ cu_q, int32_t B,
     int32_t KVH, int32_t G, int32_t RPH, int32_t max_ctx, int32_t num_workers, int32_t HG,
     uint16_t* __restrict__ out, int64_t osb, int64_t osh, int32_t* __restrict__ err_count) {
-  constexpr int NV = D > 64 ? 2 : 1;  // dims per lane: lane, lane + 64
+  constexpr int NV = D > 64 ? D / 64 : 1;  // dims per lane: lane, lane + 64, ...
   constexpr int kInFlight = 16;       // pieces loaded per lane before they are folded in
   __shared__ float s_acc[4][NV * 64];
   __shared__ float s_ml[4][2];
@@ -561,12 +580,12 @@ __global__ __launch_bounds__(256) void decode_balanced_combine_kernel(
   }
 }
 
-template <typename Tag, int D, int HG>
-int launch_balanced_hg(int W, const uint16_t* q, int64_t qsb, int64_t qsh, const uint16_t* kc,
-                       const uint16_t* vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
+template <typename Tag, int D, int HG, bool kSplitP>
+int launch_balanced_hg(int W, int32_t KVH, const uint16_t* q, int64_t qsb, int64_t qsh,
+                       const uint16_t* kc, const uint16_t* vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
                        const int32_t* bt, int64_t bt_stride, int32_t log2_bs,
                        const int32_t* ctx_lens, const int32_t* cu_q, int32_t max_q_len,
-                       int32_t B, int32_t KVH, int32_t G, int32_t max_ctx, float scale_log2,
+                       int32_t B, int32_t G, int32_t max_ctx, float scale_log2,
                        float* ws_acc, float* ws_ml, uint16_t* out, int64_t osb, int64_t osh,
                        int32_t* err_count, hipStream_t s) {
   const int Wg = W / HG > 0 ? W / HG : 1;  // workgroups of HG waves
@@ -574,11 +593,11 @@ int launch_balanced_hg(int W, const uint16_t* q, int64_t qsb, int64_t qsh, const
   // largest element offset: last slot's last head's row end
   const bool off32 = num_slots * kvs_slot + KVH * kvs_head + D < (int64_t(1) << 31);
   if (off32)
-    decode_balanced_kernel<Tag, D, true, HG><<<dim3(static_cast<unsigned>(Wg)), 64 * HG, 0, s>>>(
+    decode_balanced_kernel<Tag, D, true, HG, kSplitP><<<dim3(static_cast<unsigned>(Wg)), 64 * HG, 0, s>>>(
         q, qsb, qsh, kc, vc, num_slots, kvs_slot, kvs_head, bt, bt_stride, log2_bs, ctx_lens,
         cu_q, B, KVH, G, RPH, max_ctx, scale_log2, Wg, ws_acc, ws_ml, out, osb, osh, err_count);
   else
-    decode_balanced_kernel<Tag, D, false, HG><<<dim3(static_cast<unsigned>(Wg)), 64 * HG, 0, s>>>(
+    decode_balanced_kernel<Tag, D, false, HG, kSplitP><<<dim3(static_cast<unsigned>(Wg)), 64 * HG, 0, s>>>(
         q, qsb, qsh, kc, vc, num_slots, kvs_slot, kvs_head, bt, bt_stride, log2_bs, ctx_lens,
         cu_q, B, KVH, G, RPH, max_ctx, scale_log2, Wg, ws_acc, ws_ml, out, osb, osh, err_count);
   const int st = dsp_launch_status();
@@ -589,44 +608,22 @@ int launch_balanced_hg(int W, const uint16_t* q, int64_t qsb, int64_t qsh, const
   return dsp_launch_status();
 }
 
-template <typename Tag, int D>
-int launch_balanced_d(int W, const uint16_t* q, int64_t qsb, int64_t qsh, const uint16_t* kc,
-                      const uint16_t* vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
-                      const int32_t* bt, int64_t bt_stride, int32_t log2_bs,
-                      const int32_t* ctx_lens, const int32_t* cu_q, int32_t max_q_len,
-                      int32_t B, int32_t KVH, int32_t G, int32_t max_ctx, float scale_log2,
-                      float* ws_acc, float* ws_ml, uint16_t* out, int64_t osb, int64_t osh,
-                      int32_t* err_count, hipStream_t s) {
+template <typename Tag, int D, bool kSplitP, typename... A>
+int launch_balanced_d(int W, int32_t KVH, A... args) {
   switch (dsp_detail::balanced_head_group(KVH)) {
-    case 8:
-      return launch_balanced_hg<Tag, D, 8>(W, q, qsb, qsh, kc, vc, num_slots, kvs_slot, kvs_head,
-                                           bt, bt_stride, log2_bs, ctx_lens, cu_q, max_q_len, B,
-                                           KVH, G, max_ctx, scale_log2, ws_acc, ws_ml, out, osb,
-                                           osh, err_count, s);
-    case 4:
-      return launch_balanced_hg<Tag, D, 4>(W, q, qsb, qsh, kc, vc, num_slots, kvs_slot, kvs_head,
-                                           bt, bt_stride, log2_bs, ctx_lens, cu_q, max_q_len, B,
-                                           KVH, G, max_ctx, scale_log2, ws_acc, ws_ml, out, osb,
-                                           osh, err_count, s);
-    case 2:
-      return launch_balanced_hg<Tag, D, 2>(W, q, qsb, qsh, kc, vc, num_slots, kvs_slot, kvs_head,
-                                           bt, bt_stride, log2_bs, ctx_lens, cu_q, max_q_len, B,
-                                           KVH, G, max_ctx, scale_log2, ws_acc, ws_ml, out, osb,
-                                           osh, err_count, s);
-    default:
-      return launch_balanced_hg<Tag, D, 1>(W, q, qsb, qsh, kc, vc, num_slots, kvs_slot, kvs_head,
-                                           bt, bt_stride, log2_bs, ctx_lens, cu_q, max_q_len, B,
-                                           KVH, G, max_ctx, scale_log2, ws_acc, ws_ml, out, osb,
-                                           osh, err_count, s);
+    case 4: return launch_balanced_hg<Tag, D, 4, kSplitP>(W, KVH, args...);
+    case 2: return launch_balanced_hg<Tag, D, 2, kSplitP>(W, KVH, args...);
+    default: return launch_balanced_hg<Tag, D, 1, kSplitP>(W, KVH, args...);
   }
 }
 
-template <typename Tag, typename... A>
+template <typename Tag, bool kSplitP, typename... A>
 int launch_balanced(int D, A... args) {
   switch (D) {
-    case 32: return launch_balanced_d<Tag, 32>(args...);
-    case 64: return launch_balanced_d<Tag, 64>(args...);
-    case 128: return launch_balanced_d<Tag, 128>(args...);
+    case 32: return launch_balanced_d<Tag, 32, kSplitP>(args...);
+    case 64: return launch_balanced_d<Tag, 64, kSplitP>(args...);
+    case 128: return launch_balanced_d<Tag, 128, kSplitP>(args...);
+    case 256: return launch_balanced_d<Tag, 256, true>(args...);
     default: return DSP_EUNSUPPORTED;
   }
 }
@@ -658,17 +655,33 @@ int balanced_head_group(int32_t KVH) {
   return KVH % 4 == 0 ? 4 : (KVH % 2 == 0 ? 2 : 1);
 }
 
-bool balanced_decode_applies(int32_t B, int32_t KVH, int32_t D, int32_t max_ctx,
-                             int32_t block_size) {
+namespace {
+
+bool balanced_batch_ok(int32_t B, int32_t KVH, int32_t max_ctx, int32_t block_size) {
   if (B < 1 || B > kMaxBatch || KVH < 1 || max_ctx < 1) return false;
   if (block_size < (1 << kLog2Unit)) return false;
-  if (D != 32 && D != 64 && D != 128) return false;
   // the unit scans (here and in the merge) add up 64 sequences' unit counts in 32-bit
   // lanes: at most 64 x (2^25 - 1) units, i.e. contexts below 2^29 - 15 tokens
   if (max_ctx > (1 << 29) - 16) return false;
   // w * C stays far inside int64 for every worker index w
   const int64_t cmax = int64_t(B) * KVH * ((int64_t(max_ctx) + 15) >> kLog2Unit);
   return cmax < (int64_t(1) << 40);
+}
+
+}  // namespace
+
+bool balanced_decode_applies(int32_t B, int32_t KVH, int32_t D, int32_t max_ctx,
+                             int32_t block_size) {
+  return (D == 32 || D == 64 || D == 128) && balanced_batch_ok(B, KVH, max_ctx, block_size);
+}
+
+bool balanced_wide_applies(int32_t B, int32_t KVH, int32_t G, int32_t D, int32_t max_ctx,
+                           int32_t block_size, size_t fixed_bytes) {
+  if (!(D == 32 || D == 64 || D == 128 || D == 256) || !(D == 256 || G > 8) || G > 16 ||
+      !balanced_batch_ok(B, KVH, max_ctx, block_size))
+    return false;
+  const size_t bytes = balanced_workspace_bytes(B, KVH, G, D, max_ctx);
+  return bytes <= DSP_NOALLOC_SCRATCH_BYTES || bytes <= fixed_bytes;
 }
 
 int32_t balanced_workers(int32_t B, int32_t KVH, int32_t max_ctx) {
@@ -701,16 +714,16 @@ int balanced_decode(const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h,
   const int32_t W = balanced_workers(B, KVH, max_ctx);
   float* ws_acc = workspace;
   float* ws_ml = ws_acc + (int64_t(B) * KVH + W) * max_q_len * G * D;
-  if (!f16)
-    return launch_balanced<Bf16Tag>(D, W, q, q_stride_b, q_stride_h, k_cache, v_cache,
-                                    num_slots, kv_stride_slot, kv_stride_head, block_table,
-                                    bt_stride, log2_bs, ctx_lens, cu_q, max_q_len, B, KVH, G,
-                                    max_ctx, scale_log2, ws_acc, ws_ml, out, o_stride_b,
-                                    o_stride_h, err_count, s);
-  return launch_balanced<F16Tag>(D, W, q, q_stride_b, q_stride_h, k_cache, v_cache, num_slots,
-                                 kv_stride_slot, kv_stride_head, block_table, bt_stride, log2_bs,
-                                 ctx_lens, cu_q, max_q_len, B, KVH, G, max_ctx, scale_log2,
-                                 ws_acc, ws_ml, out, o_stride_b, o_stride_h, err_count, s);
+  auto launch = [&](auto fn) {
+    return fn(D, W, KVH, q, q_stride_b, q_stride_h, k_cache, v_cache, num_slots, kv_stride_slot,
+              kv_stride_head, block_table, bt_stride, log2_bs, ctx_lens, cu_q, max_q_len, B, G,
+              max_ctx, scale_log2, ws_acc, ws_ml, out, o_stride_b, o_stride_h, err_count, s);
+  };
+  if (cu_q == nullptr && G > 8)  // decode of wide groups: fp32 probabilities
+    return f16 ? launch([](auto... a) { return launch_balanced<F16Tag, true>(a...); })
+               : launch([](auto... a) { return launch_balanced<Bf16Tag, true>(a...); });
+  return f16 ? launch([](auto... a) { return launch_balanced<F16Tag, false>(a...); })
+             : launch([](auto... a) { return launch_balanced<Bf16Tag, false>(a...); });
 }
 
 }  // namespace dsp_detail

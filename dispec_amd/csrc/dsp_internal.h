@@ -28,6 +28,12 @@ int mq_decode(const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h, const u
 // balanced_workspace_bytes(..., max_q_len * G, ...) long.
 bool balanced_decode_applies(int32_t B, int32_t KVH, int32_t D, int32_t max_ctx,
                              int32_t block_size);
+// The automatic split of a block-table decode of 256-wide heads or of 9 to 16 query heads per
+// KV head (never asked for explicitly): the same kernel, where its workspace fits the
+// no-allocation entry point's scratch or is no larger than the fixed partitions'
+// (fixed_bytes), so that every call that entry point took before it still takes.
+bool balanced_wide_applies(int32_t B, int32_t KVH, int32_t G, int32_t D, int32_t max_ctx,
+                           int32_t block_size, size_t fixed_bytes);
 int32_t balanced_workers(int32_t B, int32_t KVH, int32_t max_ctx);
 int balanced_head_group(int32_t KVH);
 size_t balanced_workspace_bytes(int32_t B, int32_t KVH, int32_t rows_per_head, int32_t D,

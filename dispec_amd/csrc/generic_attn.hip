@@ -1,5 +1,6 @@
-// J3 / J4 for the shapes the tuned attention kernels leave out: fp32 caches, head_dim 8 or
-// 256 (any power of two from 8 to 256), GQA groups above 8 on decode.  The reference's
+// J3 / J4 for the shapes the tuned attention kernels leave out: fp32 caches, head_dim 8 (any
+// power of two from 8 to 256), and 256-wide heads or GQA groups above 8 on decode where the
+// tuned kernels' 16-byte vectors are not aligned or the keys come from a slot table.  The reference's
 // Triton kernel takes any power-of-two HEAD_DIM and loads keys and values as fp32
 // (dispec/engine/triton_attn.py:60-95, tl.arange(0, HEAD_DIM) at :71); its native path
 // attends in whatever dtype the model runs (dispec/engine/model_runner.py:160-185).  These

@@ -375,7 +375,8 @@ void launch_combine(int D, dim3 grid, hipStream_t s, const float* ws_acc, const 
     case 16: decode_combine_kernel<Tag, 16><<<grid, 256, 0, s>>>(ws_acc, ws_ml, ctx_lens, max_ctx, P, num_parts, Hq, out, osb, osh); break;
     case 32: decode_combine_kernel<Tag, 32><<<grid, 256, 0, s>>>(ws_acc, ws_ml, ctx_lens, max_ctx, P, num_parts, Hq, out, osb, osh); break;
     case 64: decode_combine_kernel<Tag, 64><<<grid, 256, 0, s>>>(ws_acc, ws_ml, ctx_lens, max_ctx, P, num_parts, Hq, out, osb, osh); break;
-    default: decode_combine_kernel<Tag, 128><<<grid, 256, 0, s>>>(ws_acc, ws_ml, ctx_lens, max_ctx, P, num_parts, Hq, out, osb, osh); break;
+    case 128: decode_combine_kernel<Tag, 128><<<grid, 256, 0, s>>>(ws_acc, ws_ml, ctx_lens, max_ctx, P, num_parts, Hq, out, osb, osh); break;
+    default: decode_combine_kernel<Tag, 256><<<grid, 256, 0, s>>>(ws_acc, ws_ml, ctx_lens, max_ctx, P, num_parts, Hq, out, osb, osh); break;
   }
 }
 
@@ -495,6 +496,10 @@ extern "C" size_t dsp_paged_decode_workspace_bytes(int32_t B, int32_t Hq, int32_
     const size_t bal = dsp_detail::balanced_workspace_bytes(B, KVH, Hq / KVH, D, max_ctx);
     if (bal > need) need = bal;
   }
+  if (dsp_detail::balanced_wide_applies(B, KVH, Hq / KVH, D, max_ctx, 16, need)) {
+    const size_t bal = dsp_detail::balanced_workspace_bytes(B, KVH, Hq / KVH, D, max_ctx);
+    if (bal > need) need = bal;
+  }
   return need;
 }
 
@@ -545,6 +550,52 @@ extern "C" int dsp_paged_decode(const void* q, int64_t q_stride_b, int64_t q_str
     DSP_HOST_CHECK(workspace_bytes >= need && (need == 0 || workspace != nullptr),
                    DSP_EWORKSPACE);
     DSP_HOST_CHECK(need == 0 || dsp_aligned(workspace, 16), DSP_EALIGN);
+    // 16-bit caches of 32- to 256-wide heads on block tables, where the MFMA kernels' 16-byte
+    // vectors are aligned: the same kernels as below, 16 query heads to a row tile.
+    const bool vec16 = q_stride_b % 8 == 0 && q_stride_h % 8 == 0 && kv_stride_slot % 8 == 0 &&
+                       kv_stride_head % 8 == 0 && dsp_aligned(q, 16) && dsp_aligned(k_cache, 16) &&
+                       dsp_aligned(v_cache, 16);
+    if (dtype != DSP_F32 && block_table && vec16 && num_slots > 0 && max_ctx > 0 && P % 32 == 0 &&
+        (D == 32 || D == 64 || D == 128 || D == 256)) {
+      const float sl2 = scale * 1.4426950408889634f;
+      hipStream_t s = static_cast<hipStream_t>(stream);
+      const uint16_t* qh = static_cast<const uint16_t*>(q);
+      const uint16_t* kh = static_cast<const uint16_t*>(k_cache);
+      const uint16_t* vh = static_cast<const uint16_t*>(v_cache);
+      uint16_t* oh = static_cast<uint16_t*>(out);
+      const bool f16 = dtype == DSP_F16;
+      const int64_t tiles = (int64_t(G) + 15) / 16;
+      const bool one_round = partition_tokens == 0 && max_ctx <= kOneRoundCtx &&
+                             int64_t(B) * KVH * tiles <= 2 * int64_t(dsp_detail::device_cus());
+      const size_t bal = dsp_detail::balanced_workspace_bytes(B, KVH, G, D, max_ctx);
+      if (partition_tokens == 0 && !one_round && workspace_bytes >= bal && workspace != nullptr &&
+          dsp_aligned(workspace, 16) &&
+          dsp_detail::balanced_wide_applies(B, KVH, G, D, max_ctx, block_size, need))
+        return dsp_detail::balanced_decode(qh, q_stride_b, q_stride_h, kh, vh, num_slots,
+                                           kv_stride_slot, kv_stride_head, block_table, bt_stride,
+                                           lbs, ctx_lens, nullptr, 1, B, KVH, G, D, sl2, max_ctx,
+                                           static_cast<float*>(workspace), oh, o_stride_b,
+                                           o_stride_h, f16, err_count, s);
+      const int Pm = one_round ? (max_ctx + 127) / 128 * 128 : P;
+      const int np = (max_ctx + Pm - 1) / Pm;
+      float* wa = static_cast<float*>(workspace);
+      float* wm = np > 1 ? wa + int64_t(B) * Hq * np * D : nullptr;
+      if (np * tiles < (int64_t(1) << 31)) {
+        const int st = dsp_detail::mq_decode(qh, q_stride_b, q_stride_h, kh, vh, num_slots,
+                                             kv_stride_slot, kv_stride_head, block_table, bt_stride,
+                                             lbs, ctx_lens, B, KVH, G, D, sl2, max_ctx, Pm, np, wa,
+                                             wm, oh, o_stride_b, o_stride_h, f16, err_count, s);
+        if (st != DSP_OK || np <= 1) return st;
+        dim3 cg(static_cast<unsigned>((Hq + 3) / 4), static_cast<unsigned>(B));
+        if (!f16)
+          launch_combine<Bf16Tag>(D, cg, s, wa, wm, ctx_lens, max_ctx, Pm, np, Hq, oh, o_stride_b,
+                                  o_stride_h);
+        else
+          launch_combine<F16Tag>(D, cg, s, wa, wm, ctx_lens, max_ctx, Pm, np, Hq, oh, o_stride_b,
+                                 o_stride_h);
+        return dsp_launch_status();
+      }
+    }
     return dsp_detail::generic_attention(
         q, q_stride_b, q_stride_h, k_cache, v_cache, num_slots, kv_stride_slot, kv_stride_head,
         tbl, block_table ? bt_stride : st_stride, lbs, nullptr, ctx_lens, B, Hq, KVH, D, scale,

@@ -39,8 +39,11 @@ using namespace dsp_mfma;
 // semantics for bad lengths (a context past max_ctx is clamped and counted, an empty one
 // gives zeros) and its workspace layout ws[(b * Hq + h) * num_parts + part], which its
 // combine kernel merges.
-template <typename Tag, int D, bool kDecode>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) void paged_mq_kernel(
+// kSplitP: the shapes that the generic kernel serves otherwise (D 256, and decode with G > 8),
+// whose probabilities are fp32: they enter P.V as two 16-bit operands (pack8); and keys of a
+// block id outside the cache are masked, as they are there.
+template <typename Tag, int D, bool kDecode, bool kSplitP>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 128 ? 2 : 3))) void paged_mq_kernel(
     const uint16_t* __restrict__ q, int64_t qst, int64_t qsh, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
     const int32_t* __restrict__ bt, int64_t bt_stride, int32_t log2_bs,
@@ -77,7 +80,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
   bool bad = false;
   if (kDecode) {
     if (ctx > max_ctx || ctx < 0) {
-      if (threadIdx.x == 0 && part == 0 && kvh == 0 && err_count) atomicAdd(err_count, 1);
+      if (threadIdx.x == 0 && tile == 0 && part == 0 && kvh == 0 && err_count)
+        atomicAdd(err_count, 1);
       ctx = ctx < 0 ? 0 : max_ctx;
     }
   } else if (ctx > max_ctx || ctx < qlen) {
@@ -136,6 +140,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
   // caching them only evicts what other workgroups reuse (config-3 fixed-512 decode
   // 389.5 -> 357.6 us per layer on one box; nt K loads as well lose 4 % of that).
   dsp_u32x4 kop[2][NKK];
+  uint32_t bad_keys[2] = {0u, 0u};  // kSplitP: keys of each half whose block id is bad (uniform)
   char* const slab = slab_base + wave * SLAB;
   auto swz = [](int r, int c) { return c ^ ((2 * ((r >> 2) & 3)) & (CPR - 1)); };
   auto load_k = [&](int t0) {
@@ -144,6 +149,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
       const int key = t0 + 16 * st + n;
       const int64_t s = key < kfin ? slot_of(key) : -1;
       any_bad |= key < kfin && s < 0;
+      if constexpr (kSplitP) bad_keys[st] = uint32_t(__ballot(key < kfin && s < 0)) & 0xffffu;
 #pragma unroll
       for (int kk = 0; kk < NKK; ++kk)
         kop[st][kk] = s >= 0 ? *reinterpret_cast<const dsp_u32x4*>(kc + s * kvs_slot + head_off +
@@ -191,6 +197,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
 #pragma unroll
       for (int kk = 0; kk < NKK; ++kk) sc[st] = mfma32<Tag>(kop[st][kk], qop[kk], sc[st]);
     }
+    const uint32_t cur_bad[2] = {bad_keys[0], bad_keys[1]};
     if (prefetch) load_k(tn);
     // Scale and causal mask; lane holds keys t0 + 16*st + 4*grp + j of packed row n.
     float s[2][4];
@@ -200,7 +207,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int key = t0 + 16 * st + 4 * grp + j;
-        const bool ok = row_ok && key <= pos_q;
+        const bool ok = row_ok && key <= pos_q &&
+                        (!kSplitP || !((cur_bad[st] >> (4 * grp + j)) & 1u));
         s[st][j] = ok ? sc[st][j] * scale_log2 : -INFINITY;
         mx = fmaxf(mx, s[st][j]);
       }
@@ -212,19 +220,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
     const float alpha = dsp_exp2(m - m_use);
     m = m_new;
     float psum = 0.f;
-    uint16_t pb[8];
+    float p8[8];
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float p = dsp_exp2(s[st][j] - m_use);
         psum += p;
-        pb[4 * st + j] = narrow<Tag>(p);
+        p8[4 * st + j] = p;
       }
     }
     lpart = lpart * alpha + psum;
-    const dsp_u32x4 pop = dsp_u32x4{pack2(pb[0], pb[1]), pack2(pb[2], pb[3]), pack2(pb[4], pb[5]),
-                                 pack2(pb[6], pb[7])};
+    dsp_u32x4 pop, plo;
+    pack8<Tag, kSplitP>(p8, pop, plo);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) acc[nt] *= alpha;
 
@@ -251,6 +259,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
       const dsp_u32x4 vop = dsp_u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]),
                                    pack2(v[6], v[7])};
       acc[nt] = mfma32<Tag>(vop, pop, acc[nt]);
+      if constexpr (kSplitP) acc[nt] = mfma32<Tag>(vop, plo, acc[nt]);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -405,12 +414,13 @@ __global__ __launch_bounds__(256) void mq_combine_kernel(
   for (int e = 0; e < 4; ++e) o[e] = narrow<Tag>(A[e] * inv);
 }
 
-template <typename Tag, bool kDecode = false, typename... A>
+template <typename Tag, bool kDecode = false, bool kSplitP = false, typename... A>
 int launch_mq(int D, dim3 grid, hipStream_t s, A... args) {
   switch (D) {
-    case 32: paged_mq_kernel<Tag, 32, kDecode><<<grid, kThreads, 0, s>>>(args...); break;
-    case 64: paged_mq_kernel<Tag, 64, kDecode><<<grid, kThreads, 0, s>>>(args...); break;
-    case 128: paged_mq_kernel<Tag, 128, kDecode><<<grid, kThreads, 0, s>>>(args...); break;
+    case 32: paged_mq_kernel<Tag, 32, kDecode, kSplitP><<<grid, kThreads, 0, s>>>(args...); break;
+    case 64: paged_mq_kernel<Tag, 64, kDecode, kSplitP><<<grid, kThreads, 0, s>>>(args...); break;
+    case 128: paged_mq_kernel<Tag, 128, kDecode, kSplitP><<<grid, kThreads, 0, s>>>(args...); break;
+    case 256: paged_mq_kernel<Tag, 256, kDecode, true><<<grid, kThreads, 0, s>>>(args...); break;
     default: return DSP_EUNSUPPORTED;
   }
   return dsp_launch_status();
@@ -421,7 +431,8 @@ int launch_mq_combine(int D, dim3 grid, hipStream_t s, A... args) {
   switch (D) {
     case 32: mq_combine_kernel<Tag, 32><<<grid, 256, 0, s>>>(args...); break;
     case 64: mq_combine_kernel<Tag, 64><<<grid, 256, 0, s>>>(args...); break;
-    default: mq_combine_kernel<Tag, 128><<<grid, 256, 0, s>>>(args...); break;
+    case 128: mq_combine_kernel<Tag, 128><<<grid, 256, 0, s>>>(args...); break;
+    default: mq_combine_kernel<Tag, 256><<<grid, 256, 0, s>>>(args...); break;
   }
   return dsp_launch_status();
 }
@@ -441,19 +452,21 @@ int mq_decode(const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h, const u
               int32_t D, float scale_log2, int32_t max_ctx, int32_t P, int32_t num_parts,
               float* ws_acc, float* ws_ml, uint16_t* out, int64_t o_stride_b, int64_t o_stride_h,
               bool f16, int32_t* err_count, hipStream_t s) {
-  dim3 grid(static_cast<unsigned>(num_parts), static_cast<unsigned>(KVH), static_cast<unsigned>(B));
+  // 16 query heads per row tile (one tile up to G = 16)
+  dim3 grid(static_cast<unsigned>(num_parts * mq_tiles(1, G)), static_cast<unsigned>(KVH),
+            static_cast<unsigned>(B));
   const int32_t* no_cu = nullptr;
-  if (!f16)
-    return launch_mq<Bf16Tag, true>(D, grid, s, q, q_stride_b, q_stride_h, k_cache, v_cache,
-                                    num_slots, kv_stride_slot, kv_stride_head, block_table,
-                                    bt_stride, log2_bs, no_cu, ctx_lens, max_ctx, G, scale_log2, P,
-                                    num_parts, int32_t(1), ws_acc, ws_ml, out, o_stride_b,
-                                    o_stride_h, err_count);
-  return launch_mq<F16Tag, true>(D, grid, s, q, q_stride_b, q_stride_h, k_cache, v_cache,
-                                 num_slots, kv_stride_slot, kv_stride_head, block_table, bt_stride,
-                                 log2_bs, no_cu, ctx_lens, max_ctx, G, scale_log2, P, num_parts,
-                                 int32_t(1), ws_acc, ws_ml, out, o_stride_b, o_stride_h,
-                                 err_count);
+  auto launch = [&](auto fn) {
+    return fn(D, grid, s, q, q_stride_b, q_stride_h, k_cache, v_cache, num_slots, kv_stride_slot,
+              kv_stride_head, block_table, bt_stride, log2_bs, no_cu, ctx_lens, max_ctx, G,
+              scale_log2, P, num_parts, int32_t(1), ws_acc, ws_ml, out, o_stride_b, o_stride_h,
+              err_count);
+  };
+  if (G > 8)
+    return f16 ? launch([](auto... a) { return launch_mq<F16Tag, true, true>(a...); })
+               : launch([](auto... a) { return launch_mq<Bf16Tag, true, true>(a...); });
+  return f16 ? launch([](auto... a) { return launch_mq<F16Tag, true>(a...); })
+             : launch([](auto... a) { return launch_mq<Bf16Tag, true>(a...); });
 }
 
 }  // namespace dsp_detail
@@ -467,13 +480,15 @@ extern "C" int dsp_paged_mq_partition_tokens(int32_t B, int32_t Hq, int32_t KVH,
   // workgroup + a fixed cost) + the merge's cost per partition, in units of keys: a split
   // pays only when it fills a round of the machine that would otherwise idle.  Long query
   // blocks run on the 128-row prefill tile, two resident per CU at D 128 and four at D 64
-  // (LDS and registers); short ones (verify) on 16-row tiles, three per CU.  (Verify, 32
+  // (LDS and registers), one at D 256; short ones (verify) on 16-row tiles, three per CU (two
+  // at D 256).  (Verify, 32
   // sequences of ~2.3k tokens, Qwen3 heads: 62-65 us with 3 partitions, 68-71 with 7;
   // 64 sequences of 300-700 tokens: 29 us unsplit, 37-42 with 2-3 partitions.)
   const bool long_q = int64_t(max_q_len) * G >= 128;
   const int64_t base = int64_t(B) * KVH *
                        (long_q ? dsp_detail::prefill_tiles(max_q_len, G) : mq_tiles(max_q_len, G));
-  const int64_t slots = (long_q ? (D <= 64 ? 4 : 2) : 3) * int64_t(dsp_detail::device_cus());
+  const int per_cu = long_q ? (D <= 64 ? 4 : D <= 128 ? 2 : 1) : (D <= 128 ? 3 : 2);
+  const int64_t slots = per_cu * int64_t(dsp_detail::device_cus());
   if (base >= slots) return static_cast<int32_t>(whole);
   int64_t best_p = whole, best_cost = INT64_MAX;
   for (int n = 1; n <= kMaxParts; ++n) {
@@ -546,8 +561,17 @@ int mq_attention_impl(const void* q, int64_t q_stride_t, int64_t q_stride_h,
   DSP_HOST_CHECK(dtype == DSP_BF16 || dtype == DSP_F16 || dtype == DSP_F32, DSP_EUNSUPPORTED);
   DSP_HOST_CHECK(dsp_is_pow2(block_size), DSP_EINVAL);
   DSP_HOST_CHECK(bt_stride * block_size >= max_ctx, DSP_EINVAL);
-  if (dtype == DSP_F32 || !(D == 32 || D == 64 || D == 128)) {
-    // fp32 caches or head dims 8, 16, 256: the generic kernel, fixed partitions only
+  // 256-wide 16-bit heads run on the same tiles where the 16-byte vectors they load are
+  // aligned (4 x 200-token chunks of 16 heads over ~2000 keys: 85 us a layer, 13.1 ms on the
+  // generic kernel, which re-reads the keys for every row and head); the generic kernel, which
+  // needs element alignment only, keeps the rest.
+  const bool wide = D == 256 && dtype != DSP_F32 && prefix_tokens == 0 &&
+                    partition_tokens >= 0 && num_slots > 0 && q_stride_t % 8 == 0 &&
+                    q_stride_h % 8 == 0 && kv_stride_slot % 8 == 0 && kv_stride_head % 8 == 0 &&
+                    dsp_aligned(q, 16) && dsp_aligned(k_cache, 16) && dsp_aligned(v_cache, 16);
+  if (dtype == DSP_F32 || !(D == 32 || D == 64 || D == 128 || wide)) {
+    // fp32 caches or head dims 8 and 16 (and 256 unaligned): the generic kernel, fixed
+    // partitions only
     DSP_HOST_CHECK(dsp_detail::generic_head_dim(D) && prefix_tokens == 0 &&
                        partition_tokens != DSP_SPLIT_BALANCED,
                    DSP_EUNSUPPORTED);
@@ -639,7 +663,8 @@ int mq_attention_impl(const void* q, int64_t q_stride_t, int64_t q_stride_h,
                                            max_q_len, max_ctx, P, tm, prefix_tokens, ws_acc,
                                            ws_ml, oh, o_stride_t, o_stride_h, f16, err_count, s);
   } else if (dsp_detail::prefill_applies(D, block_size, int64_t(max_q_len) * G, num_slots,
-                                         kv_stride_slot)) {
+                                         kv_stride_slot) &&
+             (!wide || num_slots % block_size == 0)) {
     st = dsp_detail::prefill_attention(qh, q_stride_t, q_stride_h, kh, vh, num_slots,
                                        kv_stride_slot, kv_stride_head, block_table, bt_stride, lbs,
                                        cu_q, ctx_lens, B, KVH, G, D, scale_log2, max_q_len, max_ctx,

@@ -93,7 +93,7 @@ typedef __attribute__((address_space(3))) v4i16 lds_v4i16_t;
 // [part*P, part*P + P) again).  Both kinds run side by side; the merge then folds every
 // partition up to a row's last visible key, as for an unshared launch.
 template <typename Tag, int D, bool kShared>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void paged_prefill_kernel(
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2))) void paged_prefill_kernel(
     const uint16_t* __restrict__ q, int64_t qst, int64_t qsh, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
     const int32_t* __restrict__ bt, int64_t bt_stride, int32_t log2_bs,
@@ -112,6 +112,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   static_assert(LPW >= 1, "every wave loads part of a chunk");
   __shared__ __attribute__((aligned(1024))) char lds[2][2][SLAB];  // [buffer][K | V]
   __shared__ int32_t s_cu[kShared ? kMaxSharedSeqs + 1 : 1];         // cu_q, prefix pass
+  // D 256: which 16-key groups of each buffer's chunk have a block id outside the cache
+  // (their keys are masked, as on the generic kernel that serves unaligned 256-wide heads)
+  constexpr bool kMaskBad = D > 128;
+  __shared__ int32_t s_bad[2][kWaves];
+  // and its probabilities stay fp32, as that kernel's are: two 16-bit operands (pack8; one
+  // 16-bit operand would be 16 % faster and moves the error against 64 bits from 2.8e-3 to
+  // 3.3e-3).  128 KiB of LDS: one workgroup per CU, a wave's accumulators in AGPRs.
+  constexpr bool kSplitP = D > 128;
 
   // XCD-aware order: the dispatcher hands workgroup `lin` to XCD lin % 8.  Each XCD gets a
   // contiguous range of logical ids, so the tiles of one (sequence, KV head) -- which read
@@ -230,7 +238,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   // all 64 banks once.  Rows past kfin repeat the last key's row (finite data, masked);
   // an out-of-range slot reads slot 0.
   auto kswz = [](int row) { return row & (CPR - 1); };
-  auto vswz = [](int row) { return D == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1); };
+  auto vswz = [](int row) { return D >= 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1); };
   // Wave w loads rows 16*w .. 16*w + 15 of each chunk.  Chunks start at multiples of 64
   // keys and blocks hold a multiple of 16 tokens, so those rows lie in one block: its id
   // is wave-uniform and the addresses are a scalar base plus per-lane constants.  Rows past
@@ -251,15 +259,32 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   bool any_bad = false;  // (wave-uniform) a block id of visible keys lay outside the cache
   auto issue = [&](int buf, int t0, int32_t blk_v) {
     const int32_t blk = __builtin_amdgcn_readfirstlane(blk_v);
-    int64_t slot0 = int64_t(blk) * (bmask + 1) + ((t0 + 16 * wave) & bmask);
+    // D 256: rows past kfin repeat the last key's (the generic kernel reads no other slot)
+    const int first = kMaskBad ? min(t0 + 16 * wave, kfin - 1) : t0 + 16 * wave;
+    int64_t slot0 = int64_t(blk) * (bmask + 1) + (first & bmask);
     if (blk < 0 || (int64_t(blk) + 1) * (bmask + 1) > num_slots) {
       slot0 = 0;
       any_bad |= t0 + 16 * wave < kfin;
+      if constexpr (kMaskBad) s_bad[buf][wave] = 1;
+    } else if constexpr (kMaskBad) {
+      s_bad[buf][wave] = 0;
     }
     const int64_t e = slot0 * kvs_slot + head_off;
     const char* kb = reinterpret_cast<const char*>(kc + e);
     const char* vb = reinterpret_cast<const char*>(vc + e);
     const uint32_t m0 = lds_base + uint32_t(buf * 2 * SLAB + wave * LPW * 1024);
+    if constexpr (kMaskBad) {
+      if (t0 + kChunk > kfin) {
+#pragma unroll
+        for (int j = 0; j < LPW; ++j) {
+          const int rw = j * RPI + lane / CPR, row = 16 * wave + rw, sl = lane % CPR;
+          const uint32_t ro = uint32_t(min(rw, kfin - 1 - first) * kvs_slot * 2);
+          dma16<kShared>(kb, ro + 16 * (sl ^ kswz(row)), m0 + j * 1024);
+          dma16<kShared>(vb, ro + 16 * (sl ^ vswz(row)), m0 + SLAB + j * 1024);
+        }
+        return;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < LPW; ++j) {
       dma16<kShared>(kb, koff[j], m0 + j * 1024);
@@ -326,6 +351,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
           sc[mt][j] = key <= lim ? sc[mt][j] : -INFINITY;
         }
     }
+    if constexpr (kMaskBad) {
+      // sc[mt][j] lies in the chunk's 16-key group 2*mt + j/8, the rows one wave loaded
+      const int32_t* bad = s_bad[c & 1];
+#pragma unroll
+      for (int g16 = 0; g16 < 4; ++g16)
+        if (__builtin_amdgcn_readfirstlane(bad[g16])) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) sc[g16 >> 1][8 * (g16 & 1) + j] = -INFINITY;
+        }
+    }
     float mx = -INFINITY;
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
@@ -345,20 +380,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     const float neg_m = m == -INFINITY ? 0.f : -m;
     // P^T operands of the four 16-key steps: step ps = 2*mt + half takes registers
     // j = 8*half .. 8*half + 7, i.e. keys 16*ps + 4*hl + {0..3, 8..11}.
-    dsp_u32x4 pop[4];
+    dsp_u32x4 pop[4], plo[4];
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
-        uint16_t pb[8];
+        float p8[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          const float p = dsp_exp2(fmaf(sc[mt][8 * half + i], scale_log2, neg_m));
-          lpart += p;
-          pb[i] = narrow<Tag>(p);
+          p8[i] = dsp_exp2(fmaf(sc[mt][8 * half + i], scale_log2, neg_m));
+          lpart += p8[i];
         }
-        pop[2 * mt + half] = dsp_u32x4{pack2(pb[0], pb[1]), pack2(pb[2], pb[3]),
-                                       pack2(pb[4], pb[5]), pack2(pb[6], pb[7])};
+        pack8<Tag, kSplitP>(p8, pop[2 * mt + half], plo[2 * mt + half]);
       }
 
     // ---- O^T += V^T . P^T.  Per 16-key step ps the V^T operand is dim 32*dt + col, K index
@@ -379,6 +412,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
               vs_lds + kr * ROWB + 16 * ((dim0 >> 3) ^ vswz(kr)) + 2 * (dim0 & 7)));
         }
         acc[dt] = mfma32x32<Tag>(__builtin_bit_cast(dsp_u32x4, vh), pop[ps], acc[dt]);
+        if constexpr (kSplitP)
+          acc[dt] = mfma32x32<Tag>(__builtin_bit_cast(dsp_u32x4, vh), plo[ps], acc[dt]);
       }
     }
   }
@@ -433,6 +468,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 
 template <bool kShared, typename... A>
 int launch_prefill(int D, bool f16, dim3 grid, hipStream_t s, A... args) {
+  if constexpr (!kShared) {
+    if (D == 256) {
+      if (f16) paged_prefill_kernel<F16Tag, 256, false><<<grid, kThreads, 0, s>>>(args...);
+      else paged_prefill_kernel<Bf16Tag, 256, false><<<grid, kThreads, 0, s>>>(args...);
+      return dsp_launch_status();
+    }
+  }
   if (D == 128) {
     if (f16) paged_prefill_kernel<F16Tag, 128, kShared><<<grid, kThreads, 0, s>>>(args...);
     else paged_prefill_kernel<Bf16Tag, 128, kShared><<<grid, kThreads, 0, s>>>(args...);
@@ -449,7 +491,8 @@ namespace dsp_detail {
 
 bool prefill_applies(int32_t D, int32_t block_size, int64_t max_rows, int64_t num_slots,
                      int64_t kv_stride_slot) {
-  return (D == 64 || D == 128) && block_size >= 16 && max_rows >= kRows && num_slots >= 16 &&
+  return (D == 64 || D == 128 || D == 256) && block_size >= 16 && max_rows >= kRows &&
+         num_slots >= 16 &&
          kv_stride_slot < (int64_t(1) << 25);  // 16-row lane offsets fit 32 bits
 }
 

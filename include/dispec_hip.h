@@ -203,9 +203,10 @@ int dsp_kv_scatter_ordered(void* k_pool, void* v_pool, int64_t num_layers,
  *                  must hold dsp_paged_decode_workspace_bytes(..., partition_tokens)
  *                  bytes (16-byte aligned) for the same arguments, on the same device.
  * dtype: DSP_BF16, DSP_F16 or DSP_F32 (caches, q and out all of it).  The tuned kernels
- * serve bf16 / fp16 with D in {16, 32, 64, 128} and G = Hq / KVH in 1..8; every other
- * shape with D a power of two from 8 to 256 (fp32, D 8 or 256, G above 8) runs on a
- * generic kernel -- one wave per (sequence, query head, partition), fp32 accumulation,
+ * serve bf16 / fp16 with D in {16, 32, 64, 128} and G = Hq / KVH in 1..8, and on block tables
+ * with 16-byte-aligned rows D 256 and any G too (probabilities kept to fp32 accuracy there,
+ * in P.V as well); every other shape with D a power of two from 8 to 256 (fp32, D 8, slot
+ * tables or unaligned rows with D 256 or G above 8) runs on a generic kernel -- one wave per (sequence, query head, partition), fp32 accumulation,
  * element-aligned pointers -- whose automatic partition is dsp_paged_decode_partition_tokens
  * and whose workspace is covered by dsp_paged_decode_workspace_bytes.  Other D:
  * DSP_EUNSUPPORTED.
@@ -280,8 +281,8 @@ int dsp_paged_decode_noalloc(const void* q, int64_t q_stride_b, int64_t q_stride
  *                faster on fixed partitions.  Needs max_q_len * G <= 16, blocks of >= 16
  *                tokens, B <= 512, D in {32, 64, 128} (else DSP_EUNSUPPORTED) and always
  *                `workspace` (dsp_paged_mq_workspace_bytes with DSP_SPLIT_BALANCED).
- * dtype DSP_BF16 / DSP_F16 with D in {32, 64, 128} on the tuned kernels; DSP_F32, or D 8,
- * 16 or 256, on a generic kernel (one wave per query row, head and key partition; fixed
+ * dtype DSP_BF16 / DSP_F16 with D in {32, 64, 128}, or 256 with 16-byte-aligned rows, on the
+ * tuned kernels; DSP_F32, or D 8 or 16 (or 256 unaligned), on a generic kernel (one wave per query row, head and key partition; fixed
  * partitions only -- DSP_SPLIT_BALANCED and the shared-prefix entry return
  * DSP_EUNSUPPORTED for them); any G = Hq / KVH.  A sequence with q_len > ctx or
  * ctx > max_ctx is counted in err_count and its rows written as zeros.  A block id whose
