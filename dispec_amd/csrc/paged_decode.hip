@@ -468,6 +468,14 @@ extern "C" int dsp_paged_decode_partition_tokens(int32_t B, int32_t KVH, int32_t
 
 namespace {
 
+// A decode of 256-wide heads or more than 8 query heads per KV head that runs unsplit (the
+// automatic split): as for the other shapes, contexts of at most kOneRoundCtx keys and at most
+// two row tiles of 16 query heads per CU.
+bool wide_one_round(int32_t B, int32_t KVH, int32_t G, int32_t max_ctx) {
+  return max_ctx <= kOneRoundCtx && int64_t(B) * KVH * ((int64_t(G) + 15) / 16) <=
+                                        2 * int64_t(dsp_detail::device_cus());
+}
+
 size_t fixed_workspace_bytes(int32_t B, int32_t Hq, int32_t D, int32_t max_ctx, int32_t P) {
   if (P <= 0) return 0;  // no kernel for this head dim: the launch is rejected anyway
   const int64_t np = (int64_t(max_ctx) + P - 1) / P;
@@ -496,7 +504,8 @@ extern "C" size_t dsp_paged_decode_workspace_bytes(int32_t B, int32_t Hq, int32_
     const size_t bal = dsp_detail::balanced_workspace_bytes(B, KVH, Hq / KVH, D, max_ctx);
     if (bal > need) need = bal;
   }
-  if (dsp_detail::balanced_wide_applies(B, KVH, Hq / KVH, D, max_ctx, 16, need)) {
+  if (!wide_one_round(B, KVH, Hq / KVH, max_ctx) &&
+      dsp_detail::balanced_wide_applies(B, KVH, Hq / KVH, D, max_ctx, 16, need)) {
     const size_t bal = dsp_detail::balanced_workspace_bytes(B, KVH, Hq / KVH, D, max_ctx);
     if (bal > need) need = bal;
   }
@@ -565,8 +574,7 @@ extern "C" int dsp_paged_decode(const void* q, int64_t q_stride_b, int64_t q_str
       uint16_t* oh = static_cast<uint16_t*>(out);
       const bool f16 = dtype == DSP_F16;
       const int64_t tiles = (int64_t(G) + 15) / 16;
-      const bool one_round = partition_tokens == 0 && max_ctx <= kOneRoundCtx &&
-                             int64_t(B) * KVH * tiles <= 2 * int64_t(dsp_detail::device_cus());
+      const bool one_round = partition_tokens == 0 && wide_one_round(B, KVH, G, max_ctx);
       const size_t bal = dsp_detail::balanced_workspace_bytes(B, KVH, G, D, max_ctx);
       if (partition_tokens == 0 && !one_round && workspace_bytes >= bal && workspace != nullptr &&
           dsp_aligned(workspace, 16) &&
