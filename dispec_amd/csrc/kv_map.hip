@@ -23,6 +23,7 @@
 #include <math.h>
 
 #include "dsp_common.h"
+#include "dsp_internal.h"
 
 namespace {
 
@@ -244,13 +245,23 @@ __global__ __launch_bounds__(kThreads) void map_gemm_kernel(
 // banks.  Each output still accumulates over K in 32-wide MFMA steps in increasing k, the
 // same order as map_gemm_kernel, so the two kernels give bit-identical results.
 namespace big {
-constexpr int kBM = 256, kBN = 256, kBK = 64, kWN = 2, kNW = 8, kNT = 64 * kNW;
-constexpr int kCPR = kBK / 8;                // 16-byte chunks per tile row
-constexpr int kRowB = kBK * 2;               // bytes per tile row
-constexpr int kStageB = (kBM + kBN) * kRowB;
-constexpr int kLPW = (kBM + kBN) * kCPR / 64 / kNW;  // 1-KiB DMA loads per wave per stage
-constexpr int kTM = 64, kTN = 128, kFM = kTM / 16, kFN = kTN / 16, kKS = kBK / 32;
-static_assert(kBM * kCPR % (64 * kLPW) == 0, "a wave loads rows of one operand only");
+constexpr int kBK = 64;                       // K per stage
+constexpr int kCPR = kBK / 8;                 // 16-byte chunks per tile row
+constexpr int kRowB = kBK * 2;                // bytes per tile row
+constexpr int kKS = kBK / 32;
+constexpr int kTN = 128, kFN = kTN / 16;      // a wave's columns: whole heads of 64 or 128
+// A BM x BN tile: WM waves down, BN / 128 across.
+template <int BM, int BN, int WM>
+struct Tile {
+  static constexpr int kBM = BM, kBN = BN, kWN = BN / kTN, kNW = WM * kWN, kNT = 64 * kNW;
+  static constexpr int kStageB = (BM + BN) * kRowB;
+  static constexpr int kLPW = (BM + BN) * kCPR / 64 / kNW;  // 1-KiB DMA loads per wave per stage
+  static constexpr int kTM = BM / WM, kFM = kTM / 16;
+  static_assert(BM * kCPR % (64 * kLPW) == 0, "a wave loads rows of one operand only");
+};
+using Large = Tile<256, 256, 4>;  // 8 waves of 64 x 128, 128 KiB of LDS: one workgroup per CU
+using Small = Tile<128, 128, 4>;  // 4 waves of 32 x 128, 64 KiB: two per CU
+constexpr int kBM = Large::kBM, kBN = Large::kBN, kNT = Large::kNT;
 }  // namespace big
 
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -284,73 +295,66 @@ __device__ __forceinline__ float rope_apply1(float x, float x_partner, float c, 
 
 // The epilogue flags are template parameters: with all three variants compiled into one
 // body the epilogue's live ranges push the kernel past 256 VGPRs.  kRope / kPool: the
-// fused target-RoPE and pool-scatter epilogue of dsp_kv_map_gemm_to_pool.
-template <int kBias, int kAct, int kAccum, int kRope = 0, int kPool = 0>
-__global__ __launch_bounds__(big::kNT) void map_gemm_big_kernel(
-    const uint16_t* __restrict__ a, SegOffsets a_seg, int64_t a_seg_len, int64_t lda,
+// target-RoPE and pool-scatter epilogues of dsp_kv_map_gemm_to_pool and dsp_kv_map_group
+// (kRope 2: rotate when `rotate` says so, workgroup-uniform).
+//
+// One output tile (rows m0.., columns n0..) of one problem.  seg(i) is the first row of
+// segment i of the design rows; bt / bias / c are the problem's; block_table its row of the
+// pool's table (kPool).
+template <typename TL, int kBias, int kAct, int kAccum, int kRope, int kPool, typename Seg>
+__device__ __forceinline__ void map_tile(
+    char* __restrict__ lds, Seg seg, int64_t a_seg_len, int64_t lda,
     const uint16_t* __restrict__ bt, int64_t ldb, uint16_t* __restrict__ c, int64_t ldc,
-    int64_t M, int64_t N, int64_t K, const uint16_t* __restrict__ bias,
-    int64_t a_batch_stride, int64_t c_batch_stride, PoolOut po = PoolOut()) {
-  __shared__ __attribute__((aligned(1024))) char lds[2 * big::kStageB];
-  // 1-D grid over (batch, m tile, n tile), n fastest.  Workgroup ids are dealt to the 8
-  // XCDs round-robin; remap so each XCD gets a contiguous run of tiles and the n tiles
-  // sharing one A row block run on the same L2.
-  const int tn = int((N + big::kBN - 1) / big::kBN), tm = int((M + big::kBM - 1) / big::kBM);
-  int t = int(blockIdx.x);
-  const int full = int(gridDim.x) & ~7;
-  if (t < full) t = (t & 7) * (full >> 3) + (t >> 3);
-  const int bx = t % tn, by = (t / tn) % tm, bz = t / (tn * tm);
-  a += int64_t(bz) * a_batch_stride;
-  if (!kPool) c += int64_t(bz) * c_batch_stride;
+    int64_t M, int64_t N, int64_t K, const uint16_t* __restrict__ bias, int64_t m0, int64_t n0,
+    const int32_t* __restrict__ block_table, const PoolOut& po, bool rotate) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t m0 = int64_t(by) * big::kBM, n0 = int64_t(bx) * big::kBN;
 
   // This wave's loads: instruction j covers tile rows 8 * (wave * kLPW + j) .. +7 (A rows
   // for waves 0-3, Bt rows for waves 4-7); lane l fills slot l % 8 of row l / 8, i.e.
   // chunk (l % 8) ^ (row & 7).  Rows past M / N are clamped to the last row (their outputs are
   // never stored).  Element offsets fit 32 bits (checked on the host).
-  const bool loads_a = wave * big::kLPW * 64 < big::kBM * big::kCPR;
-  uint32_t off[big::kLPW];
+  const bool loads_a = wave * TL::kLPW * 64 < TL::kBM * big::kCPR;
+  uint32_t off[TL::kLPW];
 #pragma unroll
-  for (int j = 0; j < big::kLPW; ++j) {
-    const int r = (wave * big::kLPW + j) * (64 / big::kCPR) + lane / big::kCPR;
+  for (int j = 0; j < TL::kLPW; ++j) {
+    const int r = (wave * TL::kLPW + j) * (64 / big::kCPR) + lane / big::kCPR;
     const int chunk = (lane % big::kCPR) ^ (r & 7);
-    const int64_t row = loads_a ? min<int64_t>(m0 + r, M - 1) : min<int64_t>(n0 + r - big::kBM, N - 1);
+    const int64_t row = loads_a ? min<int64_t>(m0 + r, M - 1) : min<int64_t>(n0 + r - TL::kBM, N - 1);
     off[j] = uint32_t(row * (loads_a ? lda : ldb) + chunk * 8);
   }
   // Stages are issued in order; the A source (segment seg_i, column seg_k inside it) is
   // advanced incrementally, so a segment offset is fetched once per segment boundary
   // rather than divided out and loaded at every stage (a stage never straddles segments).
   int64_t seg_i = 0, seg_k = 0;
-  const uint16_t* a_src = a + a_seg.off[0];
+  const uint16_t* a_src = seg(0);
   auto issue = [&](int buf, int64_t k0) {
     const uint16_t* src = loads_a ? a_src + seg_k : bt + k0;
-    char* dst = lds + buf * big::kStageB + wave * big::kLPW * 1024;
+    char* dst = lds + buf * TL::kStageB + wave * TL::kLPW * 1024;
 #pragma unroll
-    for (int j = 0; j < big::kLPW; ++j)
+    for (int j = 0; j < TL::kLPW; ++j)
       __builtin_amdgcn_global_load_lds(static_cast<const void*>(src + off[j]),
                                        (lds_void_t*)(dst + j * 1024), 16, 0, 0);
     seg_k += big::kBK;
     if (seg_k == a_seg_len && k0 + big::kBK < K) {
       seg_k = 0;
-      a_src = a + a_seg.get(++seg_i);
+      a_src = seg(++seg_i);
     }
   };
 
-  f32x4 acc[big::kFM][big::kFN];
+  f32x4 acc[TL::kFM][big::kFN];
 #pragma unroll
-  for (int i = 0; i < big::kFM; ++i)
+  for (int i = 0; i < TL::kFM; ++i)
 #pragma unroll
     for (int j = 0; j < big::kFN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int wm = (wave / big::kWN) * big::kTM, wn = (wave % big::kWN) * big::kTN;
+  const int wm = (wave / TL::kWN) * TL::kTM, wn = (wave % TL::kWN) * big::kTN;
   const int fr = lane & 15, fq = lane >> 4;
-  dsp_u32x4 fa[2][big::kFM], fb[2][big::kFN];
+  dsp_u32x4 fa[2][TL::kFM], fb[2][big::kFN];
   auto read_frags = [&](const char* sa, int ks, int slot) {
-    const char* sb = sa + big::kBM * big::kRowB;
+    const char* sb = sa + TL::kBM * big::kRowB;
     const int chunk = ks * 4 + fq;
 #pragma unroll
-    for (int i = 0; i < big::kFM; ++i) {
+    for (int i = 0; i < TL::kFM; ++i) {
       const int r = wm + 16 * i + fr;
       fa[slot][i] = *reinterpret_cast<const dsp_u32x4*>(sa + r * big::kRowB + ((chunk ^ (r & 7)) * 16));
     }
@@ -368,14 +372,14 @@ __global__ __launch_bounds__(big::kNT) void map_gemm_big_kernel(
     // whose buffer the next DMA overwrites
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
-    const char* sa = lds + (kt & 1) * big::kStageB;
+    const char* sa = lds + (kt & 1) * TL::kStageB;
     read_frags(sa, 0, 0);
     if (kt + 1 < nk) issue((kt + 1) & 1, int64_t(kt + 1) * big::kBK);
 #pragma unroll
     for (int ks = 0; ks < big::kKS; ++ks) {
       if (ks + 1 < big::kKS) read_frags(sa, ks + 1, (ks + 1) & 1);
 #pragma unroll
-      for (int i = 0; i < big::kFM; ++i)
+      for (int i = 0; i < TL::kFM; ++i)
 #pragma unroll
         for (int j = 0; j < big::kFN; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fb[ks & 1][j]),
@@ -384,11 +388,11 @@ __global__ __launch_bounds__(big::kNT) void map_gemm_big_kernel(
       if (ks + 1 < big::kKS) {
         // issue the next slice's fragment reads between this slice's MFMAs
 #pragma unroll
-        for (int q = 0; q < big::kFM + big::kFN; ++q) {
+        for (int q = 0; q < TL::kFM + big::kFN; ++q) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
           __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, big::kFM * big::kFN - (big::kFM + big::kFN), 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, TL::kFM * big::kFN - (TL::kFM + big::kFN), 0);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -404,16 +408,16 @@ __global__ __launch_bounds__(big::kNT) void map_gemm_big_kernel(
   // back four whole rows per instruction, so C is written in full 256-byte row runs with
   // 16-byte lanes -- half the store instructions, every cache line written whole -- with
   // non-temporal stores (same-box A/B, config 5: 73.4-74.7 against 75.7-76.8 us a launch).
-  static_assert(big::kNW * big::kTM * big::kTN * 2 <= 2 * big::kStageB, "C tile fits the stages");
+  static_assert(TL::kNW * TL::kTM * big::kTN * 2 <= 2 * TL::kStageB, "C tile fits the stages");
   float b4[big::kFN][4] = {};
   if (kBias) {
 #pragma unroll
     for (int j = 0; j < big::kFN; ++j) load_bias4(bias, n0 + wn + 16 * j + 4 * fq, N, b4[j]);
   }
   __syncthreads();   // every wave is done reading the last stage
-  char* ct = lds + wave * (big::kTM * big::kTN * 2);
+  char* ct = lds + wave * (TL::kTM * big::kTN * 2);
 #pragma unroll
-  for (int i = 0; i < big::kFM; ++i) {
+  for (int i = 0; i < TL::kFM; ++i) {
     const int r = 16 * i + fr;
 #pragma unroll
     for (int j = 0; j < big::kFN; ++j) {
@@ -432,14 +436,13 @@ __global__ __launch_bounds__(big::kNT) void map_gemm_big_kernel(
   const int64_t n = n0 + wn + 8 * cl;
   const bool vec_c = n + 7 < N;
   // kPool: the pool slot of each of this lane's 16 rows (loads issued together)
-  int64_t slot_q[kPool ? big::kTM / 4 : 1];
+  int64_t slot_q[kPool ? TL::kTM / 4 : 1];
   if constexpr (kPool) {
-    const int32_t* btz = po.block_tables + int64_t(bz) * po.bt_stride;
     const int bmask = (1 << po.log2_bs) - 1;
 #pragma unroll
-    for (int q = 0; q < big::kTM / 4; ++q) {
+    for (int q = 0; q < TL::kTM / 4; ++q) {
       const int64_t m = min<int64_t>(m0 + wm + 4 * q + (lane >> 4), M - 1);
-      slot_q[q] = (int64_t(btz[m >> po.log2_bs]) << po.log2_bs) | (m & bmask);
+      slot_q[q] = (int64_t(block_table[m >> po.log2_bs]) << po.log2_bs) | (m & bmask);
     }
   }
   // kRope: this lane's 8 columns are dims d0 .. d0 + 7 of one head; the partner chunk (half
@@ -449,7 +452,7 @@ __global__ __launch_bounds__(big::kNT) void map_gemm_big_kernel(
   const bool first_half = d0 < hd / 2;
   const int pcl = cl ^ (hd / 16);
 #pragma unroll
-  for (int q = 0; q < big::kTM / 4; ++q) {
+  for (int q = 0; q < TL::kTM / 4; ++q) {
     const int r = 4 * q + (lane >> 4);
     // r & 8 is bit 1 of q for every lane (r = 4q + 0..3): a fixed register swap
     const bool swapped = (q >> 1) & 1;
@@ -460,7 +463,7 @@ __global__ __launch_bounds__(big::kNT) void map_gemm_big_kernel(
         *reinterpret_cast<const dsp_u32x4*>(ct + r * (big::kTN * 2) + ((cl ^ (r & 15)) * 16)));
     const int64_t m = m0 + wm + r;
     if (m >= M) continue;
-    if constexpr (kRope) {
+    if (kRope == 1 || (kRope == 2 && rotate)) {
       const dsp_u32x4 vp = unswap(
           *reinterpret_cast<const dsp_u32x4*>(ct + r * (big::kTN * 2) + ((pcl ^ (r & 15)) * 16)));
       const float* cr = po.rope_cos + m * hd + d0;
@@ -514,10 +517,76 @@ __global__ __launch_bounds__(big::kNT) void map_gemm_big_kernel(
   }
 }
 
+// Workgroup ids are dealt to the 8 XCDs round-robin; remap so each XCD gets a contiguous run
+// of tiles and the n tiles sharing one A row block run on the same L2.
+__device__ __forceinline__ int xcd_tile() {
+  int t = int(blockIdx.x);
+  const int full = int(gridDim.x) & ~7;
+  if (t < full) t = (t & 7) * (full >> 3) + (t >> 3);
+  return t;
+}
+
+// One problem (or a batch sharing its weight): 1-D grid over (batch, m tile, n tile), n fastest.
+template <int kBias, int kAct, int kAccum, int kRope = 0, int kPool = 0>
+__global__ __launch_bounds__(big::kNT) void map_gemm_big_kernel(
+    const uint16_t* __restrict__ a, SegOffsets a_seg, int64_t a_seg_len, int64_t lda,
+    const uint16_t* __restrict__ bt, int64_t ldb, uint16_t* __restrict__ c, int64_t ldc,
+    int64_t M, int64_t N, int64_t K, const uint16_t* __restrict__ bias,
+    int64_t a_batch_stride, int64_t c_batch_stride, PoolOut po = PoolOut()) {
+  using TL = big::Large;
+  __shared__ __attribute__((aligned(1024))) char lds[2 * TL::kStageB];
+  const int tn = int((N + TL::kBN - 1) / TL::kBN), tm = int((M + TL::kBM - 1) / TL::kBM);
+  const int t = xcd_tile();
+  const int bx = t % tn, by = (t / tn) % tm, bz = t / (tn * tm);
+  a += int64_t(bz) * a_batch_stride;
+  if (!kPool) c += int64_t(bz) * c_batch_stride;
+  map_tile<TL, kBias, kAct, kAccum, kRope, kPool>(
+      lds, [&](int64_t i) { return a + a_seg.get(i); }, a_seg_len, lda, bt, ldb, c, ldc, M, N, K,
+      bias, int64_t(by) * TL::kBM, int64_t(bx) * TL::kBN,
+      kPool ? po.block_tables + int64_t(bz) * po.bt_stride : nullptr, po, true);
+}
+
+// Many maps in one launch (dsp_kv_map_group): the layers' key and value maps of one prompt.
+constexpr int kMaxGroup = 80;  // 40 bytes an entry: the kernel arguments stay below 4 KiB
+struct GroupEntry {
+  const uint16_t* bt;
+  const uint16_t* bias;
+  uint16_t seg[kMaxSegments];  // source layers of the design row
+  uint16_t layer, values;      // target layer; 0 keys, 1 values
+};
+struct GroupArgs {
+  GroupEntry e[kMaxGroup];
+  const uint16_t* a[2];        // source layers of keys, of values
+  uint16_t* c[2];              // target layers
+  int64_t a_layer_stride, c_layer_stride;
+};
+
+// 1-D grid over (map, m tile, n tile), n fastest: a prompt of a few hundred tokens has 4 to 16
+// tiles per map, so one map alone leaves most of the chip idle.  72 maps of 1023 tokens: 2420
+// -> 215 us in 72 launches and one; of 4095 tokens (fused rotation and pool rows) 2520 -> 850.
+template <typename TL, int kRope, int kPool>
+__global__ __launch_bounds__(TL::kNT) void map_group_kernel(GroupArgs g, int64_t seg_len, int64_t ldc,
+                                                            int64_t M, int64_t N, int64_t K,
+                                                            PoolOut po) {
+  __shared__ __attribute__((aligned(1024))) char lds[2 * TL::kStageB];
+  const int tn = int((N + TL::kBN - 1) / TL::kBN), tm = int((M + TL::kBM - 1) / TL::kBM);
+  const int t = xcd_tile();
+  const int bx = t % tn, by = (t / tn) % tm, z = t / (tn * tm);
+  const GroupEntry& e = g.e[z];
+  const int kind = e.values;
+  const uint16_t* a = kind ? g.a[1] : g.a[0];
+  uint16_t* c = (kind ? g.c[1] : g.c[0]) + int64_t(e.layer) * g.c_layer_stride;
+  map_tile<TL, 1, 0, 0, kRope ? 2 : 0, kPool>(
+      lds, [&](int64_t i) { return a + int64_t(e.seg[i]) * g.a_layer_stride; }, seg_len, seg_len,
+      e.bt, K, c, ldc, M, N, K, e.bias, int64_t(by) * TL::kBM, int64_t(bx) * TL::kBN,
+      po.block_tables, po, kind == 0);
+}
+
 // RoPE on (L, T, H, D) rows in fp32: out = x*cos + sign*rot(x)*sin, with
 // rot(x) = cat(-x2, x1) over the two halves of head_dim (transfer.py:61-80: sign -1
 // strips, +1 applies).  Input bf16 or fp32; output fp32, or bf16 rounded to nearest
-// even.  One thread per pair (d, d + D/2) of one head of one token of one layer.
+// even.  One thread per pair (d, d + D/2) of one head of one token of one layer: the general
+// form (any even D, element alignment).
 template <typename TI, typename TO>
 __global__ __launch_bounds__(256) void rope_kernel(const TI* __restrict__ x, TO* __restrict__ y,
                                                    int64_t L, int64_t T, int64_t H, int64_t D,
@@ -552,6 +621,76 @@ __global__ __launch_bounds__(256) void rope_kernel(const TI* __restrict__ x, TO*
   const float o2 = x2 * c2 + sign * (x1 * s2);
   y[yo + d] = st(o1);
   y[yo + d + half] = st(o2);
+}
+
+// The same for rows whose halves are whole 16-byte vectors (D a multiple of 16, 16-byte aligned
+// rows): one thread per 8 elements of the first half and their 8 partners, grid y the layer.
+// Memory-bound: x is read and y written once, the tables stay in the caches.  28 layers of
+// 4095 tokens x 1024 in bf16: 209 us with one thread per pair and 2-byte accesses, 76 us (6.2
+// TB/s, a copy's rate) in this form.
+template <typename T>
+__device__ __forceinline__ void load8(const T* __restrict__ p, float (&f)[8]) {
+  if constexpr (sizeof(T) == 2) {
+    const dsp_u32x4 u = *reinterpret_cast<const dsp_u32x4*>(p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f[2 * i] = dsp_bf16lo(u[i]);
+      f[2 * i + 1] = dsp_bf16hi(u[i]);
+    }
+  } else {
+    const f32x4 u = *reinterpret_cast<const f32x4*>(p), w = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f[i] = u[i];
+      f[4 + i] = w[i];
+    }
+  }
+}
+template <typename T>
+__device__ __forceinline__ void store8(T* __restrict__ p, const float (&f)[8]) {
+  if constexpr (sizeof(T) == 2) {
+    dsp_u32x4 u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      u[i] = uint32_t(dsp_f32_to_bf16(f[2 * i])) | (uint32_t(dsp_f32_to_bf16(f[2 * i + 1])) << 16);
+    *reinterpret_cast<dsp_u32x4*>(p) = u;
+  } else {
+    *reinterpret_cast<f32x4*>(p) = f32x4{f[0], f[1], f[2], f[3]};
+    *reinterpret_cast<f32x4*>(p + 4) = f32x4{f[4], f[5], f[6], f[7]};
+  }
+}
+
+template <typename TI, typename TO>
+__global__ __launch_bounds__(256) void rope_vec_kernel(const TI* x, TO* y, uint32_t per_layer,
+                                                       uint32_t per_token, uint32_t per_head,
+                                                       int64_t D, int64_t x_layer_stride,
+                                                       int64_t y_layer_stride,
+                                                       const float* __restrict__ cos_t,
+                                                       const float* __restrict__ sin_t, float sign) {
+#pragma clang fp contract(off)
+  const uint32_t r = blockIdx.x * 256u + threadIdx.x;
+  if (r >= per_layer) return;
+  const uint32_t t = r / per_token, hr = r - t * per_token, h = hr / per_head;
+  const int64_t d = int64_t(hr - h * per_head) * 8, half = D / 2;
+  const int64_t row = (int64_t(t) * (per_token / per_head) + h) * D + d;
+  const TI* xp = x + int64_t(blockIdx.y) * x_layer_stride + row;
+  TO* yp = y + int64_t(blockIdx.y) * y_layer_stride + row;
+  float x1[8], x2[8], c1[8], c2[8], s1[8], s2[8], o1[8], o2[8];
+  load8(xp, x1);
+  load8(xp + half, x2);
+  const float* cp = cos_t + int64_t(t) * D + d;
+  const float* sp = sin_t + int64_t(t) * D + d;
+  load8(cp, c1);
+  load8(cp + half, c2);
+  load8(sp, s1);
+  load8(sp + half, s2);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    o1[i] = x1[i] * c1[i] + sign * (-x2[i] * s1[i]);
+    o2[i] = x2[i] * c2[i] + sign * (x1[i] * s2[i]);
+  }
+  store8(yp, o1);
+  store8(yp + half, o2);
 }
 
 }  // namespace
@@ -700,6 +839,101 @@ extern "C" int dsp_kv_map_gemm_to_pool(
   return dsp_launch_status();
 }
 
+extern "C" int dsp_kv_map_group(
+    const void* a_keys, const void* a_values, int64_t a_layer_stride, const void* const* bts,
+    const void* const* biases, const int32_t* source_layers, const int32_t* target_layers,
+    const int32_t* is_values, int32_t num_maps, int32_t num_segments, int64_t segment_len,
+    void* out_keys, void* out_values, int64_t out_layer_stride, int64_t out_row_stride, int64_t M,
+    int64_t N, const int32_t* block_table, int64_t table_len, int32_t block_size,
+    int64_t num_slots, const float* rope_cos, const float* rope_sin, int32_t head_dim,
+    int32_t dtype, int32_t* err_count, dsp_stream_t stream) {
+  DSP_HOST_CHECK(a_keys && a_values && out_keys && out_values && bts && biases && source_layers &&
+                     target_layers && is_values,
+                 DSP_EINVAL);
+  DSP_HOST_CHECK(M >= 0 && N > 0 && num_maps >= 0 && segment_len > 0 && num_segments >= 1 &&
+                     num_segments <= kMaxSegments && a_layer_stride >= M * segment_len &&
+                     out_layer_stride >= 0 && out_row_stride >= N && num_slots >= 0,
+                 DSP_EINVAL);
+  DSP_HOST_CHECK((rope_cos == nullptr) == (rope_sin == nullptr), DSP_EINVAL);
+  DSP_HOST_CHECK(dtype == DSP_BF16, DSP_EUNSUPPORTED);
+  const bool pool = block_table != nullptr;
+  DSP_HOST_CHECK(!pool || (dsp_is_pow2(block_size) && table_len * block_size >= M), DSP_EINVAL);
+  if (M == 0 || num_maps == 0) return DSP_OK;
+  const bool rope = rope_cos != nullptr;
+  DSP_HOST_CHECK(!rope || ((head_dim == 64 || head_dim == 128) && N % head_dim == 0 &&
+                           dsp_aligned(rope_cos, 16) && dsp_aligned(rope_sin, 16)),
+                 DSP_EUNSUPPORTED);
+  const int64_t K = num_segments * segment_len;
+  bool ok = dsp_aligned(a_keys, 16) && dsp_aligned(a_values, 16) && dsp_aligned(out_keys, 16) &&
+            dsp_aligned(out_values, 16) && a_layer_stride % 8 == 0 && out_layer_stride % 8 == 0 &&
+            out_row_stride % 8 == 0 && N % 8 == 0 && segment_len % big::kBK == 0 &&
+            M * segment_len <= int64_t(UINT32_MAX) && N * K <= int64_t(UINT32_MAX);
+  for (int i = 0; i < num_maps; ++i) {
+    DSP_HOST_CHECK(bts[i] && biases[i], DSP_EINVAL);
+    DSP_HOST_CHECK(is_values[i] == 0 || is_values[i] == 1, DSP_EINVAL);
+    ok = ok && dsp_aligned(bts[i], 16) && target_layers[i] >= 0 && target_layers[i] < 65536;
+    for (int j = 0; j < num_segments; ++j)
+      ok = ok && source_layers[i * num_segments + j] >= 0 &&
+           source_layers[i * num_segments + j] < 65536;
+  }
+  DSP_HOST_CHECK(ok, DSP_EUNSUPPORTED);
+  // 256 x 256 tiles feed the matrix cores best; 128 x 128 ones waste fewer rows of a short
+  // prompt and give the chip more workgroups.  Rounds of resident workgroups (one 256-row
+  // tile per CU, two 128-row ones) times what a round takes, 40 to 24.  Large against small,
+  // 72 maps of 1024 x 1024: 127 against 119 us at 256 tokens, 204 against 214 at 700, 247
+  // against 279 at 1023, 799 against 1006 at 4095; 60 maps of 128 x 128: 61 against 54 at 256,
+  // 112 against 86 at 4095 (both columns with ~50 us of host time).
+  auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  const int64_t cus = dsp_detail::device_cus();
+  const int64_t tl = tiles(256, 256), ts = tiles(128, 128);
+  const int64_t large_cost = (tl * num_maps + cus - 1) / cus * 40;
+  const int64_t small_cost = (ts * num_maps + 2 * cus - 1) / (2 * cus) * 24;
+  const bool large = large_cost <= small_cost;
+  DSP_HOST_CHECK((large ? tl : ts) * kMaxGroup < (int64_t(1) << 31), DSP_EUNSUPPORTED);
+  PoolOut po;
+  po.block_tables = block_table;
+  po.log2_bs = pool ? dsp_log2i(block_size) : 0;
+  po.num_slots = num_slots;
+  po.rope_cos = rope_cos;
+  po.rope_sin = rope_sin;
+  po.head_dim = head_dim;
+  po.err_count = err_count;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  GroupArgs g;
+  g.a[0] = static_cast<const uint16_t*>(a_keys);
+  g.a[1] = static_cast<const uint16_t*>(a_values);
+  g.c[0] = static_cast<uint16_t*>(out_keys);
+  g.c[1] = static_cast<uint16_t*>(out_values);
+  g.a_layer_stride = a_layer_stride;
+  g.c_layer_stride = out_layer_stride;
+  for (int first = 0; first < num_maps; first += kMaxGroup) {
+    const int n = num_maps - first < kMaxGroup ? num_maps - first : kMaxGroup;
+    for (int i = 0; i < n; ++i) {
+      GroupEntry& e = g.e[i];
+      e = GroupEntry{};
+      e.bt = static_cast<const uint16_t*>(bts[first + i]);
+      e.bias = static_cast<const uint16_t*>(biases[first + i]);
+      for (int j = 0; j < num_segments; ++j)
+        e.seg[j] = static_cast<uint16_t>(source_layers[(first + i) * num_segments + j]);
+      e.layer = static_cast<uint16_t>(target_layers[first + i]);
+      e.values = static_cast<uint16_t>(is_values[first + i]);
+    }
+    const unsigned grid = static_cast<unsigned>((large ? tl : ts) * n);
+#define DSP_GROUP(TL, R, P)                                                               \
+  map_group_kernel<big::TL, R, P><<<grid, big::TL::kNT, 0, s>>>(g, segment_len, out_row_stride, \
+                                                               M, N, K, po)
+#define DSP_GROUP_T(TL)                                                 \
+  if (rope && pool) DSP_GROUP(TL, 1, 1); else if (rope) DSP_GROUP(TL, 1, 0); \
+  else if (pool) DSP_GROUP(TL, 0, 1); else DSP_GROUP(TL, 0, 0)
+    if (large) { DSP_GROUP_T(Large); } else { DSP_GROUP_T(Small); }
+#undef DSP_GROUP_T
+#undef DSP_GROUP
+    const int st = dsp_launch_status();
+    if (st != DSP_OK) return st;
+  }
+  return DSP_OK;
+}
+
 extern "C" int dsp_kv_rope(const void* x, int64_t x_layer_stride, void* y,
                            int64_t y_layer_stride, int64_t L, int64_t T, int64_t H, int64_t D,
                            const float* cos_table, const float* sin_table, int32_t direction,
@@ -718,6 +952,28 @@ extern "C" int dsp_kv_rope(const void* x, int64_t x_layer_stride, void* y,
   hipStream_t s = static_cast<hipStream_t>(stream);
   const unsigned nb = static_cast<unsigned>(blocks);
   const float sg = float(direction);
+  // Whole 16-byte vectors in either half of every row (rows are contiguous, so the layer
+  // strides and the bases decide), a layer's vectors counted in 32 bits and at most 65535
+  // layers: the vector form.
+  const int64_t xe = in_dtype == DSP_BF16 ? 2 : 4, ye = out_dtype == DSP_BF16 ? 2 : 4;
+  const int64_t vecs = T * H * (D / 16);
+  if (D % 16 == 0 && vecs < (int64_t(1) << 31) && L <= 65535 && dsp_aligned(x, 16) &&
+      dsp_aligned(y, 16) && x_layer_stride * xe % 16 == 0 && y_layer_stride * ye % 16 == 0 &&
+      dsp_aligned(cos_table, 16) && dsp_aligned(sin_table, 16)) {
+    const dim3 vg(static_cast<unsigned>((vecs + 255) / 256), static_cast<unsigned>(L));
+    const uint32_t ph = static_cast<uint32_t>(D / 16), pt = static_cast<uint32_t>(H * (D / 16));
+#define DSP_ROPE_VEC(TI, TO)                                                                  \
+  rope_vec_kernel<TI, TO><<<vg, 256, 0, s>>>(static_cast<const TI*>(x), static_cast<TO*>(y),  \
+                                             static_cast<uint32_t>(vecs), pt, ph, D,          \
+                                             x_layer_stride, y_layer_stride, cos_table,       \
+                                             sin_table, sg)
+    if (in_dtype == DSP_BF16 && out_dtype == DSP_BF16) DSP_ROPE_VEC(uint16_t, uint16_t);
+    else if (in_dtype == DSP_BF16) DSP_ROPE_VEC(uint16_t, float);
+    else if (out_dtype == DSP_BF16) DSP_ROPE_VEC(float, uint16_t);
+    else DSP_ROPE_VEC(float, float);
+#undef DSP_ROPE_VEC
+    return dsp_launch_status();
+  }
 #define DSP_ROPE(TI, TO)                                                                      \
   rope_kernel<TI, TO><<<nb, 256, 0, s>>>(static_cast<const TI*>(x), static_cast<TO*>(y), L, T, \
                                          H, D, x_layer_stride, y_layer_stride, cos_table,    \

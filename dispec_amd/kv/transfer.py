@@ -11,6 +11,8 @@ Every step runs on the HIP kernels of libdispec_hip.so:
   strip_rope / apply_rope   -> dsp_kv_rope (fp32 math, one launch for all layers)
   LayerMap.apply            -> dsp_kv_map_gemm (MFMA; the design row is read in place
                                from the source buffer, never concatenated in memory)
+  all dense layer maps      -> dsp_kv_map_group (one launch, RoPE and the pool scatter in
+  of a prompt                  its epilogue)
 and the bf16 result is rounded at the same points the reference's bf16 torch ops round
 (x @ W, then + b; F.linear's bias fused; gelu; the residual add).
 
@@ -381,18 +383,61 @@ class CrossModelKVMap:
 
     def _apply(self, source: torch.Tensor, maps: list[LayerMap], use_residual: bool,
                rope: tuple[torch.Tensor, torch.Tensor] | None = None,
-               out: torch.Tensor | None = None) -> torch.Tensor:
-        """Target layers (L_tgt, T, H, D) from contiguous source layers (L_src, T, H, D)."""
+               out: torch.Tensor | None = None, done=frozenset()) -> torch.Tensor:
+        """Target layers (L_tgt, T, H, D) from contiguous source layers (L_src, T, H, D);
+        layers in `done` are already in `out`, rotated."""
         L_src, T, H, D = source.shape
         kv = H * D
         if out is None:
             out = torch.empty((len(maps), T, H, D), dtype=torch.bfloat16, device=source.device)
         for layer, m in enumerate(maps):
-            m.apply_into(source, [s * T * kv for s in m.source_layers], kv, kv, T,
-                         out[layer].view(T, kv), use_residual)
-        if rope is not None:
+            if layer not in done:
+                m.apply_into(source, [s * T * kv for s in m.source_layers], kv, kv, T,
+                             out[layer].view(T, kv), use_residual)
+                if rope is not None and done:
+                    _rope(out[layer:layer + 1], rope[0], rope[1], +1, out=out[layer:layer + 1])
+        if rope is not None and not done:
             _rope(out, rope[0], rope[1], +1, out=out)
         return out
+
+    def _apply_grouped(self, content: torch.Tensor, vals: torch.Tensor, use_residual: bool,
+                       out: tuple[torch.Tensor, torch.Tensor],
+                       rope: tuple[torch.Tensor, torch.Tensor], table: torch.Tensor | None = None,
+                       block_size: int = 1, err: torch.Tensor | None = None):
+        """Every dense map (no factors, no residual in use) in one launch per design width,
+        keys rotated with `rope` (fp32 tables, contiguous): rows of `out` = (keys, values), each
+        (L_tgt, T or pool slots, H, D), by token or, with a block table, by pool slot.  Returns
+        the layers done, (keys, values), as sets: none where the launch does not take the shape
+        (the caller runs those layers one at a time)."""
+        L_src, T, H, D = content.shape
+        kv = H * D
+        jobs: dict[int, list] = {}     # number of source layers -> [(kind, layer, map)]
+        for kind, maps in enumerate((self.keys, self.values)):
+            for layer, m in enumerate(maps):
+                m._prepare()
+                if m.factors is None and not (use_residual and m.residual is not None) \
+                        and tuple(m._wt.shape) == (kv, kv * len(m.source_layers)):
+                    jobs.setdefault(len(m.source_layers), []).append((kind, layer, m))
+        done: tuple[set, set] = (set(), set())
+        for n_seg, group in jobs.items():
+            n = len(group)
+            pointers, ints = ctypes.c_void_p * n, ctypes.c_int32 * n
+            st = _lib.lib().dsp_kv_map_group(
+                content.data_ptr(), vals.data_ptr(), T * kv,
+                pointers(*[m._wt.data_ptr() for _, _, m in group]),
+                pointers(*[m._b.data_ptr() for _, _, m in group]),
+                (ctypes.c_int32 * (n * n_seg))(*[s for _, _, m in group for s in m.source_layers]),
+                ints(*[layer for _, layer, _ in group]), ints(*[kind for kind, _, _ in group]),
+                n, n_seg, kv, out[0].data_ptr(), out[1].data_ptr(), out[0].stride(0), kv, T, kv,
+                _lib.ptr(table), 0 if table is None else table.numel(), block_size,
+                out[0].shape[1], rope[0].data_ptr(), rope[1].data_ptr(), D, _lib.DSP_BF16,
+                _lib.ptr(err), _lib.stream_of(content))
+            if st == _lib.DSP_EUNSUPPORTED:
+                continue
+            _lib.check(st, "dsp_kv_map_group")
+            for kind, layer, _ in group:
+                done[kind].add(layer)
+        return done
 
     @torch.inference_mode()
     def map_into(self, k: torch.Tensor, v: torch.Tensor,
@@ -426,11 +471,19 @@ class CrossModelKVMap:
         content = _rope(k, *source_rope, direction=-1, out_dtype=torch.bfloat16)
         vals = v.to(torch.bfloat16).contiguous()
         tcos, tsin = target_rope[0].float().contiguous(), target_rope[1].float().contiguous()
-        cu = torch.tensor([0, T], dtype=torch.long).to(k.device)
+        if tuple(tcos.shape) != (T, D) or tuple(tsin.shape) != (T, D):
+            raise ValueError(f"rope tables {tuple(tcos.shape)} do not match {T} rows of "
+                             f"head_dim {D}")
+        done = self._apply_grouped(content, vals, use_residual, (cache.key, cache.value),
+                                   (tcos, tsin), table, cache.block_size, cache._err)
+        if len(done[0]) + len(done[1]) < 2 * cache.num_layers:
+            cu = torch.tensor([0, T], dtype=torch.long).to(k.device)
         for layer in range(cache.num_layers):
             jobs = ((self.keys[layer], content, cache.key, (tcos, tsin)),
                     (self.values[layer], vals, cache.value, None))
-            for m, src, pool, rope in jobs:
+            for kind, (m, src, pool, rope) in enumerate(jobs):
+                if layer in done[kind]:
+                    continue
                 offs = [s * T * kv for s in m.source_layers]
                 if (not use_residual or m.residual is None) and m.apply_to_pool(
                         src, offs, kv, kv, T, pool[layer], table, cache.block_size, rope,
@@ -459,7 +512,15 @@ class CrossModelKVMap:
         if self.dtype != torch.bfloat16:
             raise ValueError("the HIP map runs bf16 maps (load with dtype=torch.bfloat16)")
         content = _rope(k, *source_rope, direction=-1, out_dtype=torch.bfloat16)
-        keys = self._apply(content, self.keys, use_residual, rope=target_rope)
-        del content
-        values = self._apply(v.to(torch.bfloat16).contiguous(), self.values, use_residual)
+        vals = v.to(torch.bfloat16).contiguous()
+        L_src, T, H, D = k.shape
+        cos, sin = (t.float().contiguous() for t in target_rope)
+        outs = tuple(torch.empty((len(maps), *src.shape[1:]), dtype=torch.bfloat16,
+                                 device=k.device)
+                     for maps, src in ((self.keys, content), (self.values, vals)))
+        done = (frozenset(), frozenset())
+        if tuple(cos.shape) == tuple(sin.shape) == (T, D) and vals.shape[1:] == content.shape[1:]:
+            done = self._apply_grouped(content, vals, use_residual, outs, (cos, sin))
+        keys = self._apply(content, self.keys, use_residual, (cos, sin), outs[0], done[0])
+        values = self._apply(vals, self.values, use_residual, None, outs[1], done[1])
         return keys.to(k.dtype), values.to(v.dtype)

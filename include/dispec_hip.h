@@ -385,6 +385,35 @@ int dsp_kv_map_gemm_to_pool(const void* a, const int64_t* a_segment_offsets,
                             const float* rope_sin, int32_t head_dim, int32_t dtype,
                             int32_t* err_count, dsp_stream_t stream);
 
+/* J5b for many layers at once: the dense maps of one prompt, keys and values, in one launch
+ * (more than 80 maps: one launch per 80).  Replaces the layer loop of CrossModelKVMap._apply
+ * (transfer.py:243-253) with LayerMap.apply's dense form (:104-112): map i reads the design
+ * rows a + source_layers[i * num_segments + j] * a_layer_stride (j < num_segments; a = a_keys
+ * or a_values by is_values[i]; rows of segment_len elements, contiguous) and writes
+ * bf16(bf16(x @ W_i) + bias_i) as rows of target layer target_layers[i] of out_keys or
+ * out_values, keys re-rotated with rope_cos / rope_sin when given (as in
+ * dsp_kv_map_gemm_to_pool).  Same rounding as dsp_kv_map_gemm with bias_mode 1 followed by
+ * dsp_kv_rope: bit-identical to them.
+ *   bts, biases, source_layers, target_layers, is_values : HOST arrays (of device pointers,
+ *                 of int32) of num_maps entries (source_layers: num_maps * num_segments);
+ *                 W_i is N x (num_segments * segment_len), K contiguous.
+ *   out_*       : target layers out_layer_stride elements apart, rows out_row_stride apart.
+ *   block_table : device int32 [table_len], or NULL.  NULL: row m of a layer is token m.  Else
+ *                 row m goes to pool slot block_table[m / block_size] * block_size +
+ *                 m % block_size; slots outside [0, num_slots) are skipped and counted in
+ *                 err_count (>= 1 per row and map).
+ * Layers up to 65535; the alignment and size limits of dsp_kv_map_gemm_to_pool, else
+ * DSP_EUNSUPPORTED with nothing launched. */
+int dsp_kv_map_group(const void* a_keys, const void* a_values, int64_t a_layer_stride,
+                     const void* const* bts, const void* const* biases,
+                     const int32_t* source_layers, const int32_t* target_layers,
+                     const int32_t* is_values, int32_t num_maps, int32_t num_segments,
+                     int64_t segment_len, void* out_keys, void* out_values,
+                     int64_t out_layer_stride, int64_t out_row_stride, int64_t M, int64_t N,
+                     const int32_t* block_table, int64_t table_len, int32_t block_size,
+                     int64_t num_slots, const float* rope_cos, const float* rope_sin,
+                     int32_t head_dim, int32_t dtype, int32_t* err_count, dsp_stream_t stream);
+
 /* RoPE strip (direction -1) or apply (+1) on (L, T, H, D) rows in fp32:
  *     y = x * cos + direction * rotate_half(x) * sin,   rotate_half(x) = cat(-x2, x1)
  * Replaces strip_rope / apply_rope (dispec/kv/transfer.py:66-80).  cos/sin are fp32
