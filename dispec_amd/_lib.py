@@ -74,8 +74,7 @@ SIGNATURES: dict[str, tuple] = {
                                         c_int64, c_int64, _P, c_int64, c_int32, c_int64, c_int64,
                                         c_int64, c_int32, c_int64, _P, _P, _P, c_int32, c_int32,
                                         _P, _P]),
-    "dsp_kv_map_group": (c_int, [_P, _P, c_int64, POINTER(c_void_p), POINTER(c_void_p),
-                                 POINTER(c_int32), POINTER(c_int32), POINTER(c_int32), c_int32,
+    "dsp_kv_map_group": (c_int, [_P, _P, c_int64, _P, _P, _P, _P, _P, c_int32,
                                  c_int32, c_int64, _P, _P, c_int64, c_int64, c_int64, c_int64, _P,
                                  c_int64, c_int32, c_int64, _P, _P, c_int32, c_int32, _P, _P]),
     "dsp_kv_rope": (c_int, [_P, c_int64, _P, c_int64, c_int64, c_int64, c_int64, c_int64, _P, _P,
