@@ -206,13 +206,14 @@ int dsp_kv_scatter_ordered(void* k_pool, void* v_pool, int64_t num_layers,
  * serve bf16 / fp16 with D in {16, 32, 64, 128} and G = Hq / KVH in 1..8, and on block tables
  * with 16-byte-aligned rows D 256 and any G too (probabilities kept to fp32 accuracy there,
  * in P.V as well); every other shape with D a power of two from 8 to 256 (fp32, D 8, slot
- * tables or unaligned rows with D 256 or G above 8) runs on a generic kernel -- one wave per (sequence, query head, partition), fp32 accumulation,
- * element-aligned pointers -- whose automatic partition is dsp_paged_decode_partition_tokens
+ * tables or unaligned rows with D 256 or G above 8) runs on a generic kernel -- fp32 on 16-row
+ * tiles of the fp32 matrix cores, 16-bit one wave per (sequence, query head, partition); fp32
+ * accumulation, element-aligned pointers -- whose automatic partition is dsp_paged_decode_partition_tokens
  * and whose workspace is covered by dsp_paged_decode_workspace_bytes.  Other D:
  * DSP_EUNSUPPORTED.
  * err_count (optional) is incremented for a context length outside [0, max_ctx]
- * (clamped) and, on block tables and the generic kernel, once per wave that met a block id
- * whose slots lie outside the cache (those keys are skipped). */
+ * (clamped) and, on block tables and the generic kernel, once per wave (fp32: per
+ * query row and partition) that met a block id whose slots lie outside the cache (those keys are skipped). */
 size_t dsp_paged_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t KVH, int32_t D,
                                         int32_t max_ctx, int32_t partition_tokens);
 int dsp_paged_decode_partition_tokens(int32_t B, int32_t KVH, int32_t D, int32_t max_ctx);
