@@ -124,10 +124,16 @@ __device__ __forceinline__ int64_t active_workers(int64_t C, int num_workers) {
 // a worker is a workgroup of HG waves, wave i taking KV head HG*group + i of every piece,
 // so the waves of a workgroup read the same keys' rows side by side (HG x 256 bytes of
 // each 2 KiB slot row at D 128: the pool's DRAM pages are then read HG slices at a time).
-// kSplitP: the shapes that the generic kernel serves otherwise (D 256 and G > 8), whose
-// probabilities are fp32: they enter P.V as two 16-bit operands (pack8); and keys of a block id
-// outside the cache are masked, as they are there.
-template <typename Tag, int D, bool kOff32, int HG, bool kSplitP>
+// kMode: kPlain; kWide, the shapes that the generic kernel serves otherwise (D 256 and G > 8),
+// whose probabilities are fp32: they enter P.V as two 16-bit operands (pack8), and keys of a
+// block id outside the cache are masked, as they are there; kSlots, decode by per-token slot
+// table (`bt` is the slot table), which the VALU kernel serves otherwise: fp32 probabilities as
+// in kWide, bad slots masked and each counted, as they are there.  A slot-table window holds the
+// slots of 64 keys, one per lane, the next window's loaded while it is in use; a lane takes the
+// slots of its K and V rows from it by permute (24 sequences of 200-3000 keys, 28 heads over 4:
+// kernel and merge 42 -> 26 us a layer).
+enum Mode { kPlain, kWide, kSlots };
+template <typename Tag, int D, bool kOff32, int HG, int kMode>
 __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128 ? 2 : kOcc))) void decode_balanced_kernel(
     const uint16_t* __restrict__ q, int64_t qsb, int64_t qsh, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
@@ -136,6 +142,7 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
     int32_t KVH, int32_t G, int32_t RPH, int32_t max_ctx, float scale_log2,
     int32_t num_workers, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
     uint16_t* __restrict__ out, int64_t osb, int64_t osh, int32_t* __restrict__ err_count) {
+  constexpr bool kSplitP = kMode != kPlain;
   constexpr int NKK = D / 32;       // 32-dim K steps of the score MFMA
   constexpr int NT = D / 16;        // 16-dim output tiles
   constexpr int CPR = D / 8;        // 16-byte chunks per K/V row
@@ -188,6 +195,7 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
   char* const slab_l = slab[hw];
   auto swz = [](int r, int c) { return c ^ ((2 * ((r >> 2) & 3)) & (CPR - 1)); };
   bool any_bad = false;
+  int bad_slots = 0;  // kSlots: bad slots met so far (uniform)
 
   for (;;) {
     // ---- piece: units [u, u1) of segment (b, kvh), keys [kb, ke)
@@ -214,17 +222,19 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
                                                              8 * grp)
                        : dsp_u32x4{0u, 0u, 0u, 0u};
 
+    // (kSlots: entries are the slots of keys, and a "block" below is one key.)
     // Block-table windows: lane i holds the id of block wblk + i (win) and wblk + 64 + i
     // (win2).  Chunks advance by 32 keys, i.e. by at most 32 blocks, so a chunk always
     // lies within win and win2 once the windows have been advanced for its first key.
-    int wblk = kb >> log2_bs;
+    const int wsh = kMode == kSlots ? 0 : log2_bs;
+    int wblk = kb >> wsh;
     auto load_win = [&](int first) -> int32_t {
       const int64_t j = int64_t(first) + lane;
       return j < bt_stride ? bt[bt_row + j] : -1;
     };
     int32_t win = load_win(wblk), win2 = load_win(wblk + 64);
     auto advance = [&](int key) {
-      if ((key >> log2_bs) - wblk >= 64) {
+      if ((key >> wsh) - wblk >= 64) {
         wblk += 64;
         win = win2;
         win2 = load_win(wblk + 64);
@@ -232,7 +242,14 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
     };
     // Block ids of the chunk starting at t0: its first block and the next one (scalars).
     int32_t cb0 = 0, cb1 = 0;
+    // kSlots: which of the chunk's 32 keys have slots inside the cache (uniform; a chunk, 32
+    // keys from a multiple of 32 into the window, lies in `win`).
+    uint32_t okm = 0;
     auto chunk_blocks = [&](int t0) {
+      if constexpr (kMode == kSlots) {
+        okm = uint32_t(__ballot(win >= 0 && win < num_slots) >> (t0 - wblk));
+        return;
+      }
       const int j = (t0 >> log2_bs) - wblk;  // < 64 after advance(t0); j + 1 < 128
       cb0 = j < 64 ? __builtin_amdgcn_readlane(win, j) : __builtin_amdgcn_readlane(win2, j - 64);
       cb1 = j + 1 < 64 ? __builtin_amdgcn_readlane(win, j + 1)
@@ -253,6 +270,10 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
     // Element offset of `key` of the chunk starting at t0 in one layer's cache (head
     // included), -1 when its block id is out of range.
     auto elem_of = [&](int t0, int key) -> int64_t {
+      if constexpr (kMode == kSlots) {
+        const int32_t sl = __builtin_amdgcn_ds_bpermute((key - wblk) << 2, win);
+        return sl >= 0 && sl < num_slots ? sl * kvs_slot + head_off : int64_t(-1);
+      }
       const int32_t blk = ((key >> log2_bs) != (t0 >> log2_bs)) ? cb1 : cb0;
       const int64_t sl = int64_t(blk) * (bmask + 1) + (key & bmask);
       return (sl >= 0 && sl < num_slots) ? sl * kvs_slot + head_off : int64_t(-1);
@@ -315,7 +336,7 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
     // K before V, as inside the loop: the loop head then waits for K only (vmcnt(VINS)),
     // with this chunk's V still in flight, on entry and on every later iteration alike.
     chunk_blocks(kb);
-    if constexpr (kSplitP) valid_limits(kb);
+    if constexpr (kMode == kWide) valid_limits(kb);
     load_k(kb);
     load_v(kb);
     for (int t0 = kb; t0 < ke; t0 += 32) {
@@ -328,12 +349,25 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
 #pragma unroll
         for (int kk = 0; kk < NKK; ++kk) sc[st] = mfma32<Tag>(kop[st][kk], qop[kk], sc[st]);
       }
-      const int cur[2] = {kSplitP ? min(lim, vlim[0]) : lim, kSplitP ? min(lim, vlim[1]) : lim};
+      const int cur[2] = {kMode == kWide ? min(lim, vlim[0]) : lim,
+                          kMode == kWide ? min(lim, vlim[1]) : lim};
+      const uint32_t ok_cur = okm;
       if (prefetch) {
         advance(tn);
         chunk_blocks(tn);
-        if constexpr (kSplitP) valid_limits(tn);
+        if constexpr (kMode == kWide) valid_limits(tn);
         load_k(tn);
+      }
+      if constexpr (kMode == kSlots) {
+        const uint32_t bad = ~ok_cur & (ke - t0 < 32 ? (1u << (ke - t0)) - 1u : ~0u);
+        bad_slots += __popc(bad);
+        if (bad) {  // uniform, rare
+#pragma unroll
+          for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              if ((bad >> (16 * st + 4 * grp + j)) & 1u) sc[st][j] = -INFINITY;
+        }
       }
       // Scale and mask; lane holds keys t0 + 16*st + 4*grp + j of packed row n.
       float s[2][4];
@@ -444,7 +478,11 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
       if (b >= B) break;
     }
   }
-  if (err_count && __ballot(any_bad) && lane == 0) atomicAdd(err_count, 1);
+  if constexpr (kMode == kSlots) {
+    if (err_count && bad_slots && lane == 0) atomicAdd(err_count, bad_slots);
+  } else {
+    if (err_count && __ballot(any_bad) && lane == 0) atomicAdd(err_count, 1);
+  }
 }
 
 // One workgroup (4 waves) per (sequence b, query head h, query i).  Merges the pieces of
@@ -580,7 +618,7 @@ __global__ __launch_bounds__(256) void decode_balanced_combine_kernel(
   }
 }
 
-template <typename Tag, int D, int HG, bool kSplitP>
+template <typename Tag, int D, int HG, int kMode>
 int launch_balanced_hg(int W, int32_t KVH, const uint16_t* q, int64_t qsb, int64_t qsh,
                        const uint16_t* kc, const uint16_t* vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
                        const int32_t* bt, int64_t bt_stride, int32_t log2_bs,
@@ -593,11 +631,11 @@ int launch_balanced_hg(int W, int32_t KVH, const uint16_t* q, int64_t qsb, int64
   // largest element offset: last slot's last head's row end
   const bool off32 = num_slots * kvs_slot + KVH * kvs_head + D < (int64_t(1) << 31);
   if (off32)
-    decode_balanced_kernel<Tag, D, true, HG, kSplitP><<<dim3(static_cast<unsigned>(Wg)), 64 * HG, 0, s>>>(
+    decode_balanced_kernel<Tag, D, true, HG, kMode><<<dim3(static_cast<unsigned>(Wg)), 64 * HG, 0, s>>>(
         q, qsb, qsh, kc, vc, num_slots, kvs_slot, kvs_head, bt, bt_stride, log2_bs, ctx_lens,
         cu_q, B, KVH, G, RPH, max_ctx, scale_log2, Wg, ws_acc, ws_ml, out, osb, osh, err_count);
   else
-    decode_balanced_kernel<Tag, D, false, HG, kSplitP><<<dim3(static_cast<unsigned>(Wg)), 64 * HG, 0, s>>>(
+    decode_balanced_kernel<Tag, D, false, HG, kMode><<<dim3(static_cast<unsigned>(Wg)), 64 * HG, 0, s>>>(
         q, qsb, qsh, kc, vc, num_slots, kvs_slot, kvs_head, bt, bt_stride, log2_bs, ctx_lens,
         cu_q, B, KVH, G, RPH, max_ctx, scale_log2, Wg, ws_acc, ws_ml, out, osb, osh, err_count);
   const int st = dsp_launch_status();
@@ -608,22 +646,22 @@ int launch_balanced_hg(int W, int32_t KVH, const uint16_t* q, int64_t qsb, int64
   return dsp_launch_status();
 }
 
-template <typename Tag, int D, bool kSplitP, typename... A>
+template <typename Tag, int D, int kMode, typename... A>
 int launch_balanced_d(int W, int32_t KVH, A... args) {
   switch (dsp_detail::balanced_head_group(KVH)) {
-    case 4: return launch_balanced_hg<Tag, D, 4, kSplitP>(W, KVH, args...);
-    case 2: return launch_balanced_hg<Tag, D, 2, kSplitP>(W, KVH, args...);
-    default: return launch_balanced_hg<Tag, D, 1, kSplitP>(W, KVH, args...);
+    case 4: return launch_balanced_hg<Tag, D, 4, kMode>(W, KVH, args...);
+    case 2: return launch_balanced_hg<Tag, D, 2, kMode>(W, KVH, args...);
+    default: return launch_balanced_hg<Tag, D, 1, kMode>(W, KVH, args...);
   }
 }
 
-template <typename Tag, bool kSplitP, typename... A>
+template <typename Tag, int kMode, typename... A>
 int launch_balanced(int D, A... args) {
   switch (D) {
-    case 32: return launch_balanced_d<Tag, 32, kSplitP>(args...);
-    case 64: return launch_balanced_d<Tag, 64, kSplitP>(args...);
-    case 128: return launch_balanced_d<Tag, 128, kSplitP>(args...);
-    case 256: return launch_balanced_d<Tag, 256, true>(args...);
+    case 32: return launch_balanced_d<Tag, 32, kMode>(args...);
+    case 64: return launch_balanced_d<Tag, 64, kMode>(args...);
+    case 128: return launch_balanced_d<Tag, 128, kMode>(args...);
+    case 256: return launch_balanced_d<Tag, 256, kMode == kPlain ? kWide : kMode>(args...);
     default: return DSP_EUNSUPPORTED;
   }
 }
@@ -719,11 +757,14 @@ int balanced_decode(const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h,
               kv_stride_head, block_table, bt_stride, log2_bs, ctx_lens, cu_q, max_q_len, B, G,
               max_ctx, scale_log2, ws_acc, ws_ml, out, o_stride_b, o_stride_h, err_count, s);
   };
+  if (log2_bs < 0)  // a slot table
+    return f16 ? launch([](auto... a) { return launch_balanced<F16Tag, kSlots>(a...); })
+               : launch([](auto... a) { return launch_balanced<Bf16Tag, kSlots>(a...); });
   if (cu_q == nullptr && G > 8)  // decode of wide groups: fp32 probabilities
-    return f16 ? launch([](auto... a) { return launch_balanced<F16Tag, true>(a...); })
-               : launch([](auto... a) { return launch_balanced<Bf16Tag, true>(a...); });
-  return f16 ? launch([](auto... a) { return launch_balanced<F16Tag, false>(a...); })
-             : launch([](auto... a) { return launch_balanced<Bf16Tag, false>(a...); });
+    return f16 ? launch([](auto... a) { return launch_balanced<F16Tag, kWide>(a...); })
+               : launch([](auto... a) { return launch_balanced<Bf16Tag, kWide>(a...); });
+  return f16 ? launch([](auto... a) { return launch_balanced<F16Tag, kPlain>(a...); })
+             : launch([](auto... a) { return launch_balanced<Bf16Tag, kPlain>(a...); });
 }
 
 }  // namespace dsp_detail

@@ -25,7 +25,8 @@ int mq_decode(const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h, const u
 // cu_q null, max_q_len 1, q/out rows indexed by sequence.  Multi-query (verify): cu_q as
 // for dsp_paged_mq_attention, max_q_len * G <= 16 query rows per KV head, q/out rows
 // indexed by token.  `applies` says whether the shape is one it serves; the workspace is
-// balanced_workspace_bytes(..., max_q_len * G, ...) long.
+// balanced_workspace_bytes(..., max_q_len * G, ...) long.  log2_bs < 0: decode by per-token slot
+// table (block_table and bt_stride are the slot table's).
 bool balanced_decode_applies(int32_t B, int32_t KVH, int32_t D, int32_t max_ctx,
                              int32_t block_size);
 // The automatic split of a block-table decode of 256-wide heads or of 9 to 16 query heads per

@@ -23,7 +23,8 @@
 //
 // dsp_paged_decode sends block-table calls with head_dim >= 32 to the multi-query MFMA
 // kernel of paged_mq.hip in its decode mode (measured faster on every decode shape, most
-// for GQA groups of 6+); this VALU kernel serves per-token slot tables and head_dim 16.
+// for GQA groups of 6+); this VALU kernel serves small launches by per-token slot table,
+// explicit partitions of them, and head_dim 16.
 #include <float.h>
 
 #include <atomic>
@@ -657,6 +658,23 @@ extern "C" int dsp_paged_decode(const void* q, int64_t q_stride_b, int64_t q_str
                                        scale_log2, max_ctx, static_cast<float*>(workspace), oh,
                                        o_stride_b,
                                        o_stride_h, dtype == DSP_F16, err_count, s);
+  }
+  // Slot tables, automatic split: the same kernel, from 16 sequences and 16384 table entries
+  // up.  Below, the VALU kernel's fixed partitions start and merge faster (us, VALU against
+  // balanced, heads / KV heads / head_dim 14/2/64 and 28/4/128: 1 x 4000 keys 12.4/15.1 and
+  // 14.3/15.4, 8 x 1000 12.5/13.6 and 15.5/16.8, ragged 8 x 1600 12.5/14.2 and 18.4/17.7;
+  // 16 x 1600 17.2/14.3 and 28.4/21.9, 32 x 600 16.6/14.0 and 23.9/20.2, 48 x 5000 51.7/41.0
+  // and 142/96).
+  const bool many_slots = B >= 16 && int64_t(B) * max_ctx >= 16384 && max_ctx > kOneRoundCtx;
+  if (!bm && partition_tokens == 0 && many_slots && num_slots > 0 &&
+      dsp_detail::balanced_decode_applies(B, KVH, D, max_ctx, 16)) {
+    const size_t need = dsp_detail::balanced_workspace_bytes(B, KVH, G, D, max_ctx);
+    if (workspace_bytes >= need && workspace != nullptr && dsp_aligned(workspace, 16))
+      return dsp_detail::balanced_decode(qh, q_stride_b, q_stride_h, kh, vh, num_slots,
+                                         kv_stride_slot, kv_stride_head, table, table_stride, -1,
+                                         ctx_lens, nullptr, 1, B, KVH, G, D, scale_log2, max_ctx,
+                                         static_cast<float*>(workspace), oh, o_stride_b,
+                                         o_stride_h, dtype == DSP_F16, err_count, s);
   }
   int P = partition_tokens > 0 ? partition_tokens
           : one_round          ? (max_ctx + 127) / 128 * 128

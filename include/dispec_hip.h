@@ -196,8 +196,10 @@ int dsp_kv_scatter_ordered(void* k_pool, void* v_pool, int64_t num_layers,
  *                  cut into equal contiguous shares, one per wave, computed on the device
  *                  from ctx_lens -- and a log-sum-exp combine kernel.  DSP_SPLIT_BALANCED
  *                  asks for the balanced split whatever the size (block tables, D in {32,
- *                  64, 128}, G <= 8, B <= 512; else DSP_EUNSUPPORTED).  Otherwise (or with
- *                  a slot table) fixed partitions of partition_tokens keys (0: chosen by
+ *                  64, 128}, G <= 8, B <= 512; else DSP_EUNSUPPORTED).  0 with a slot table
+ *                  of 16 to 512 sequences, more than 512 wide and of 16384 entries or
+ *                  more: the balanced split too (probabilities kept to fp32 accuracy,
+ *                  bad slots masked and counted once per KV head).  Otherwise fixed partitions of partition_tokens keys (0: chosen by
  *                  dsp_paged_decode_partition_tokens) per (sequence, KV head), merged by
  *                  the combine kernel when a sequence spans more than one.  `workspace`
  *                  must hold dsp_paged_decode_workspace_bytes(..., partition_tokens)
