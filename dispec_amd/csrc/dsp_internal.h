@@ -88,6 +88,20 @@ int prefill_shared_prefix(const uint16_t* q, int64_t q_stride_t, int64_t q_strid
                           int64_t o_stride_t, int64_t o_stride_h, bool f16, int32_t* err_count,
                           hipStream_t s);
 
+// dsp_paged_mq_attention on 128-row tiles with the launch's 64-key chunks in equal shares
+// (dsp_paged_mq_attention_ragged); the caller has checked the arguments and the workspace.
+// bytes 0 / DSP_EUNSUPPORTED: a shape it does not serve.
+size_t ragged_workspace_bytes(int32_t B, int32_t KVH, int32_t G, int32_t D, int32_t max_q_len,
+                              int32_t max_ctx);
+int prefill_ragged(const uint16_t* q, int64_t q_stride_t, int64_t q_stride_h,
+                   const uint16_t* k_cache, const uint16_t* v_cache, int64_t num_slots,
+                   int64_t kv_stride_slot, int64_t kv_stride_head, const int32_t* block_table,
+                   int64_t bt_stride, int32_t block_size, const int32_t* cu_q,
+                   const int32_t* ctx_lens, int32_t B, int32_t KVH, int32_t G, int32_t D,
+                   float scale_log2, int32_t max_q_len, int32_t max_ctx, float* workspace,
+                   uint16_t* out, int64_t o_stride_t, int64_t o_stride_h, bool f16,
+                   int32_t* err_count, hipStream_t s);
+
 // Attention for shapes outside the tuned kernels (generic_attn.hip): fp32 caches, head
 // dims 8..256 (powers of two), any GQA group.  Decode: cu_q null, max_q_len 1, one row per
 // sequence with its context clamped to [0, max_ctx]; multi-query: the semantics of

@@ -742,6 +742,46 @@ extern "C" int dsp_paged_mq_attention(const void* q, int64_t q_stride_t, int64_t
                            o_stride_h, dtype, err_count, stream, 0);
 }
 
+extern "C" size_t dsp_paged_mq_ragged_workspace_bytes(int32_t B, int32_t Hq, int32_t KVH,
+                                                     int32_t D, int32_t max_q_len,
+                                                     int32_t max_ctx) {
+  if (B <= 0 || KVH <= 0 || Hq <= 0 || Hq % KVH != 0 || max_q_len <= 0 || max_ctx <= 0) return 0;
+  return dsp_detail::ragged_workspace_bytes(B, KVH, Hq / KVH, D, max_q_len, max_ctx);
+}
+
+extern "C" int dsp_paged_mq_attention_ragged(
+    const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k_cache,
+    const void* v_cache, int64_t num_slots, int64_t kv_stride_slot, int64_t kv_stride_head,
+    const int32_t* block_table, int64_t bt_stride, int32_t block_size, const int32_t* cu_q,
+    const int32_t* ctx_lens, int32_t B, int32_t Hq, int32_t KVH, int32_t D, float scale,
+    int32_t max_q_len, int32_t max_ctx, void* workspace, size_t workspace_bytes, void* out,
+    int64_t o_stride_t, int64_t o_stride_h, int32_t dtype, int32_t* err_count,
+    dsp_stream_t stream) {
+  DSP_HOST_CHECK(q && k_cache && v_cache && block_table && cu_q && ctx_lens && out, DSP_EINVAL);
+  DSP_HOST_CHECK(B >= 0 && Hq > 0 && KVH > 0 && Hq % KVH == 0 && max_q_len >= 0 && max_ctx >= 0 &&
+                     num_slots >= 0,
+                 DSP_EINVAL);
+  DSP_HOST_CHECK(dtype == DSP_BF16 || dtype == DSP_F16, DSP_EUNSUPPORTED);
+  DSP_HOST_CHECK(dsp_is_pow2(block_size) && bt_stride * block_size >= max_ctx, DSP_EINVAL);
+  if (B == 0 || max_q_len == 0) return DSP_OK;
+  DSP_HOST_CHECK(q_stride_t % 8 == 0 && q_stride_h % 8 == 0 && kv_stride_slot % 8 == 0 &&
+                     kv_stride_head % 8 == 0 && dsp_aligned(q, 16) && dsp_aligned(k_cache, 16) &&
+                     dsp_aligned(v_cache, 16),
+                 DSP_EALIGN);
+  const int G = Hq / KVH;
+  const size_t need = dsp_detail::ragged_workspace_bytes(B, KVH, G, D, max_q_len, max_ctx);
+  DSP_HOST_CHECK(need > 0, DSP_EUNSUPPORTED);
+  DSP_HOST_CHECK(workspace != nullptr && workspace_bytes >= need, DSP_EWORKSPACE);
+  DSP_HOST_CHECK(dsp_aligned(workspace, 16), DSP_EALIGN);
+  return dsp_detail::prefill_ragged(
+      static_cast<const uint16_t*>(q), q_stride_t, q_stride_h,
+      static_cast<const uint16_t*>(k_cache), static_cast<const uint16_t*>(v_cache), num_slots,
+      kv_stride_slot, kv_stride_head, block_table, bt_stride, block_size, cu_q, ctx_lens, B, KVH, G,
+      D, scale * 1.4426950408889634f, max_q_len, max_ctx, static_cast<float*>(workspace),
+      static_cast<uint16_t*>(out), o_stride_t, o_stride_h, dtype == DSP_F16, err_count,
+      static_cast<hipStream_t>(stream));
+}
+
 extern "C" int dsp_paged_mq_attention_shared_prefix(
     const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k_cache,
     const void* v_cache, int64_t num_slots, int64_t kv_stride_slot, int64_t kv_stride_head,

@@ -82,26 +82,19 @@ __device__ __forceinline__ void dma16(const void* sbase, uint32_t voff, uint32_t
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4i16 lds_v4i16_t;
 
-// kShared: a shared-prefix (cascade) launch, two kinds of workgroup in one grid.  For
-// x < prefix_x (per KV head) a workgroup is a prefix tile: packed row r is token r / G of
-// the whole batch (every sequence's queries), query head kvh*G + r % G; the keys are the
-// first prefix_tokens of block-table row 0, which every sequence shares and every query
-// sees whole (no mask); partition `part` covers keys [part*P, part*P + P) and is written,
-// for every row, to that row's own (sequence, 16-row tile) slot of the merge layout.  The
-// other workgroups are suffix tiles: one sequence's rows over one partition of P of its
-// keys from prefix_tokens on (causal), numbered on from the prefix's partitions (keys
-// [part*P, part*P + P) again).  Both kinds run side by side; the merge then folds every
-// partition up to a row's last visible key, as for an unshared launch.
-template <typename Tag, int D, bool kShared>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2))) void paged_prefill_kernel(
-    const uint16_t* __restrict__ q, int64_t qst, int64_t qsh, const uint16_t* __restrict__ kc,
-    const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
-    const int32_t* __restrict__ bt, int64_t bt_stride, int32_t log2_bs,
-    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ ctx_lens, int32_t max_ctx,
-    int32_t G, float scale_log2, int32_t P, int32_t num_parts, int32_t tiles16_max,
-    float* __restrict__ ws_acc, float* __restrict__ ws_ml, uint16_t* __restrict__ out,
-    int64_t ost, int64_t osh, int32_t* __restrict__ err_count, int32_t nseq,
-    int32_t prefix_tokens, int32_t ws_parts, int32_t prefix_x) {
+// One workgroup's keys [kbeg, kfin) of one (sequence, KV head), in 64-key chunks, for the rows
+// whose Q^T operands are in qop: the running (max, sum, accumulator) of each row is updated.
+// lim: the last key this lane's row sees; lim_min: the least of them in the wave (uniform).
+// blk_first / blk_second: this wave's block ids of the first two chunks, loaded early and
+// unclamped.  Every wave of the workgroup calls it (it has barriers).
+template <typename Tag, int D, bool kNonTemporal, typename Lds>
+__device__ __forceinline__ void attend_chunks(
+    Lds& lds, int32_t (&s_bad)[2][kWaves], const uint16_t* __restrict__ kc,
+    const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t head_off,
+    const int32_t* __restrict__ bt, int64_t bt_row, int32_t log2_bs, int kbeg, int kfin, int lim,
+    int lim_min, bool wave_has_rows, const dsp_u32x4 (&qop)[D / 16], float scale_log2,
+    int32_t blk_first, int32_t blk_second, float& m, float& lpart, f32x16 (&acc)[D / 32],
+    bool& any_bad) {
   constexpr int NKS = D / 16;        // 16-dim steps of the score MFMA
   constexpr int NDT = D / 32;        // 32-dim output tiles
   constexpr int CPR = D / 8;         // 16-byte chunks per K/V row
@@ -109,126 +102,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
   constexpr int SLAB = kChunk * ROWB;            // one K (or V) chunk
   constexpr int RPI = 1024 / ROWB;               // rows per 1-KiB DMA load
   constexpr int LPW = SLAB / 1024 / kWaves;      // DMA loads per wave per slab
-  static_assert(LPW >= 1, "every wave loads part of a chunk");
-  __shared__ __attribute__((aligned(1024))) char lds[2][2][SLAB];  // [buffer][K | V]
-  __shared__ int32_t s_cu[kShared ? kMaxSharedSeqs + 1 : 1];         // cu_q, prefix pass
-  // D 256: which 16-key groups of each buffer's chunk have a block id outside the cache
-  // (their keys are masked, as on the generic kernel that serves unaligned 256-wide heads)
-  constexpr bool kMaskBad = D > 128;
-  __shared__ int32_t s_bad[2][kWaves];
-  // and its probabilities stay fp32, as that kernel's are: two 16-bit operands (pack8; one
+  // D 256: s_bad says which 16-key groups of each buffer's chunk have a block id outside the
+  // cache (their keys are masked, as on the generic kernel that serves unaligned 256-wide
+  // heads), and probabilities stay fp32, as that kernel's are: two 16-bit operands (pack8; one
   // 16-bit operand would be 16 % faster and moves the error against 64 bits from 2.8e-3 to
   // 3.3e-3).  128 KiB of LDS: one workgroup per CU, a wave's accumulators in AGPRs.
-  constexpr bool kSplitP = D > 128;
-
-  // XCD-aware order: the dispatcher hands workgroup `lin` to XCD lin % 8.  Each XCD gets a
-  // contiguous range of logical ids, so the tiles of one (sequence, KV head) -- which read
-  // the same K/V -- run on one XCD and share its L2.  Within a (sequence, KV head) the
-  // heaviest tiles (the last rows see the most keys) come first.
-  const int X = gridDim.x, KVH = gridDim.y;
-  const int64_t nwg = int64_t(X) * KVH * gridDim.z;
-  const int64_t lin = blockIdx.x + int64_t(X) * (blockIdx.y + int64_t(KVH) * blockIdx.z);
-  const int64_t q8 = nwg / 8, r8 = nwg % 8, xcd = lin % 8, pos = lin / 8;
-  const int64_t lg = xcd < r8 ? xcd * (q8 + 1) + pos : r8 * (q8 + 1) + (xcd - r8) * q8 + pos;
-  const int xl = int(lg % X);
-  const int kvh = int((lg / X) % KVH);
-  int b = int(lg / X / KVH), part, tile;
-  bool pre = false;  // a prefix tile of a shared-prefix launch
-  if constexpr (kShared) {
-    pre = xl < prefix_x;
-    if (pre) {
-      part = xl % num_parts;
-      tile = prefix_x / num_parts - 1 - xl / num_parts;
-    } else {
-      // suffix tiles: per sequence tiles_s row tiles x nsp partitions of its keys past the
-      // prefix (partition index continues the prefix's: key range [part*P, part*P + P))
-      const int first = prefix_tokens / P, nsp = ws_parts - first;
-      const int per_seq = (X - prefix_x) / nseq, idx = xl - prefix_x;
-      const int tiles_s = per_seq / nsp, k = idx % per_seq;
-      b = idx / per_seq;
-      tile = tiles_s - 1 - k / nsp;
-      part = first + k % nsp;
-    }
-  } else {
-    const int ntiles = X / num_parts;
-    part = xl % num_parts;
-    tile = ntiles - 1 - xl / num_parts;
-  }
-  // The first two chunks' block ids are loaded now, beside the lengths below: chunk keys
-  // start at part * P whatever the lengths are (clamped into the table's width here; a
-  // wave whose rows turn out to start past the partition's end reloads its id below).
-  const int wave_e = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t bt_row_e = int64_t(b) * bt_stride;
-  const int key_cap = max(max_ctx - 1, 0);
-  auto early_blk = [&](int t) {
-    return bt[bt_row_e + (min(t + 16 * wave_e, key_cap) >> log2_bs)];
-  };
-  int32_t blk_first = early_blk(part * P), blk_second = early_blk(part * P + kChunk);
-  int q0, qlen, ctx, kend = 0;
-  if (pre) {
-    // all tokens of the batch; the causal limit never binds (ctx - qlen + qi >= max_ctx)
-    q0 = 0;
-    qlen = cu_q[nseq];
-    ctx = qlen + max_ctx;
-    kend = prefix_tokens;
-    // staged for the epilogue's row -> sequence search (published by the first chunk's
-    // barrier: every workgroup that gets past the checks below runs at least one chunk)
-    for (int i = threadIdx.x; i <= nseq; i += kThreads) s_cu[i] = cu_q[i];
-  } else {
-    q0 = cu_q[b];
-    qlen = cu_q[b + 1] - q0;
-    ctx = ctx_lens[b];
-  }
-  const int rows = qlen * G;
-  const int r0 = tile * kRows;
-  if (qlen <= 0 || r0 >= rows) return;
-  if (!pre) {
-    // bad lengths (and, in a shared-prefix launch, queries that start inside the prefix):
-    // counted once, the rows are zeros
-    if (ctx > max_ctx || ctx < qlen || (kShared && ctx - qlen < prefix_tokens)) {
-      if (!kShared && part != 0) return;
-      if (threadIdx.x == 0 && tile == 0 && kvh == 0 && err_count) atomicAdd(err_count, 1);
-      for (int i = threadIdx.x; i < kRows * D; i += kThreads) {
-        const int rr = r0 + i / D;
-        if (rr < rows)
-          out[int64_t(q0 + rr / G) * ost + int64_t(kvh * G + rr % G) * osh + i % D] = 0;
-      }
-      return;
-    }
-    const int r_last = min(r0 + kRows - 1, rows - 1);
-    kend = ctx - qlen + r_last / G + 1;  // keys any row of the tile sees
-  }
-  // partition `part` covers keys [part*P, part*P + P) of the tile's visible range (a
-  // suffix tile's partitions start at the prefix's end, which is a multiple of P)
-  const int kbeg = part * P;
-  if (kbeg >= kend) return;
-  const int kfin = min(kbeg + P, kend);
-
+  constexpr bool kMaskBad = D > 128, kSplitP = D > 128;
+  static_assert(LPW >= 1, "every wave loads part of a chunk");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hl = lane >> 5;        // lane half: key sub-range of the operands
   const int col = lane & 31;       // this lane's row within the wave
-  const int r = r0 + 32 * wave + col;
-  const bool row_ok = r < rows;
-  const bool wave_has_rows = r0 + 32 * wave < rows;  // wave-uniform
-  const int qi = row_ok ? r / G : 0;
-  const int h = kvh * G + (row_ok ? r % G : 0);
-  // Keys 0..lim are visible to this row (causal limit, and the partition's end); lim_min
-  // is the smallest limit among the wave's rows (its first row), wave-uniform.  Rows past
-  // `rows` have q = 0: finite scores, never stored.
-  const int lim = min(ctx - qlen + qi, kfin - 1);
-  const int lim_min = min(ctx - qlen + (r0 + 32 * wave) / G, kfin - 1);
-  const int64_t bt_row = int64_t(b) * bt_stride;
-  const int64_t head_off = int64_t(kvh) * kvs_head;
   const int bmask = (1 << log2_bs) - 1;
-
-  // Q^T (B operand): lane holds dims 16*ks + 8*hl .. +8 of its row.
-  dsp_u32x4 qop[NKS];
-#pragma unroll
-  for (int ks = 0; ks < NKS; ++ks)
-    qop[ks] = row_ok ? *reinterpret_cast<const dsp_u32x4*>(q + int64_t(q0 + qi) * qst +
-                                                           int64_t(h) * qsh + 16 * ks + 8 * hl)
-                     : dsp_u32x4{0u, 0u, 0u, 0u};
 
   // K/V chunk rows into LDS: load j of this wave covers rows (wave*LPW + j)*RPI ..; lane l
   // fills slot l % CPR of row l / CPR with global chunk slot ^ swz(row).  K rows are
@@ -256,7 +141,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
   auto load_blk = [&](int t0) {
     return bt[bt_row + (min(t0 + 16 * wave, kfin - 1) >> log2_bs)];
   };
-  bool any_bad = false;  // (wave-uniform) a block id of visible keys lay outside the cache
   auto issue = [&](int buf, int t0, int32_t blk_v) {
     const int32_t blk = __builtin_amdgcn_readfirstlane(blk_v);
     // D 256: rows past kfin repeat the last key's (the generic kernel reads no other slot)
@@ -279,25 +163,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
         for (int j = 0; j < LPW; ++j) {
           const int rw = j * RPI + lane / CPR, row = 16 * wave + rw, sl = lane % CPR;
           const uint32_t ro = uint32_t(min(rw, kfin - 1 - first) * kvs_slot * 2);
-          dma16<kShared>(kb, ro + 16 * (sl ^ kswz(row)), m0 + j * 1024);
-          dma16<kShared>(vb, ro + 16 * (sl ^ vswz(row)), m0 + SLAB + j * 1024);
+          dma16<kNonTemporal>(kb, ro + 16 * (sl ^ kswz(row)), m0 + j * 1024);
+          dma16<kNonTemporal>(vb, ro + 16 * (sl ^ vswz(row)), m0 + SLAB + j * 1024);
         }
         return;
       }
     }
 #pragma unroll
     for (int j = 0; j < LPW; ++j) {
-      dma16<kShared>(kb, koff[j], m0 + j * 1024);
-      dma16<kShared>(vb, voff[j], m0 + SLAB + j * 1024);
+      dma16<kNonTemporal>(kb, koff[j], m0 + j * 1024);
+      dma16<kNonTemporal>(vb, voff[j], m0 + SLAB + j * 1024);
     }
   };
-
-  float m = -INFINITY, lpart = 0.f;
-  f32x16 acc[NDT];
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc[dt][j] = 0.f;
 
   const int nch = (kfin - kbeg + kChunk - 1) / kChunk;
   // block ids run one chunk ahead of the DMAs, which run one chunk ahead of the MFMAs; the
@@ -417,6 +294,153 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
       }
     }
   }
+}
+
+// kShared: a shared-prefix (cascade) launch, two kinds of workgroup in one grid.  For
+// x < prefix_x (per KV head) a workgroup is a prefix tile: packed row r is token r / G of
+// the whole batch (every sequence's queries), query head kvh*G + r % G; the keys are the
+// first prefix_tokens of block-table row 0, which every sequence shares and every query
+// sees whole (no mask); partition `part` covers keys [part*P, part*P + P) and is written,
+// for every row, to that row's own (sequence, 16-row tile) slot of the merge layout.  The
+// other workgroups are suffix tiles: one sequence's rows over one partition of P of its
+// keys from prefix_tokens on (causal), numbered on from the prefix's partitions (keys
+// [part*P, part*P + P) again).  Both kinds run side by side; the merge then folds every
+// partition up to a row's last visible key, as for an unshared launch.
+template <typename Tag, int D, bool kShared>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2))) void paged_prefill_kernel(
+    const uint16_t* __restrict__ q, int64_t qst, int64_t qsh, const uint16_t* __restrict__ kc,
+    const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
+    const int32_t* __restrict__ bt, int64_t bt_stride, int32_t log2_bs,
+    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ ctx_lens, int32_t max_ctx,
+    int32_t G, float scale_log2, int32_t P, int32_t num_parts, int32_t tiles16_max,
+    float* __restrict__ ws_acc, float* __restrict__ ws_ml, uint16_t* __restrict__ out,
+    int64_t ost, int64_t osh, int32_t* __restrict__ err_count, int32_t nseq,
+    int32_t prefix_tokens, int32_t ws_parts, int32_t prefix_x) {
+  constexpr int NKS = D / 16;        // 16-dim steps of the score MFMA
+  constexpr int NDT = D / 32;        // 32-dim output tiles
+  constexpr int SLAB = kChunk * 2 * D;  // one K (or V) chunk
+  __shared__ __attribute__((aligned(1024))) char lds[2][2][SLAB];  // [buffer][K | V]
+  __shared__ int32_t s_cu[kShared ? kMaxSharedSeqs + 1 : 1];         // cu_q, prefix pass
+  __shared__ int32_t s_bad[2][kWaves];
+
+  // XCD-aware order: the dispatcher hands workgroup `lin` to XCD lin % 8.  Each XCD gets a
+  // contiguous range of logical ids, so the tiles of one (sequence, KV head) -- which read
+  // the same K/V -- run on one XCD and share its L2.  Within a (sequence, KV head) the
+  // heaviest tiles (the last rows see the most keys) come first.
+  const int X = gridDim.x, KVH = gridDim.y;
+  const int64_t nwg = int64_t(X) * KVH * gridDim.z;
+  const int64_t lin = blockIdx.x + int64_t(X) * (blockIdx.y + int64_t(KVH) * blockIdx.z);
+  const int64_t q8 = nwg / 8, r8 = nwg % 8, xcd = lin % 8, pos = lin / 8;
+  const int64_t lg = xcd < r8 ? xcd * (q8 + 1) + pos : r8 * (q8 + 1) + (xcd - r8) * q8 + pos;
+  const int xl = int(lg % X);
+  const int kvh = int((lg / X) % KVH);
+  int b = int(lg / X / KVH), part, tile;
+  bool pre = false;  // a prefix tile of a shared-prefix launch
+  if constexpr (kShared) {
+    pre = xl < prefix_x;
+    if (pre) {
+      part = xl % num_parts;
+      tile = prefix_x / num_parts - 1 - xl / num_parts;
+    } else {
+      // suffix tiles: per sequence tiles_s row tiles x nsp partitions of its keys past the
+      // prefix (partition index continues the prefix's: key range [part*P, part*P + P))
+      const int first = prefix_tokens / P, nsp = ws_parts - first;
+      const int per_seq = (X - prefix_x) / nseq, idx = xl - prefix_x;
+      const int tiles_s = per_seq / nsp, k = idx % per_seq;
+      b = idx / per_seq;
+      tile = tiles_s - 1 - k / nsp;
+      part = first + k % nsp;
+    }
+  } else {
+    const int ntiles = X / num_parts;
+    part = xl % num_parts;
+    tile = ntiles - 1 - xl / num_parts;
+  }
+  // The first two chunks' block ids are loaded now, beside the lengths below: chunk keys
+  // start at part * P whatever the lengths are (clamped into the table's width here; a
+  // wave whose rows turn out to start past the partition's end reloads its id below).
+  const int wave_e = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t bt_row_e = int64_t(b) * bt_stride;
+  const int key_cap = max(max_ctx - 1, 0);
+  auto early_blk = [&](int t) {
+    return bt[bt_row_e + (min(t + 16 * wave_e, key_cap) >> log2_bs)];
+  };
+  int32_t blk_first = early_blk(part * P), blk_second = early_blk(part * P + kChunk);
+  int q0, qlen, ctx, kend = 0;
+  if (pre) {
+    // all tokens of the batch; the causal limit never binds (ctx - qlen + qi >= max_ctx)
+    q0 = 0;
+    qlen = cu_q[nseq];
+    ctx = qlen + max_ctx;
+    kend = prefix_tokens;
+    // staged for the epilogue's row -> sequence search (published by the first chunk's
+    // barrier: every workgroup that gets past the checks below runs at least one chunk)
+    for (int i = threadIdx.x; i <= nseq; i += kThreads) s_cu[i] = cu_q[i];
+  } else {
+    q0 = cu_q[b];
+    qlen = cu_q[b + 1] - q0;
+    ctx = ctx_lens[b];
+  }
+  const int rows = qlen * G;
+  const int r0 = tile * kRows;
+  if (qlen <= 0 || r0 >= rows) return;
+  if (!pre) {
+    // bad lengths (and, in a shared-prefix launch, queries that start inside the prefix):
+    // counted once, the rows are zeros
+    if (ctx > max_ctx || ctx < qlen || (kShared && ctx - qlen < prefix_tokens)) {
+      if (!kShared && part != 0) return;
+      if (threadIdx.x == 0 && tile == 0 && kvh == 0 && err_count) atomicAdd(err_count, 1);
+      for (int i = threadIdx.x; i < kRows * D; i += kThreads) {
+        const int rr = r0 + i / D;
+        if (rr < rows)
+          out[int64_t(q0 + rr / G) * ost + int64_t(kvh * G + rr % G) * osh + i % D] = 0;
+      }
+      return;
+    }
+    const int r_last = min(r0 + kRows - 1, rows - 1);
+    kend = ctx - qlen + r_last / G + 1;  // keys any row of the tile sees
+  }
+  // partition `part` covers keys [part*P, part*P + P) of the tile's visible range (a
+  // suffix tile's partitions start at the prefix's end, which is a multiple of P)
+  const int kbeg = part * P;
+  if (kbeg >= kend) return;
+  const int kfin = min(kbeg + P, kend);
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hl = lane >> 5;        // lane half: key sub-range of the operands
+  const int col = lane & 31;       // this lane's row within the wave
+  const int r = r0 + 32 * wave + col;
+  const bool row_ok = r < rows;
+  const bool wave_has_rows = r0 + 32 * wave < rows;  // wave-uniform
+  const int qi = row_ok ? r / G : 0;
+  const int h = kvh * G + (row_ok ? r % G : 0);
+  // Keys 0..lim are visible to this row (causal limit, and the partition's end); lim_min
+  // is the smallest limit among the wave's rows (its first row), wave-uniform.  Rows past
+  // `rows` have q = 0: finite scores, never stored.
+  const int lim = min(ctx - qlen + qi, kfin - 1);
+  const int lim_min = min(ctx - qlen + (r0 + 32 * wave) / G, kfin - 1);
+  const int64_t bt_row = int64_t(b) * bt_stride;
+  const int64_t head_off = int64_t(kvh) * kvs_head;
+
+  // Q^T (B operand): lane holds dims 16*ks + 8*hl .. +8 of its row.
+  dsp_u32x4 qop[NKS];
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks)
+    qop[ks] = row_ok ? *reinterpret_cast<const dsp_u32x4*>(q + int64_t(q0 + qi) * qst +
+                                                           int64_t(h) * qsh + 16 * ks + 8 * hl)
+                     : dsp_u32x4{0u, 0u, 0u, 0u};
+
+  bool any_bad = false;  // (wave-uniform) a block id of visible keys lay outside the cache
+  float m = -INFINITY, lpart = 0.f;
+  f32x16 acc[NDT];
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[dt][j] = 0.f;
+  attend_chunks<Tag, D, kShared>(lds, s_bad, kc, vc, num_slots, kvs_slot, head_off, bt, bt_row,
+                                 log2_bs, kbeg, kfin, lim, lim_min, wave_has_rows, qop, scale_log2,
+                                 blk_first, blk_second, m, lpart, acc, any_bad);
 
   if (err_count && any_bad && lane == 0) atomicAdd(err_count, 1);  // once per wave
 
@@ -464,6 +488,390 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
     ws_ml[2 * (slot * 16 + rr)] = m;
     ws_ml[2 * (slot * 16 + rr) + 1] = lpart;
   }
+}
+
+// ---- equal shares of a ragged batch ------------------------------------------------------
+// A batch that mixes prompt chunks with decodes has few 128-row tiles for the size of its grid
+// (which the longest query block sizes for every sequence), and their keys differ widely: one
+// chunk's tiles and 24 one-row tiles, each walking its context alone, leave most of the chip
+// idle behind the longest.  Here the work is the list of (sequence, KV head, tile, 64-key
+// chunk) units, in that order, and each of W workgroups -- as many as fit the chip at once --
+// takes an equal run of it, computed on the device from the lengths (as decode_balanced.hip
+// does, so nothing waits for the host).  A tile inside one run is normalised and written; a
+// tile that crosses runs leaves a partial (128 rows' max, sum and accumulator) per run in the
+// workspace: slot 2w for worker w's first piece when it continues a tile, 2w + 1 for its last
+// when it begins one; the merge kernel's workgroup w folds the tile that worker w began.
+// 24 decodes of 100-2860 keys beside a 700-token chunk over 1501 keys: 118 -> 55 us a layer with
+// the merge (28 heads over 4 of 128), 52 -> 32 (14 over 2 of 64), 151 -> 70 (32 over 8).  The
+// merge is 8-12 us of it: a partial is 64 KiB a tile at D 128.
+constexpr int kMinChunks = 2;       // a worker gets at least this many chunks
+// Run ends this many chunks from a tile's end or less move onto it: 2 decodes and a 1000-token
+// prompt 45 -> 41 us at 2, 42 at 4, where batches of short contexts lose (4 decodes and 64
+// tokens 17 -> 19 at 2, 23 at 4).
+constexpr int kSnap = 2;
+constexpr int kMaxRaggedSeqs = 512; // every wave scans the lengths
+
+// Division by the launch's G (values below 2^24): a reciprocal and one correction step, a few
+// instructions where the compiler's division is tens; every worker runs a chain of them before
+// its first load.
+struct DivG {
+  int G;
+  float inv;
+  __device__ __forceinline__ explicit DivG(int g) : G(g), inv(1.f / float(g)) {}
+  __device__ __forceinline__ int div(int x) const {
+    int q = int(float(x) * inv);
+    const int r = x - q * G;
+    return r < 0 ? q - 1 : (r >= G ? q + 1 : q);
+  }
+  // sum of floor(k / G) over 0 <= k < x
+  __device__ __forceinline__ int floors(int x) const {
+    const int q = div(x);
+    return G * (q * (q - 1) / 2) + q * (x - q * G);
+  }
+  // sum of floor((a + 2 t) / G) over 0 <= t < n.  The sum over every k in [a, a + 2n) is this
+  // one plus the sum over the odd steps, floor((a + 2 t + 1) / G), which exceeds this one by 1
+  // where G divides a + 2 t + 1: for odd G every G-th t from t0 on; for even G every G/2-th t
+  // where a is odd, none where it is even.
+  __device__ __forceinline__ int every_other(int a, int n) const {
+    const int all = floors(a + 2 * n) - floors(a);
+    const int r = a + 1 - div(a + 1) * G;      // (a + 1) mod G
+    const int miss = r == 0 ? 0 : G - r;       // 2 t0 = miss (mod G)
+    int hits = 0;
+    if (G & 1) {
+      const int t0 = (miss & 1) ? (miss + G) / 2 : miss / 2;   // below G
+      hits = t0 < n ? div(n - 1 - t0) + 1 : 0;
+    } else if (!(miss & 1)) {
+      const int t0 = miss / 2;
+      hits = t0 < n ? div(2 * (n - 1 - t0)) + 1 : 0;
+    }
+    return (all - hits) / 2;
+  }
+};
+
+// One sequence's tiles: `tiles` of 128 packed rows (the first max_q_len queries); tile t but
+// the last sees ceil((c0 + (128 t + 127) / G + 1) / 64) = floor((a + 2 t) / G) chunks.
+struct RaggedSeq {
+  int q0, qlen, ctx, rows, tiles, a, last, units;
+  __device__ __forceinline__ int before(int t, const DivG& g) const {
+    return t > 0 ? g.every_other(a, t) : 0;
+  }
+  __device__ __forceinline__ int chunks(int t, const DivG& g) const {
+    return t + 1 < tiles ? g.div(a + 2 * t) : last;
+  }
+};
+__device__ __forceinline__ bool ragged_bad(int qlen, int ctx, int max_ctx) {
+  return qlen > 0 && (ctx < qlen || ctx > max_ctx);
+}
+__device__ __forceinline__ RaggedSeq ragged_seq(int q0, int q1, int ctx, const DivG& g,
+                                                int max_q_len, int max_ctx) {
+  RaggedSeq s;
+  s.q0 = q0;
+  s.qlen = q1 - q0;
+  s.ctx = ctx;
+  const bool none = s.qlen <= 0 || ragged_bad(s.qlen, s.ctx, max_ctx);
+  s.rows = none ? 0 : min(s.qlen, max_q_len) * g.G;
+  s.tiles = (s.rows + kRows - 1) / kRows;
+  const int c0 = none ? 0 : s.ctx - s.qlen;
+  s.a = (g.G * (c0 + kChunk) + kRows - 1) / kChunk;
+  s.last = none ? 0 : (c0 + min(s.qlen, max_q_len) - 1 + kChunk) / kChunk;
+  s.units = none ? 0 : s.before(s.tiles - 1, g) + s.last;
+  return s;
+}
+__device__ __forceinline__ RaggedSeq lane_seq(const RaggedSeq& s, int l) {
+  RaggedSeq r;
+  r.q0 = __builtin_amdgcn_readlane(s.q0, l);
+  r.qlen = __builtin_amdgcn_readlane(s.qlen, l);
+  r.ctx = __builtin_amdgcn_readlane(s.ctx, l);
+  r.rows = __builtin_amdgcn_readlane(s.rows, l);
+  r.tiles = __builtin_amdgcn_readlane(s.tiles, l);
+  r.a = __builtin_amdgcn_readlane(s.a, l);
+  r.last = __builtin_amdgcn_readlane(s.last, l);
+  r.units = __builtin_amdgcn_readlane(s.units, l);
+  return r;
+}
+__device__ __forceinline__ int wave_incl_scan(int v) {
+  const int lane = __lane_id();
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(v, d);
+    if (lane >= d) v += o;
+  }
+  return v;
+}
+
+template <typename Tag, int D>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2))) void prefill_ragged_kernel(
+    const uint16_t* __restrict__ q, int64_t qst, int64_t qsh, const uint16_t* __restrict__ kc,
+    const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
+    const int32_t* __restrict__ bt, int64_t bt_stride, int32_t log2_bs,
+    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ ctx_lens, int32_t B, int32_t KVH,
+    int32_t G, int32_t max_q_len, int32_t max_ctx, float scale_log2, float* __restrict__ ws_acc,
+    float* __restrict__ ws_ml, int32_t* __restrict__ ws_desc, uint16_t* __restrict__ out,
+    int64_t ost, int64_t osh, int32_t* __restrict__ err_count) {
+  constexpr int NKS = D / 16, NDT = D / 32, SLAB = kChunk * 2 * D;
+  __shared__ __attribute__((aligned(1024))) char lds[2][2][SLAB];
+  __shared__ int32_t s_bad[2][kWaves];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hl = lane >> 5, col = lane & 31;
+  const int lin = blockIdx.x;
+
+  // Lane l holds sequence b0 + l of the 64 the wave looks at; most batches are one such group,
+  // whose lanes' values serve the whole kernel.
+  const DivG g(G);
+  int b0 = 0;
+  RaggedSeq lane_s;
+  int incl = 0;
+  auto look = [&](int first) {
+    b0 = first;
+    const int b = min(b0 + lane, B - 1);
+    lane_s = ragged_seq(cu_q[b], cu_q[b + 1], ctx_lens[b], g, max_q_len, max_ctx);
+    if (b0 + lane >= B) lane_s.units = 0;
+    incl = wave_incl_scan(lane_s.units);
+  };
+  int total = 0;  // units per KV head
+  for (int first = 0; first < B; first += 64) {
+    look(first);
+    total += __builtin_amdgcn_readlane(incl, 63);
+    // bad lengths: counted once, the rows written as zeros, one sequence per workgroup
+    for (int b = lin; b < B; b += gridDim.x) {
+      if (b < first || b >= first + 64) continue;
+      const int l = b - first, qa = __builtin_amdgcn_readlane(lane_s.q0, l);
+      const int ql = __builtin_amdgcn_readlane(lane_s.qlen, l);
+      if (!ragged_bad(ql, __builtin_amdgcn_readlane(lane_s.ctx, l), max_ctx)) continue;
+      if (threadIdx.x == 0 && err_count) atomicAdd(err_count, 1);
+      const int row = KVH * G * D, n = min(ql, max_q_len);
+      for (int i = 0; i < n; ++i)
+        for (int e = threadIdx.x; e < row; e += kThreads)
+          out[int64_t(qa + i) * ost + int64_t(e / D) * osh + e % D] = 0;
+    }
+  }
+  const int C = total * KVH;
+  const int W = min((C + kMinChunks - 1) / kMinChunks, int(gridDim.x));
+  if (lin >= W) {
+    if (threadIdx.x == 0) ws_desc[4 * lin + 3] = 0;
+    return;
+  }
+  // XCD-aware: workgroup lin runs on XCD lin % 8; each XCD takes a contiguous run of workers,
+  // so that the tiles of one (sequence, KV head) share an L2
+  const int q8 = W / 8, r8 = W % 8, xcd = lin % 8, pos = lin / 8;
+  const int w = xcd < r8 ? xcd * (q8 + 1) + pos : r8 * (q8 + 1) + (xcd - r8) * q8 + pos;
+  // worker w's run starts at unit floor(w * C / W) (C = share * W + extra)
+  const int share = C / W, extra = C - share * W;
+  const int U = w * share + w * extra / W;
+  int left = (w + 1) * share + (w + 1) * extra / W - U;
+  int b = 0, base = 0;  // base: units (of all KV heads) before sequence b
+  for (int first = 0, pre = 0; first < B; first += 64) {
+    if (first != b0 || B > 64) look(first);
+    const uint64_t hit = __ballot(KVH * (pre + incl) > U);
+    if (hit) {
+      const int f = __builtin_amdgcn_readfirstlane(__ffsll(static_cast<unsigned long long>(hit)) - 1);
+      b = first + f;
+      base = KVH * (pre + __builtin_amdgcn_readlane(incl, f) -
+                    __builtin_amdgcn_readlane(lane_s.units, f));
+      break;
+    }
+    pre += __builtin_amdgcn_readlane(incl, 63);
+  }
+  RaggedSeq sq = lane_seq(lane_s, b - b0);
+  int kvh = 0, u = U - base;
+  for (; u >= sq.units; u -= sq.units) ++kvh;
+  // the tile of unit u: 64 candidates a step
+  int tile = 0;
+  for (int step = (sq.tiles + 63) / 64;; step = 1) {
+    const int t = tile + lane * step;
+    const bool at = t < sq.tiles && sq.before(t, g) <= u;
+    tile += (__popcll(__ballot(at)) - 1) * step;
+    if (step == 1) break;
+  }
+  tile = __builtin_amdgcn_readfirstlane(tile);
+  // Run ends within kSnap chunks of a tile's either end move onto it: a piece of one or two
+  // chunks costs its start-up and a partial of the whole tile.  (Both neighbours move their
+  // common end alike: first the beginning, then the end of the tile.)
+  int c0 = u - sq.before(tile, g);
+  // the next tile, KV head or sequence with units (false: none is left)
+  auto next_tile = [&]() {
+    c0 = 0;
+    if (++tile < sq.tiles) return true;
+    tile = 0;
+    if (++kvh < KVH) return true;
+    kvh = 0;
+    base += KVH * sq.units;
+    while (++b < B) {
+      sq = ragged_seq(cu_q[b], cu_q[b + 1], ctx_lens[b], g, max_q_len, max_ctx);
+      if (sq.units > 0) return true;
+    }
+    return false;
+  };
+  bool work = true;
+  if (c0 <= kSnap) {
+    left += c0;
+    c0 = 0;
+  } else if (sq.chunks(tile, g) - c0 <= kSnap) {
+    left -= sq.chunks(tile, g) - c0;
+    work = left > 0 && next_tile();
+  }
+  int32_t d_b = 0, d_kvh = 0, d_tile = 0, d_np = 0;
+  bool any_bad = false;
+  for (bool again = false; work; again = true) {
+    const int nch = sq.chunks(tile, g);
+    int c1 = min(nch, c0 + left);
+    if (c1 < nch) {
+      if (c1 <= kSnap) break;  // the next worker's
+      if (nch - c1 <= kSnap) c1 = nch;
+    }
+    const int r0 = tile * kRows, rows = sq.rows;
+    const int r_last = min(r0 + kRows - 1, rows - 1);
+    const int kend = sq.ctx - sq.qlen + r_last / G + 1;
+    const int kbeg = c0 * kChunk, kfin = min(c1 * kChunk, kend);
+    const int64_t bt_row = int64_t(b) * bt_stride;
+    const int32_t blk0 = bt[bt_row + (min(kbeg + 16 * wave, kfin - 1) >> log2_bs)];
+    const int32_t blk1 = bt[bt_row + (min(kbeg + kChunk + 16 * wave, kfin - 1) >> log2_bs)];
+    const int r = r0 + 32 * wave + col;
+    const bool row_ok = r < rows;
+    const bool wave_has_rows = r0 + 32 * wave < rows;
+    const int qi = row_ok ? r / G : 0;
+    const int h = kvh * G + (row_ok ? r % G : 0);
+    const int lim = min(sq.ctx - sq.qlen + qi, kfin - 1);
+    const int lim_min = min(sq.ctx - sq.qlen + (r0 + 32 * wave) / G, kfin - 1);
+    dsp_u32x4 qop[NKS];
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks)
+      qop[ks] = row_ok ? *reinterpret_cast<const dsp_u32x4*>(q + int64_t(sq.q0 + qi) * qst +
+                                                             int64_t(h) * qsh + 16 * ks + 8 * hl)
+                       : dsp_u32x4{0u, 0u, 0u, 0u};
+    float m = -INFINITY, lpart = 0.f;
+    f32x16 acc[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc[dt][j] = 0.f;
+    if (again) __syncthreads();  // every wave is done with the previous piece's buffers
+    attend_chunks<Tag, D, false>(lds, s_bad, kc, vc, num_slots, kvs_slot,
+                                 int64_t(kvh) * kvs_head, bt, bt_row, log2_bs, kbeg, kfin, lim,
+                                 lim_min, wave_has_rows, qop, scale_log2, blk0, blk1, m, lpart, acc,
+                                 any_bad);
+    lpart += dsp_shfl_xor(lpart, 32);
+    if (c0 == 0 && c1 == nch) {
+      const float inv = lpart > 0.f ? 1.f / lpart : 0.f;
+      if (row_ok) {
+        uint16_t* o = out + int64_t(sq.q0 + qi) * ost + int64_t(h) * osh;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+          for (int j = 0; j < 16; ++j)
+            o[32 * dt + 8 * (j >> 2) + 4 * hl + (j & 3)] = narrow<Tag>(acc[dt][j] * inv);
+      }
+    } else {
+      const int64_t wrow = int64_t(2 * w + (c0 == 0 ? 1 : 0)) * kRows + 32 * wave + col;
+      if (row_ok) {
+        float* dst = ws_acc + wrow * D;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+          for (int j4 = 0; j4 < 4; ++j4)
+            *reinterpret_cast<f32x4*>(dst + 32 * dt + 8 * j4 + 4 * hl) =
+                f32x4{acc[dt][4 * j4], acc[dt][4 * j4 + 1], acc[dt][4 * j4 + 2],
+                      acc[dt][4 * j4 + 3]};
+        if (hl == 0) {
+          ws_ml[2 * wrow] = m;
+          ws_ml[2 * wrow + 1] = lpart;
+        }
+      }
+      if (c0 == 0) {  // this worker began the tile: its merge is described here
+        const int end = base + kvh * sq.units + sq.before(tile, g) + nch;
+        d_b = b;
+        d_kvh = kvh;
+        d_tile = tile;
+        // the last worker whose run begins before the tile's end (less the chunks it would skip)
+        d_np = int32_t((int64_t(end - kSnap) * W - 1) / C) - w + 1;
+      }
+    }
+    left -= c1 - c0;
+    work = left > 0 && next_tile();
+  }
+  if (err_count && any_bad && lane == 0) atomicAdd(err_count, 1);  // once per wave
+  if (threadIdx.x == 0) {
+    int32_t* d = ws_desc + 4 * w;
+    d[0] = d_b;
+    d[1] = d_kvh;
+    d[2] = d_tile;
+    d[3] = d_np;
+  }
+}
+
+// Grid (workers, 128 / R): R rows of the tile that worker x began and did not finish, one
+// thread per (row, 4 dims); its pieces are loaded 16 at a time before they are folded.
+constexpr int ragged_merge_rows(int D) { return 1024 / D; }
+
+template <typename Tag, int D>
+__global__ __launch_bounds__(256) void prefill_ragged_merge_kernel(
+    const float* __restrict__ ws_acc, const float* __restrict__ ws_ml,
+    const int32_t* __restrict__ ws_desc, const int32_t* __restrict__ cu_q, int32_t G,
+    int32_t max_q_len, uint16_t* __restrict__ out, int64_t ost, int64_t osh) {
+  constexpr int TPR = D / 4, R = ragged_merge_rows(D), kBatch = 16;
+  const int64_t w = blockIdx.x;
+  const int32_t* desc = ws_desc + 4 * w;
+  const int b = desc[0], kvh = desc[1], tile = desc[2], np = desc[3];
+  if (np <= 0) return;
+  const int q0 = cu_q[b], rows = min(cu_q[b + 1] - q0, max_q_len) * G;
+  const int lr = blockIdx.y * R + threadIdx.x / TPR, d = 4 * (threadIdx.x % TPR);
+  const int r = tile * kRows + lr;
+  if (r >= rows) return;
+  float M = -INFINITY, L = 0.f;
+  f32x4 A = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int p0 = 0; p0 < np; p0 += kBatch) {
+    const int n = min(np - p0, kBatch);
+    f32x4 va[kBatch];
+    float vm[kBatch], vl[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i)
+      if (i < n) {
+        const int p = p0 + i;
+        const int64_t row = (p == 0 ? 2 * w + 1 : 2 * (w + p)) * kRows + lr;
+        va[i] = *reinterpret_cast<const f32x4*>(ws_acc + row * D + d);
+        vm[i] = ws_ml[2 * row];
+        vl[i] = ws_ml[2 * row + 1];
+      }
+    float bm = M;
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) bm = i < n ? fmaxf(bm, vm[i]) : bm;
+    const float Mu = bm == -INFINITY ? 0.f : bm;
+    const float keep = dsp_exp2(M - Mu);
+    L *= keep;
+    A *= keep;
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const float x = i < n ? dsp_exp2(vm[i] - Mu) : 0.f;
+      L = fmaf(i < n ? vl[i] : 0.f, x, L);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) A[e] = fmaf(i < n ? va[i][e] : 0.f, x, A[e]);
+    }
+    M = bm;
+  }
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  uint16_t* o = out + int64_t(q0 + r / G) * ost + int64_t(kvh * G + r % G) * osh + d;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = narrow<Tag>(A[e] * inv);
+}
+
+template <typename Tag, int D>
+int launch_ragged(int W, hipStream_t s, const uint16_t* q, int64_t qst, int64_t qsh,
+                  const uint16_t* kc, const uint16_t* vc, int64_t num_slots, int64_t kvs_slot,
+                  int64_t kvs_head, const int32_t* bt, int64_t bt_stride, int32_t log2_bs,
+                  const int32_t* cu_q, const int32_t* ctx_lens, int32_t B, int32_t KVH, int32_t G,
+                  int32_t max_q_len, int32_t max_ctx, float scale_log2, float* ws, uint16_t* out,
+                  int64_t ost, int64_t osh, int32_t* err_count) {
+  float* ws_ml = ws + int64_t(2) * W * kRows * D;
+  int32_t* ws_desc = reinterpret_cast<int32_t*>(ws_ml + int64_t(4) * W * kRows);
+  prefill_ragged_kernel<Tag, D><<<W, kThreads, 0, s>>>(
+      q, qst, qsh, kc, vc, num_slots, kvs_slot, kvs_head, bt, bt_stride, log2_bs, cu_q, ctx_lens, B,
+      KVH, G, max_q_len, max_ctx, scale_log2, ws, ws_ml, ws_desc, out, ost, osh, err_count);
+  const int st = dsp_launch_status();
+  if (st != DSP_OK) return st;
+  prefill_ragged_merge_kernel<Tag, D><<<dim3(W, kRows / ragged_merge_rows(D)), 256, 0, s>>>(
+      ws, ws_ml, ws_desc, cu_q, G, max_q_len, out, ost, osh);
+  return dsp_launch_status();
 }
 
 template <bool kShared, typename... A>
@@ -554,6 +962,62 @@ bool shared_prefix_applies(int32_t D, int32_t block_size, int32_t B, int64_t num
                            int64_t kv_stride_slot) {
   return (D == 64 || D == 128) && block_size >= 16 && B >= 1 && B <= kMaxSharedSeqs &&
          num_slots >= 16 && kv_stride_slot < (int64_t(1) << 25);
+}
+
+namespace {
+
+// workgroups that fit the chip at once: LDS and registers hold four per CU at D 64, two at 128
+int32_t ragged_workers(int32_t D) {
+  return (D <= 64 ? 4 : D <= 128 ? 2 : 1) * dsp_detail::device_cus();
+}
+
+bool ragged_applies(int32_t B, int32_t KVH, int32_t G, int32_t D, int32_t max_q_len,
+                    int32_t max_ctx) {
+  // the launch's units stay inside 31 bits, the numbers DivG divides inside 24 and their sums
+  // of floors inside 31, the tile search inside 64 steps of 64 tiles
+  const int64_t tiles = prefill_tiles(max_q_len, G);
+  const int64_t chunks = (int64_t(max_ctx) + kChunk - 1) / kChunk;
+  const int64_t reach = G * (chunks + 2) + 2 * tiles + 2;
+  return (D == 64 || D == 128 || D == 256) && B >= 1 && B <= kMaxRaggedSeqs && KVH >= 1 &&
+         max_q_len >= 1 && max_ctx >= 1 && tiles <= 4096 &&
+         reach < (int64_t(1) << 24) && reach / G * reach < (int64_t(1) << 31) &&
+         (int64_t(max_ctx) + 2 * kChunk) * G < (int64_t(1) << 31) &&
+         tiles * chunks * B * KVH < (int64_t(1) << 31);
+}
+
+}  // namespace
+
+size_t ragged_workspace_bytes(int32_t B, int32_t KVH, int32_t G, int32_t D, int32_t max_q_len,
+                              int32_t max_ctx) {
+  if (!ragged_applies(B, KVH, G, D, max_q_len, max_ctx)) return 0;
+  return size_t(ragged_workers(D)) * (size_t(2) * kRows * (D + 2) + 4) * sizeof(float);
+}
+
+int prefill_ragged(const uint16_t* q, int64_t q_stride_t, int64_t q_stride_h,
+                   const uint16_t* k_cache, const uint16_t* v_cache, int64_t num_slots,
+                   int64_t kv_stride_slot, int64_t kv_stride_head, const int32_t* block_table,
+                   int64_t bt_stride, int32_t block_size, const int32_t* cu_q,
+                   const int32_t* ctx_lens, int32_t B, int32_t KVH, int32_t G, int32_t D,
+                   float scale_log2, int32_t max_q_len, int32_t max_ctx, float* workspace,
+                   uint16_t* out, int64_t o_stride_t, int64_t o_stride_h, bool f16,
+                   int32_t* err_count, hipStream_t s) {
+  if (!ragged_applies(B, KVH, G, D, max_q_len, max_ctx) ||
+      !prefill_applies(D, block_size, kRows, num_slots, kv_stride_slot) ||
+      (D == 256 && num_slots % block_size != 0))
+    return DSP_EUNSUPPORTED;
+  auto launch = [&](auto fn) {
+    return fn(ragged_workers(D), s, q, q_stride_t, q_stride_h, k_cache, v_cache, num_slots,
+              kv_stride_slot, kv_stride_head, block_table, bt_stride, dsp_log2i(block_size), cu_q,
+              ctx_lens, B, KVH, G, max_q_len, max_ctx, scale_log2, workspace, out, o_stride_t,
+              o_stride_h, err_count);
+  };
+#define DSP_RAGGED(DD)                                                                \
+  return f16 ? launch([](auto... a) { return launch_ragged<F16Tag, DD>(a...); })      \
+             : launch([](auto... a) { return launch_ragged<Bf16Tag, DD>(a...); })
+  if (D == 64) DSP_RAGGED(64);
+  if (D == 128) DSP_RAGGED(128);
+  DSP_RAGGED(256);
+#undef DSP_RAGGED
 }
 
 }  // namespace dsp_detail

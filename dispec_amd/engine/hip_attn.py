@@ -34,6 +34,24 @@ def _mq_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx, P) -> int:
     return _lib.lib().dsp_paged_mq_workspace_bytes(B, Hq, KVH, D, max_q_len, max_ctx, P)
 
 
+@functools.lru_cache(maxsize=256)
+def _ragged_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx) -> int:
+    return _lib.lib().dsp_paged_mq_ragged_workspace_bytes(B, Hq, KVH, D, max_q_len, max_ctx)
+
+
+def _prefer_ragged(T, B, KVH, G, max_q_len) -> bool:
+    """Whether a batch of long query blocks runs with its chunks dealt out in equal shares
+    (dsp_paged_mq_attention_ragged) rather than as a grid of the longest block's tiles for
+    every sequence: when that grid has at least three times the tiles that the T query tokens
+    can fill, and is not small.  (us, grid / shares, heads 14 over 2 of 64, 28 over 4 and 32
+    over 8 of 128: 24 decodes and a 700-token chunk 52/36, 118/56, 153/69; 30 decodes and two
+    1000-token chunks 155/56, 498/135, 605/165; but 2 decodes and a 1000-token prompt, 2.9
+    times the tiles, 27/27, 41/46, 46/52, and four equal chunks 54/67, 128/155, 135/161.)"""
+    grid = KVH * B * (-(-max_q_len * G // 128))
+    filled = KVH * (B + (T - B) * G / 128)
+    return grid >= 256 and grid >= 3 * filled
+
+
 # Split-K workspaces of calls that bring none, one per (device, stream): kernels on one
 # stream run in order, so consecutive calls can share it; it grows to the largest need.
 # Under graph capture a call allocates its own (from the graph's pool), so that no captured
@@ -238,16 +256,30 @@ def paged_mq_attention(q, k_cache, v_cache, block_table, cu_q, ctx_lens, kv_grou
     else:
         P = int(partition_tokens)   # 0: the library picks the partition
     stream = _lib.stream_of(q)
-    need = _mq_ws_bytes(B, Hq, KVH, D, int(max_q_len), int(max_ctx), P)
-    if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
-        workspace = _workspace(need, q.device, stream)
-    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    ragged = 0
+    if (not sp and not P and q.dtype != torch.float32 and D in (64, 128, 256)
+            and block_size >= 16 and max_q_len * kv_groups >= 128
+            and _prefer_ragged(T, B, KVH, kv_groups, int(max_q_len))):
+        ragged = _ragged_ws_bytes(B, Hq, KVH, D, int(max_q_len), int(max_ctx))
     head = (q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(), S,
             k_cache.stride(0), k_cache.stride(1), block_table.data_ptr(), block_table.stride(0),
             block_size, cu_q.data_ptr(), ctx_lens.data_ptr(), B, Hq, KVH, D, float(scale),
             int(max_q_len), int(max_ctx))
-    tail = (_lib.ptr(workspace), ws_bytes, out.data_ptr(), out.stride(0), out.stride(1),
-            _lib.dtype_code(q.dtype), _lib.ptr(err), stream)
+    tail = (out.data_ptr(), out.stride(0), out.stride(1), _lib.dtype_code(q.dtype),
+            _lib.ptr(err), stream)
+    if ragged:
+        # up to 67 MB whatever the batch: taken from torch's stream-ordered allocator per call
+        parts = torch.empty(ragged // 4, dtype=torch.float32, device=q.device)
+        st = L.dsp_paged_mq_attention_ragged(*head, parts.data_ptr(), ragged, *tail)
+        # a pool or rows it does not take: the grid of fixed partitions below
+        if st not in (_lib.DSP_EUNSUPPORTED, _lib.DSP_EALIGN):
+            _lib.check(st, "dsp_paged_mq_attention_ragged")
+            return out
+    need = _mq_ws_bytes(B, Hq, KVH, D, int(max_q_len), int(max_ctx), P)
+    if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
+        workspace = _workspace(need, q.device, stream)
+    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    tail = (_lib.ptr(workspace), ws_bytes, *tail)
     if sp:
         _lib.check(L.dsp_paged_mq_attention_shared_prefix(*head, sp, int(P), *tail),
                    "dsp_paged_mq_attention_shared_prefix")

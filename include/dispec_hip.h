@@ -310,6 +310,28 @@ int dsp_paged_mq_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
                            int64_t o_stride_h, int32_t dtype, int32_t* err_count,
                            dsp_stream_t stream);
 
+/* J4 for ragged batches: dsp_paged_mq_attention (same arguments and results, no partition) on
+ * 128-row tiles whose 64-key chunks are dealt to the workgroups in equal shares, on the device,
+ * from the lengths -- a batch that mixes prompt chunks with decodes, or has few tiles, otherwise
+ * leaves the chip idle behind its longest tile.  bf16 / fp16, D 64, 128 or 256, blocks of >= 16
+ * tokens, B <= 512 and at most 4096 tiles of 128 rows per KV head in a sequence (else
+ * DSP_EUNSUPPORTED; the workspace size is then 0, or the pool smaller than 16 slots or, at D
+ * 256, not whole blocks).  workspace: dsp_paged_mq_ragged_workspace_bytes bytes, always needed,
+ * 16-byte aligned.  Bad lengths and block ids as for dsp_paged_mq_attention on its 128-row tile
+ * (of a sequence with more than max_q_len queries the first max_q_len are computed). */
+size_t dsp_paged_mq_ragged_workspace_bytes(int32_t B, int32_t Hq, int32_t KVH, int32_t D,
+                                           int32_t max_q_len, int32_t max_ctx);
+int dsp_paged_mq_attention_ragged(const void* q, int64_t q_stride_t, int64_t q_stride_h,
+                                  const void* k_cache, const void* v_cache, int64_t num_slots,
+                                  int64_t kv_stride_slot, int64_t kv_stride_head,
+                                  const int32_t* block_table, int64_t bt_stride,
+                                  int32_t block_size, const int32_t* cu_q,
+                                  const int32_t* ctx_lens, int32_t B, int32_t Hq, int32_t KVH,
+                                  int32_t D, float scale, int32_t max_q_len, int32_t max_ctx,
+                                  void* workspace, size_t workspace_bytes, void* out,
+                                  int64_t o_stride_t, int64_t o_stride_h, int32_t dtype,
+                                  int32_t* err_count, dsp_stream_t stream);
+
 /* J4, shared prefix (cascade).  The same attention when the first prefix_tokens context
  * tokens of every sequence are the same physical blocks -- copy-on-write forks of one
  * prompt (BlockManager.fork, dispec/kv/block_manager.py:119-126) or prefix-cache hits

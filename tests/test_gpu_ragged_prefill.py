@@ -1,0 +1,139 @@
+"""Ragged batches of long query blocks in equal shares (dsp_paged_mq_attention_ragged) against
+the grid of fixed partitions that serves them otherwise, and the rule that chooses.
+
+Bound: both round fp32 results to 16 bits after summing keys in other chunks and orders, with
+probabilities rounded to 16 bits against different running maxima: each weight errs by 2^-9
+(bf16) or 2^-12 (fp16) of itself, so a row moves by at most that times sum p |v| <= max |v| on
+either side, plus one unit in the last place of the output (2^-7, 2^-10 of the value)."""
+
+import numpy as np
+import pytest
+import torch
+
+from tests._util import randn, random_block_tables
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+P_ERR = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}
+
+
+def _run(q_lens, ctx, G, KVH, D, dtype, bs=16, max_q=None, spoil=None, strided=False, max_ctx=None):
+    """(ragged, grid) outputs and error counts."""
+    from dispec_amd import _lib
+    seed = len(q_lens) + G + D
+    NB = sum(-(-max(n, 1) // bs) for n in ctx) + 2
+    tables = random_block_tables(NB, ctx, bs, seed)
+    width = max(-(-max(ctx) // bs), 1)
+    bt = torch.zeros((len(ctx), width), dtype=torch.int32)
+    for i, t in enumerate(tables):
+        bt[i, :len(t)] = torch.tensor(t, dtype=torch.int32)
+    max_ctx = max_ctx or width * bs
+    lens = torch.tensor(ctx, dtype=torch.int32)
+    if spoil:
+        spoil(bt, lens)
+    kc, vc = randn((NB * bs, KVH, D), 1, dtype).to(DEV), randn((NB * bs, KVH, D), 2, dtype).to(DEV)
+    T, Hq = sum(q_lens), G * KVH
+    q = randn((T, Hq, D), 3, dtype).to(DEV)
+    if strided:   # a view of a fused projection: rows 8 elements longer
+        buf = torch.zeros((T, Hq * D + 8), dtype=dtype, device=DEV)
+        buf[:, :Hq * D] = q.view(T, -1)
+        q = buf[:, :Hq * D].unflatten(1, (Hq, D))
+    cu = torch.tensor([0] + list(np.cumsum(q_lens)), dtype=torch.int32, device=DEV)
+    bt, lens = bt.to(DEV), lens.to(DEV)
+    max_q = max_q or max(q_lens)
+    L, res = _lib.lib(), []
+    for ragged in (True, False):
+        out = torch.full((T, Hq, D), 7.0, dtype=dtype, device=DEV)
+        err = torch.zeros(1, dtype=torch.int32, device=DEV)
+        size = L.dsp_paged_mq_ragged_workspace_bytes if ragged else L.dsp_paged_mq_workspace_bytes
+        need = size(len(ctx), Hq, KVH, D, max_q, max_ctx, *(() if ragged else (0,)))
+        ws = torch.full((need // 4 + 1,), float("nan"), dtype=torch.float32, device=DEV)
+        fn = L.dsp_paged_mq_attention_ragged if ragged else L.dsp_paged_mq_attention
+        _lib.check(fn(q.data_ptr(), q.stride(0), q.stride(1), kc.data_ptr(), vc.data_ptr(),
+                      NB * bs, kc.stride(0), kc.stride(1), bt.data_ptr(), bt.stride(0), bs,
+                      cu.data_ptr(), lens.data_ptr(), len(ctx), Hq, KVH, D, D ** -0.5, max_q,
+                      max_ctx, *(() if ragged else (0,)), ws.data_ptr(), need, out.data_ptr(),
+                      out.stride(0), out.stride(1), _lib.dtype_code(dtype), err.data_ptr(),
+                      _lib.stream_of(q)), "mq")
+        res.append((out.float(), int(err.item())))
+    v = float(vc.float().abs().max())
+    bound = 2 * P_ERR[dtype] * v + 4 * P_ERR[dtype] * res[1][0].abs()
+    worst = float(((res[0][0] - res[1][0]).abs() - bound).max())
+    assert worst <= 0, f"{q_lens[:5]}.. {ctx[:5]}.. G={G} KVH={KVH} D={D}: {worst:.3g} over"
+    return res[0][1], res[1][1]
+
+
+BATCHES = [  # query lengths, context lengths
+    ([1] * 24 + [700], [100 + 90 * i for i in range(24)] + [1501]),
+    ([130], [130]), ([64, 1], [64, 5000]), ([200, 0, 1, 333], [200, 0, 1, 900]),
+    ([1] * 70 + [150, 1, 1], list(range(1, 71)) + [2000, 63, 65]),       # two groups of lanes
+    ([128, 129, 127, 256], [128, 193, 4000, 256]),
+    ([1, 2, 3, 1000], [64, 128, 129, 1000]),
+]
+
+
+@pytest.mark.parametrize("q_lens,ctx", BATCHES)
+@pytest.mark.parametrize("G,KVH,D", [(1, 2, 128), (2, 8, 128), (7, 2, 64), (7, 4, 128),
+                                     (3, 2, 256), (8, 1, 64), (5, 3, 128)])
+def test_ragged_is_the_grid(hip, q_lens, ctx, G, KVH, D):
+    assert _run(q_lens, ctx, G, KVH, D, torch.bfloat16) == (0, 0)
+
+
+@pytest.mark.parametrize("bs", [16, 32, 128])
+def test_block_sizes_dtype_and_strides(hip, bs):
+    assert _run(*BATCHES[0], 4, 2, 128, torch.float16, bs=bs, strided=True) == (0, 0)
+    assert _run(*BATCHES[3], 6, 2, 64, torch.float16, bs=bs, strided=True) == (0, 0)
+
+
+def test_bad_lengths_are_counted_once_and_zeroed(hip):
+    def spoil(bt, lens):
+        lens[1], lens[3] = 3000, 100     # past max_ctx; shorter than its 333 queries
+    assert _run([200, 7, 1, 333], [200, 50, 1, 900], 4, 2, 128, torch.bfloat16, spoil=spoil) == (2, 2)
+
+
+def test_query_block_longer_than_max_q_len(hip):
+    """The first max_q_len rows are computed (whole 128-row tiles of them on the grid)."""
+    assert _run([128, 1, 256], [128, 700, 300], 1, 2, 128, torch.bfloat16, max_q=256) == (0, 0)
+
+
+def test_bad_block_ids_are_counted(hip):
+    def spoil(bt, lens):
+        bt[0, 1] = 10 ** 6
+    got, want = _run([1, 300], [60, 300], 4, 2, 256, torch.bfloat16, spoil=spoil)
+    assert got > 0 and want > 0
+
+
+def test_the_rule_and_its_refusals(hip, monkeypatch):
+    """Ragged batches take the equal shares, uniform ones and explicit partitions the grid, and
+    a pool the ragged launch refuses (256-wide heads, half a block at its end) the grid."""
+    from dispec_amd import _lib
+    from dispec_amd.engine import hip_attn
+    took = []
+
+    class Spy:
+        def __getattr__(self, name):
+            fn = getattr(real, name)
+            if not name.startswith("dsp_paged_mq_attention"):
+                return fn
+            return lambda *a: (lambda st: (took.append((name, st)), st)[1])(fn(*a))
+
+    real = _lib.calls()
+    monkeypatch.setattr(_lib, "calls", lambda: Spy())
+
+    def call(q_lens, ctx, G=4, KVH=8, D=128, slots=None, **kw):
+        took.clear()
+        n = len(ctx)
+        bt = torch.arange(n * 64, dtype=torch.int32, device=DEV).view(n, 64) % 64
+        kc = torch.zeros((slots or 1024, KVH, D), dtype=torch.bfloat16, device=DEV)
+        q = torch.zeros((sum(q_lens), G * KVH, D), dtype=torch.bfloat16, device=DEV)
+        cu = torch.tensor([0] + list(np.cumsum(q_lens)), dtype=torch.int32, device=DEV)
+        hip_attn.paged_mq_attention(q, kc, kc, bt, cu, torch.tensor(ctx, dtype=torch.int32,
+                                    device=DEV), G, max_q_len=max(q_lens), max_ctx=1024, **kw)
+        torch.cuda.synchronize()
+        return [(n.replace("dsp_paged_mq_attention", ""), st) for n, st in took]
+
+    mixed = ([1] * 20 + [512], [600] * 20 + [1000])
+    assert call(*mixed) == [("_ragged", 0)]
+    assert call(*mixed, partition_tokens=256) == [("", 0)]
+    assert call([256] * 4, [1000] * 4) == [("", 0)]
+    assert call(*mixed, G=2, D=256, slots=1016) == [("_ragged", _lib.DSP_EUNSUPPORTED), ("", 0)]
