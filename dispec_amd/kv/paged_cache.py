@@ -195,30 +195,34 @@ class PagedKVCache:
         return self.slots_for_positions(block_ids, pos)
 
     def block_table(self, tables: list[list[int]], width: int | None = None) -> torch.Tensor:
-        """Device int32 [len(tables), width] block table, padded with zeros."""
-        return self._upload_tables(tables, [], width)[0]
+        """Device int32 [len(tables), width] block table, padded with zeros, complete on
+        return: a caller may read it on any stream."""
+        return self._upload_tables(tables, [], width, wait=True)[0]
 
-    def _upload_tables(self, tables: list[list[int]], cu: list[int],
-                       width: int | None = None) -> tuple[torch.Tensor, torch.Tensor]:
+    def _upload_tables(self, tables: list[list[int]], cu: list[int], width: int | None = None,
+                       wait: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
         """Device block table (int32 [len(tables), width], padded with zeros) and token offsets
         (int64 [len(cu)]) in one copy from pinned memory, which waits for nothing: a copy from
         pageable memory would hold the host until the stream's earlier kernels are done, and
         the launches after it would find the GPU idle (export, map and import of a 1023-token
         prompt: 400 -> 339 us).  The staging goes back to torch's host allocator, which keeps
-        it from reuse until the copy is done."""
+        it from reuse until the copy is done; the result is for the current stream only.  With
+        `wait`, or under graph capture (where a replay would copy whatever the staging holds
+        by then, so the copy is left to fail as any pageable one does), the copy is pageable."""
+        wait = wait or torch.cuda.is_current_stream_capturing()
         width = max([len(t) for t in tables] + [1]) if width is None else width
         for i, ids in enumerate(tables):
             if len(ids) > width:
                 raise ValueError(f"sequence {i} has {len(ids)} blocks, table width {width}")
         n_cu = 2 * len(cu)     # int64 offsets first, so that they are aligned
-        host = torch.zeros(n_cu + len(tables) * width, dtype=torch.int32, pin_memory=True)
+        host = torch.zeros(n_cu + len(tables) * width, dtype=torch.int32, pin_memory=not wait)
         if cu:
             host[:n_cu].view(torch.int64).copy_(torch.tensor(cu, dtype=torch.long))
         rows = host[n_cu:].view(len(tables), width)
         for i, ids in enumerate(tables):
             if ids:
                 rows[i, :len(ids)] = torch.tensor(ids, dtype=torch.int32)
-        dev = host.to(self.key.device, non_blocking=True)
+        dev = host.to(self.key.device, non_blocking=not wait)
         return dev[n_cu:].view(len(tables), width), dev[:n_cu].view(torch.int64)
 
     # -- whole-sequence export / import (P/D disaggregation, escalation) ------------------

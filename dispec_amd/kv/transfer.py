@@ -466,7 +466,7 @@ class CrossModelKVMap:
         if cache.dtype != torch.bfloat16:
             raise ValueError("map_into fills bf16 caches")
         cache._check_blocks(block_ids, T)
-        table = cache.block_table([block_ids])
+        table = cache._upload_tables([block_ids], [])[0]
         kv = H * D
         content = _rope(k, *source_rope, direction=-1, out_dtype=torch.bfloat16)
         vals = v.to(torch.bfloat16).contiguous()
