@@ -87,7 +87,7 @@ typedef __attribute__((address_space(3))) v4i16 lds_v4i16_t;
 // lim: the last key this lane's row sees; lim_min: the least of them in the wave (uniform).
 // blk_first / blk_second: this wave's block ids of the first two chunks, loaded early and
 // unclamped.  Every wave of the workgroup calls it (it has barriers).
-template <typename Tag, int D, bool kNonTemporal, typename Lds>
+template <typename Tag, int D, bool kNonTemporal, bool kMaskBad, bool kSplitP, typename Lds>
 __device__ __forceinline__ void attend_chunks(
     Lds& lds, int32_t (&s_bad)[2][kWaves], const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t head_off,
@@ -102,12 +102,12 @@ __device__ __forceinline__ void attend_chunks(
   constexpr int SLAB = kChunk * ROWB;            // one K (or V) chunk
   constexpr int RPI = 1024 / ROWB;               // rows per 1-KiB DMA load
   constexpr int LPW = SLAB / 1024 / kWaves;      // DMA loads per wave per slab
-  // D 256: s_bad says which 16-key groups of each buffer's chunk have a block id outside the
-  // cache (their keys are masked, as on the generic kernel that serves unaligned 256-wide
-  // heads), and probabilities stay fp32, as that kernel's are: two 16-bit operands (pack8; one
+  // kMaskBad: s_bad says which 16-key groups of each buffer's chunk have a block id outside the
+  // cache (their keys are masked, as on the 16-row tiles and on the generic kernel that serves
+  // unaligned 256-wide heads), and no slot past kfin is read.
+  // kSplitP: probabilities stay fp32: two 16-bit operands (pack8).  D 256 (as on the generic kernel; one
   // 16-bit operand would be 16 % faster and moves the error against 64 bits from 2.8e-3 to
   // 3.3e-3).  128 KiB of LDS: one workgroup per CU, a wave's accumulators in AGPRs.
-  constexpr bool kMaskBad = D > 128, kSplitP = D > 128;
   static_assert(LPW >= 1, "every wave loads part of a chunk");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -143,7 +143,7 @@ __device__ __forceinline__ void attend_chunks(
   };
   auto issue = [&](int buf, int t0, int32_t blk_v) {
     const int32_t blk = __builtin_amdgcn_readfirstlane(blk_v);
-    // D 256: rows past kfin repeat the last key's (the generic kernel reads no other slot)
+    // kMaskBad: rows past kfin repeat the last key's (a stale row there may hold anything)
     const int first = kMaskBad ? min(t0 + 16 * wave, kfin - 1) : t0 + 16 * wave;
     int64_t slot0 = int64_t(blk) * (bmask + 1) + (first & bmask);
     if (blk < 0 || (int64_t(blk) + 1) * (bmask + 1) > num_slots) {
@@ -438,7 +438,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
   for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[dt][j] = 0.f;
-  attend_chunks<Tag, D, kShared>(lds, s_bad, kc, vc, num_slots, kvs_slot, head_off, bt, bt_row,
+  attend_chunks<Tag, D, kShared, (D > 128), (D > 128)>(lds, s_bad, kc, vc, num_slots, kvs_slot, head_off, bt, bt_row,
                                  log2_bs, kbeg, kfin, lim, lim_min, wave_has_rows, qop, scale_log2,
                                  blk_first, blk_second, m, lpart, acc, any_bad);
 
@@ -501,6 +501,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
 // tile that crosses runs leaves a partial (128 rows' max, sum and accumulator) per run in the
 // workspace: slot 2w for worker w's first piece when it continues a tile, 2w + 1 for its last
 // when it begins one; the merge kernel's workgroup w folds the tile that worker w began.
+// Verifies of 17 to 127 rows, whose 16-row tiles would each read the keys: 32 of 5 over 500-4000
+// keys 86 -> 41 us (28 heads over 4).
 // 24 decodes of 100-2860 keys beside a 700-token chunk over 1501 keys: 118 -> 55 us a layer with
 // the merge (28 heads over 4 of 128), 52 -> 32 (14 over 2 of 64), 151 -> 70 (32 over 8).  The
 // merge is 8-12 us of it: a partial is 64 KiB a tile at D 128.
@@ -599,7 +601,10 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
   return v;
 }
 
-template <typename Tag, int D>
+// kSplitP: blocks below 128 rows (verify), which the 16-row tiles would serve: their running
+// maximum is exact, here it lags by up to 2^8, and one 16-bit probability would err 4 % more
+// (3.1e-3 -> 3.2e-3 against 64 bits, 32 verifies of 28 heads over 4).
+template <typename Tag, int D, bool kSplitP>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2))) void prefill_ragged_kernel(
     const uint16_t* __restrict__ q, int64_t qst, int64_t qsh, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
@@ -747,7 +752,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
 #pragma unroll
       for (int j = 0; j < 16; ++j) acc[dt][j] = 0.f;
     if (again) __syncthreads();  // every wave is done with the previous piece's buffers
-    attend_chunks<Tag, D, false>(lds, s_bad, kc, vc, num_slots, kvs_slot,
+    attend_chunks<Tag, D, false, true, kSplitP>(lds, s_bad, kc, vc, num_slots, kvs_slot,
                                  int64_t(kvh) * kvs_head, bt, bt_row, log2_bs, kbeg, kfin, lim,
                                  lim_min, wave_has_rows, qop, scale_log2, blk0, blk1, m, lpart, acc,
                                  any_bad);
@@ -864,9 +869,15 @@ int launch_ragged(int W, hipStream_t s, const uint16_t* q, int64_t qst, int64_t 
                   int64_t ost, int64_t osh, int32_t* err_count) {
   float* ws_ml = ws + int64_t(2) * W * kRows * D;
   int32_t* ws_desc = reinterpret_cast<int32_t*>(ws_ml + int64_t(4) * W * kRows);
-  prefill_ragged_kernel<Tag, D><<<W, kThreads, 0, s>>>(
-      q, qst, qsh, kc, vc, num_slots, kvs_slot, kvs_head, bt, bt_stride, log2_bs, cu_q, ctx_lens, B,
-      KVH, G, max_q_len, max_ctx, scale_log2, ws, ws_ml, ws_desc, out, ost, osh, err_count);
+  auto launch = [&](auto kernel) {
+    kernel<<<W, kThreads, 0, s>>>(q, qst, qsh, kc, vc, num_slots, kvs_slot, kvs_head, bt, bt_stride,
+                                  log2_bs, cu_q, ctx_lens, B, KVH, G, max_q_len, max_ctx, scale_log2,
+                                  ws, ws_ml, ws_desc, out, ost, osh, err_count);
+  };
+  if (D > 128 || int64_t(max_q_len) * G < kRows)
+    launch(prefill_ragged_kernel<Tag, D, true>);
+  else
+    launch(prefill_ragged_kernel<Tag, D, (D > 128)>);
   const int st = dsp_launch_status();
   if (st != DSP_OK) return st;
   prefill_ragged_merge_kernel<Tag, D><<<dim3(W, kRows / ragged_merge_rows(D)), 256, 0, s>>>(

@@ -39,14 +39,29 @@ def _ragged_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx) -> int:
     return _lib.lib().dsp_paged_mq_ragged_workspace_bytes(B, Hq, KVH, D, max_q_len, max_ctx)
 
 
-def _prefer_ragged(T, B, KVH, G, max_q_len) -> bool:
-    """Whether a batch of long query blocks runs with its chunks dealt out in equal shares
+def _prefer_ragged(T, B, KVH, G, D, max_q_len, max_ctx) -> bool:
+    """Whether a batch runs on 128-row tiles with their chunks dealt out in equal shares
     (dsp_paged_mq_attention_ragged) rather than as a grid of the longest block's tiles for
-    every sequence: when that grid has at least three times the tiles that the T query tokens
+    every sequence.
+
+    Blocks of 17 to 127 rows (verify): the grid's 16-row tiles read the keys once each, the
+    128-row tile once for all of them, which pays for its start-up and merge from about
+    256K keys of 128 (sequences times KV heads times max_ctx).  A long context over few KV
+    heads would be cut into more than 64 pieces for one merge, so it stays on the grid.
+    (us, grid / shares: 28 heads over 4, 32 verifies of 5 over 500-4000 keys 86/41; 12 over 2,
+    64 of 3-8 83/40; 32 over 8, 24 of 5 95/57; 14 over 2 of 64, 64 of 2-9 50/34; 16 over 8, 32
+    of 2-9 79/69.  Below the line: 32 over 8, 5 of 1-7 over 1109-5647 26/30; 14 over 2 of 64, 26
+    of 1-4 25/30; one of 6000 keys among 19 of 50-400, 12 over 2, 24/32, among 39 39/33.  One
+    of 30000 among 7, 12 over 2, 41/90.)
+
+    Longer blocks: when that grid has at least three times the tiles that the T query tokens
     can fill, and is not small.  (us, grid / shares, heads 14 over 2 of 64, 28 over 4 and 32
     over 8 of 128: 24 decodes and a 700-token chunk 52/36, 118/56, 153/69; 30 decodes and two
     1000-token chunks 155/56, 498/135, 605/165; but 2 decodes and a 1000-token prompt, 2.9
     times the tiles, 27/27, 41/46, 46/52, and four equal chunks 54/67, 128/155, 135/161.)"""
+    if max_q_len * G < 128:
+        return (max_q_len * G > 16 and B * KVH * max_ctx * D >= 128 * (256 << 10)
+                and (max_ctx <= 6144 or KVH >= 8 and D >= 128))
     grid = KVH * B * (-(-max_q_len * G // 128))
     filled = KVH * (B + (T - B) * G / 128)
     return grid >= 256 and grid >= 3 * filled
@@ -258,8 +273,8 @@ def paged_mq_attention(q, k_cache, v_cache, block_table, cu_q, ctx_lens, kv_grou
     stream = _lib.stream_of(q)
     ragged = 0
     if (not sp and not P and q.dtype != torch.float32 and D in (64, 128, 256)
-            and block_size >= 16 and max_q_len * kv_groups >= 128
-            and _prefer_ragged(T, B, KVH, kv_groups, int(max_q_len))):
+            and block_size >= 16 and (max_q_len * kv_groups >= 128 or S % block_size == 0)
+            and _prefer_ragged(T, B, KVH, kv_groups, D, int(max_q_len), int(max_ctx))):
         ragged = _ragged_ws_bytes(B, Hq, KVH, D, int(max_q_len), int(max_ctx))
     head = (q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(), S,
             k_cache.stride(0), k_cache.stride(1), block_table.data_ptr(), block_table.stride(0),

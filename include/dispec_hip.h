@@ -317,8 +317,8 @@ int dsp_paged_mq_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
  * tokens, B <= 512 and at most 4096 tiles of 128 rows per KV head in a sequence (else
  * DSP_EUNSUPPORTED; the workspace size is then 0, or the pool smaller than 16 slots or, at D
  * 256, not whole blocks).  workspace: dsp_paged_mq_ragged_workspace_bytes bytes, always needed,
- * 16-byte aligned.  Bad lengths and block ids as for dsp_paged_mq_attention on its 128-row tile
- * (of a sequence with more than max_q_len queries the first max_q_len are computed). */
+ * 16-byte aligned.  Bad lengths as for dsp_paged_mq_attention on its 128-row tile, keys of bad
+ * block ids counted and masked out (of a sequence with more than max_q_len queries the first max_q_len are computed). */
 size_t dsp_paged_mq_ragged_workspace_bytes(int32_t B, int32_t Hq, int32_t KVH, int32_t D,
                                            int32_t max_q_len, int32_t max_ctx);
 int dsp_paged_mq_attention_ragged(const void* q, int64_t q_stride_t, int64_t q_stride_h,

@@ -79,6 +79,37 @@ def test_ragged_is_the_grid(hip, q_lens, ctx, G, KVH, D):
     assert _run(q_lens, ctx, G, KVH, D, torch.bfloat16) == (0, 0)
 
 
+@pytest.mark.parametrize("q_lens,ctx", [
+    ([5] * 33, [200 + 61 * i for i in range(33)]), ([1, 9, 3], [1, 9, 4000]),
+    ([9] * 70, list(range(9, 79))), ([18, 2, 0, 17], [18, 65, 0, 3000])])
+@pytest.mark.parametrize("G,KVH,D", [(2, 8, 128), (7, 4, 128), (7, 2, 64), (3, 2, 256)])
+def test_short_blocks_are_the_16_row_tiles(hip, q_lens, ctx, G, KVH, D):
+    """Below 128 rows (one tile, its last chunk cut inside a block)."""
+    assert _run(q_lens, ctx, G, KVH, D, torch.bfloat16) == (0, 0)
+    assert _run(q_lens, ctx, G, KVH, D, torch.float16, strided=True) == (0, 0)
+
+
+def test_stale_rows_past_the_context_are_not_read(hip):
+    """Slots of a sequence's last block past its context may hold anything, NaN too: one
+    sequence's blocks are 0..n, its context ends inside the last."""
+    from dispec_amd import _lib
+    G, KVH, D, ctx, bs = 5, 2, 128, 200, 16
+    kc, vc = (randn((256, KVH, D), i, torch.bfloat16).to(DEV) for i in (1, 2))
+    kc[ctx:], vc[ctx:] = float("nan"), float("nan")
+    q = randn((5, G * KVH, D), 3, torch.bfloat16).to(DEV)
+    bt = torch.arange(16, dtype=torch.int32, device=DEV).view(1, 16)
+    cu, lens = (torch.tensor(x, dtype=torch.int32, device=DEV) for x in ([0, 5], [ctx]))
+    L = _lib.lib()
+    need = L.dsp_paged_mq_ragged_workspace_bytes(1, G * KVH, KVH, D, 5, 256)
+    ws, out = torch.empty(need // 4, device=DEV), torch.empty_like(q)
+    _lib.check(L.dsp_paged_mq_attention_ragged(
+        q.data_ptr(), q.stride(0), q.stride(1), kc.data_ptr(), vc.data_ptr(), 256, kc.stride(0),
+        kc.stride(1), bt.data_ptr(), 16, bs, cu.data_ptr(), lens.data_ptr(), 1, G * KVH, KVH, D,
+        D ** -0.5, 5, 256, ws.data_ptr(), need, out.data_ptr(), out.stride(0), out.stride(1),
+        _lib.dtype_code(q.dtype), None, _lib.stream_of(q)), "ragged")
+    assert bool(torch.isfinite(out).all())
+
+
 @pytest.mark.parametrize("bs", [16, 32, 128])
 def test_block_sizes_dtype_and_strides(hip, bs):
     assert _run(*BATCHES[0], 4, 2, 128, torch.float16, bs=bs, strided=True) == (0, 0)
@@ -136,4 +167,9 @@ def test_the_rule_and_its_refusals(hip, monkeypatch):
     assert call(*mixed) == [("_ragged", 0)]
     assert call(*mixed, partition_tokens=256) == [("", 0)]
     assert call([256] * 4, [1000] * 4) == [("", 0)]
+    # verify: above 16 rows and from 256K keys, on whole blocks of the pool
+    assert call([5] * 32, [1000] * 32) == [("_ragged", 0)]
+    assert call([5] * 31, [1000] * 31) == [("", 0)]
+    assert call([4] * 32, [1000] * 32) == [("", 0)]
+    assert call([5] * 32, [1000] * 32, slots=1032) == [("", 0)]
     assert call(*mixed, G=2, D=256, slots=1016) == [("_ragged", _lib.DSP_EUNSUPPORTED), ("", 0)]
