@@ -271,15 +271,16 @@ def paged_mq_attention(q, k_cache, v_cache, block_table, cu_q, ctx_lens, kv_grou
     else:
         P = int(partition_tokens)   # 0: the library picks the partition
     stream = _lib.stream_of(q)
+    max_q_len, max_ctx, rows = int(max_q_len), int(max_ctx), int(max_q_len) * kv_groups
     ragged = 0
-    if (not sp and not P and q.dtype != torch.float32 and D in (64, 128, 256)
-            and block_size >= 16 and (max_q_len * kv_groups >= 128 or S % block_size == 0)
-            and _prefer_ragged(T, B, KVH, kv_groups, D, int(max_q_len), int(max_ctx))):
-        ragged = _ragged_ws_bytes(B, Hq, KVH, D, int(max_q_len), int(max_ctx))
+    if (rows > 16 and not sp and not P and q.dtype != torch.float32 and D in (64, 128, 256)
+            and block_size >= 16 and (rows >= 128 or S % block_size == 0)
+            and _prefer_ragged(T, B, KVH, kv_groups, D, max_q_len, max_ctx)):
+        ragged = _ragged_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx)
     head = (q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(), S,
             k_cache.stride(0), k_cache.stride(1), block_table.data_ptr(), block_table.stride(0),
             block_size, cu_q.data_ptr(), ctx_lens.data_ptr(), B, Hq, KVH, D, float(scale),
-            int(max_q_len), int(max_ctx))
+            max_q_len, max_ctx)
     tail = (out.data_ptr(), out.stride(0), out.stride(1), _lib.dtype_code(q.dtype),
             _lib.ptr(err), stream)
     if ragged:
@@ -290,7 +291,7 @@ def paged_mq_attention(q, k_cache, v_cache, block_table, cu_q, ctx_lens, kv_grou
         if st not in (_lib.DSP_EUNSUPPORTED, _lib.DSP_EALIGN):
             _lib.check(st, "dsp_paged_mq_attention_ragged")
             return out
-    need = _mq_ws_bytes(B, Hq, KVH, D, int(max_q_len), int(max_ctx), P)
+    need = _mq_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx, P)
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = _workspace(need, q.device, stream)
     ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
