@@ -226,11 +226,14 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
     // Block-table windows: lane i holds the id of block wblk + i (win) and wblk + 64 + i
     // (win2).  Chunks advance by 32 keys, i.e. by at most 32 blocks, so a chunk always
     // lies within win and win2 once the windows have been advanced for its first key.
+    // No entry past max_ctx is read: a row may end there (a column-offset view of a wider
+    // table), however far apart the rows are.
     const int wsh = kMode == kSlots ? 0 : log2_bs;
+    const int wend = ((max_ctx - 1) >> wsh) + 1;
     int wblk = kb >> wsh;
     auto load_win = [&](int first) -> int32_t {
-      const int64_t j = int64_t(first) + lane;
-      return j < bt_stride ? bt[bt_row + j] : -1;
+      const int j = first + lane;
+      return j < wend ? bt[bt_row + j] : -1;
     };
     int32_t win = load_win(wblk), win2 = load_win(wblk + 64);
     auto advance = [&](int key) {

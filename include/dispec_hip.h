@@ -187,6 +187,8 @@ int dsp_kv_scatter_ordered(void* k_pool, void* v_pool, int64_t num_layers,
  *   q, out       : [B, Hq, D] with strides (q_stride_b, q_stride_h), D contiguous.
  *   k/v_cache    : one layer, [num_slots, KVH, D] with strides (kv_stride_slot,
  *                  kv_stride_head), D contiguous; same strides for K and V.
+ *   tables       : int32, row b at b * st_stride or b * bt_stride; of a row only the entries
+ *                  of its first max_ctx tokens are read (a view of a wider table may end there).
  *   ctx_lens     : int32 [B], each in [0, max_ctx].  ctx_len 0 writes zeros.
  *   partition_tokens : 0 (automatic), DSP_SPLIT_BALANCED, or a split-K partition length.
  *                  0 with a block table, D in {32, 64, 128}: max_ctx <= 512 with at most

@@ -61,3 +61,41 @@ def test_bad_slots_are_skipped_and_counted_alike(hip):
     bad = [(0, 0), (0, 31), (0, 32), (0, 1499), (1, 39), (1, 16), (5, 450), (15, 899)]
     got, want = _both(lens, 5, 4, 128, torch.bfloat16, 90, bad)
     assert got == want == len(bad) * 4        # once per slot and KV head
+
+
+@pytest.mark.parametrize("off", [1, 100, 127])
+@pytest.mark.parametrize("form", ["slots", "blocks"])
+def test_table_entries_past_max_ctx_are_not_read(hip, off, form):
+    """A table that is the last columns of a wider one: its last row ends where the buffer ends
+    (here a whole 16 MiB allocation), so the window of entries read ahead has to stop at max_ctx
+    and not at the row stride."""
+    from dispec_amd import _lib
+    B, KVH, G, D, S, stride, bs = 16, 1, 4, 64, 4096, 1 << 18, 16
+    buf = torch.full((B, stride), 2 ** 30, dtype=torch.int32, device=DEV)
+    per = 1 if form == "slots" else bs           # tokens an entry stands for
+    width = stride - off
+    max_ctx = width * per if form == "slots" else 3000 * bs
+    table = buf[:, off:] if form == "slots" else buf[:, stride - 3000:]
+    lens = [max_ctx - 3] + [700 + i for i in range(B - 2)] + [max_ctx]
+    for b, n in enumerate(lens):
+        n = -(-n // per)
+        table[b, :n] = torch.randint(0, S // per, (n,), generator=gen(b)).int().to(DEV)
+    q = randn((B, G * KVH, D), 1, torch.bfloat16).to(DEV)
+    kc, vc = (randn((S, KVH, D), s, torch.bfloat16).to(DEV) for s in (2, 3))
+    cl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    at, row = table.data_ptr(), table.stride(0)
+    where = (None, 0, bs, at, row) if form == "slots" else (at, row, bs, None, 0)
+    L, res = _lib.lib(), []
+    for P in (0, 512):
+        out, err = torch.empty_like(q), torch.zeros(1, dtype=torch.int32, device=DEV)
+        need = L.dsp_paged_decode_workspace_bytes(B, G * KVH, KVH, D, max_ctx, P)
+        ws = torch.empty(need // 4 + 1, dtype=torch.float32, device=DEV)
+        _lib.check(L.dsp_paged_decode(
+            q.data_ptr(), q.stride(0), q.stride(1), kc.data_ptr(), vc.data_ptr(), S, kc.stride(0),
+            kc.stride(1), *where, cl.data_ptr(), B, G * KVH, KVH, D, D ** -0.5, max_ctx, P,
+            ws.data_ptr(), ws.numel() * 4, out.data_ptr(), out.stride(0), out.stride(1),
+            _lib.DSP_BF16, err.data_ptr(), _lib.stream_of(q)), "decode")
+        assert int(err.item()) == 0
+        res.append(out.float())
+    bound = 2.0 ** -7 * res[1].abs() + 2.0 ** -8 * vc.float().abs().max()
+    assert bool(((res[0] - res[1]).abs() <= bound).all())
