@@ -405,7 +405,8 @@ __global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu
     }
     const int i = row / G, h = kvh * G + row % G;
     if (np == 1) {
-      out[int64_t(q0 + i) * ost + int64_t(h) * osh + d] = L > 0.f ? A * (1.f / L) : 0.f;
+      // (no keys: 0 * 0; a NaN score makes L and A NaN, and the row with them)
+      out[int64_t(q0 + i) * ost + int64_t(h) * osh + d] = A * (L > 0.f ? 1.f / L : 0.f);
     } else {
       const int64_t w = ((int64_t(b) * max_q_len + i) * Hq + h) * num_parts + part;
       ws_acc[w * D + d] = A;
