@@ -125,7 +125,7 @@ __device__ __forceinline__ int64_t active_workers(int64_t C, int num_workers) {
 // so the waves of a workgroup read the same keys' rows side by side (HG x 256 bytes of
 // each 2 KiB slot row at D 128: the pool's DRAM pages are then read HG slices at a time).
 // kMode: kPlain; kWide, the shapes that the generic kernel serves otherwise (D 256 and G > 8),
-// whose probabilities are fp32: they enter P.V as two 16-bit operands (pack8), and keys of a
+// whose probabilities are fp32: they enter P.V as three 16-bit operands (pack8), and keys of a
 // block id outside the cache are masked, as they are there; kSlots, decode by per-token slot
 // table (`bt` is the slot table), which the VALU kernel serves otherwise: fp32 probabilities as
 // in kWide, bad slots masked and each counted, as they are there.  A slot-table window holds the
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
     int32_t KVH, int32_t G, int32_t RPH, int32_t max_ctx, float scale_log2,
     int32_t num_workers, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
     uint16_t* __restrict__ out, int64_t osb, int64_t osh, int32_t* __restrict__ err_count) {
-  constexpr bool kSplitP = kMode != kPlain;
+  constexpr int kTerms = kMode == kPlain ? 1 : 3;
   constexpr int NKK = D / 32;       // 32-dim K steps of the score MFMA
   constexpr int NT = D / 16;        // 16-dim output tiles
   constexpr int CPR = D / 8;        // 16-byte chunks per K/V row
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
       cb1 = j + 1 < 64 ? __builtin_amdgcn_readlane(win, j + 1)
                        : __builtin_amdgcn_readlane(win2, j + 1 - 64);
     };
-    // kSplitP: the keys of the chunk's two 16-key halves below which block ids are valid (a
+    // kWide: the keys of the chunk's two 16-key halves below which block ids are valid (a
     // half lies in one block; its slots inside the cache are a prefix of it).  Scalars.
     int vlim[2] = {0, 0};
     auto valid_limits = [&](int t0) {
@@ -396,14 +396,14 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
       for (int st = 0; st < 2; ++st) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const float p = dsp_exp2(s[st][j] - m_use);
+          const float p = dsp_exp2(s[st][j] - m_use) * p_scale<Tag, kTerms>();
           psum += p;
           p8[4 * st + j] = p;
         }
       }
       lpart = lpart * alpha + psum;
-      dsp_u32x4 pop, plo;
-      pack8<Tag, kSplitP>(p8, pop, plo);
+      dsp_u32x4 pop[kTerms];
+      pack8<Tag, kTerms>(p8, pop);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) acc[nt] *= alpha;
 
@@ -432,8 +432,8 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
         }
         const dsp_u32x4 vop = dsp_u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]),
                                         pack2(v[6], v[7])};
-        acc[nt] = mfma32<Tag>(vop, pop, acc[nt]);
-        if constexpr (kSplitP) acc[nt] = mfma32<Tag>(vop, plo, acc[nt]);
+#pragma unroll
+        for (int k = 0; k < kTerms; ++k) acc[nt] = mfma32<Tag>(vop, pop[k], acc[nt]);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();

@@ -47,19 +47,35 @@ __device__ __forceinline__ uint32_t pack2(uint16_t lo, uint16_t hi) {
   return uint32_t(lo) | (uint32_t(hi) << 16);
 }
 
-// Eight fp32 values as a 16-bit MFMA operand and, kSplit, the operand of what that rounding
-// left over: hi + lo holds a probability to 16 bits (bf16) or 22 (fp16), so two MFMAs over
-// them give P.V as fp32 probabilities would, for the shapes whose probabilities are fp32.
-template <typename Tag, bool kSplit>
-__device__ __forceinline__ void pack8(const float (&p)[8], dsp_u32x4& hi, dsp_u32x4& lo) {
-  uint16_t h[8], l[8];
+// Eight fp32 probabilities as kTerms 16-bit MFMA operands: the first is their rounding, each
+// further one the rounding of what the ones before it left over.  Three terms hold all 24 bits
+// of an fp32 value: P.V over them is P.V of fp32 probabilities, for the shapes whose
+// probabilities are fp32 (two hold 16 bits in bf16, 22 in fp16; the third costs the 256-wide
+// prefill tile 80 -> 91 us at 4 x 200 tokens over 1999, 24 slot-table decodes 20.7 -> 21.3).  bf16 has fp32's exponents.
+// fp16 ends at 2^-24, so three terms expect p * p_scale there, p <= 1: at 2^15 the last bit
+// kept is 2^-39, whatever p's size; the row sum takes the same factor, and the division by it
+// cancels the two.
+template <typename Tag, int kTerms>
+constexpr float p_scale() {
+  return kTerms == 3 && std::is_same<Tag, F16Tag>::value ? 32768.f : 1.f;
+}
+
+template <typename Tag, int kTerms>
+__device__ __forceinline__ void pack8(const float* p, dsp_u32x4 (&t)[kTerms]) {
+  uint16_t h[kTerms][8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    h[i] = narrow<Tag>(p[i]);
-    l[i] = kSplit ? narrow<Tag>(p[i] - widen<Tag>(h[i])) : uint16_t(0);
+    float rest = p[i];
+#pragma unroll
+    for (int k = 0; k < kTerms; ++k) {
+      h[k][i] = narrow<Tag>(rest);
+      rest -= widen<Tag>(h[k][i]);
+    }
   }
-  hi = dsp_u32x4{pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7])};
-  lo = dsp_u32x4{pack2(l[0], l[1]), pack2(l[2], l[3]), pack2(l[4], l[5]), pack2(l[6], l[7])};
+#pragma unroll
+  for (int k = 0; k < kTerms; ++k)
+    t[k] = dsp_u32x4{pack2(h[k][0], h[k][1]), pack2(h[k][2], h[k][3]), pack2(h[k][4], h[k][5]),
+                     pack2(h[k][6], h[k][7])};
 }
 
 }  // namespace dsp_mfma

@@ -40,7 +40,7 @@ using namespace dsp_mfma;
 // gives zeros) and its workspace layout ws[(b * Hq + h) * num_parts + part], which its
 // combine kernel merges.
 // kSplitP: the shapes that the generic kernel serves otherwise (D 256, and decode with G > 8),
-// whose probabilities are fp32: they enter P.V as two 16-bit operands (pack8); and keys of a
+// whose probabilities are fp32: they enter P.V as three 16-bit operands (pack8); and keys of a
 // block id outside the cache are masked, as they are there.
 template <typename Tag, int D, bool kDecode, bool kSplitP>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 128 ? 2 : 3))) void paged_mq_kernel(
@@ -51,6 +51,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
     int32_t G, float scale_log2, int32_t P, int32_t num_parts, int32_t tiles_max,
     float* __restrict__ ws_acc, float* __restrict__ ws_ml, uint16_t* __restrict__ out,
     int64_t ost, int64_t osh, int32_t* __restrict__ err_count) {
+  constexpr int kTerms = kSplitP ? 3 : 1;
   constexpr int NKK = D / 32;        // 32-dim K steps of the score MFMA
   constexpr int NT = D / 16;         // 16-dim output tiles
   constexpr int CPR = D / 8;         // 16-byte chunks per K/V row
@@ -225,14 +226,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
     for (int st = 0; st < 2; ++st) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float p = dsp_exp2(s[st][j] - m_use);
+        const float p = dsp_exp2(s[st][j] - m_use) * p_scale<Tag, kTerms>();
         psum += p;
         p8[4 * st + j] = p;
       }
     }
     lpart = lpart * alpha + psum;
-    dsp_u32x4 pop, plo;
-    pack8<Tag, kSplitP>(p8, pop, plo);
+    dsp_u32x4 pop[kTerms];
+    pack8<Tag, kTerms>(p8, pop);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) acc[nt] *= alpha;
 
@@ -258,8 +259,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
       }
       const dsp_u32x4 vop = dsp_u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]),
                                    pack2(v[6], v[7])};
-      acc[nt] = mfma32<Tag>(vop, pop, acc[nt]);
-      if constexpr (kSplitP) acc[nt] = mfma32<Tag>(vop, plo, acc[nt]);
+#pragma unroll
+      for (int k = 0; k < kTerms; ++k) acc[nt] = mfma32<Tag>(vop, pop[k], acc[nt]);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();

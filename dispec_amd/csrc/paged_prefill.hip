@@ -87,7 +87,7 @@ typedef __attribute__((address_space(3))) v4i16 lds_v4i16_t;
 // lim: the last key this lane's row sees; lim_min: the least of them in the wave (uniform).
 // blk_first / blk_second: this wave's block ids of the first two chunks, loaded early and
 // unclamped.  Every wave of the workgroup calls it (it has barriers).
-template <typename Tag, int D, bool kNonTemporal, bool kMaskBad, bool kSplitP, typename Lds>
+template <typename Tag, int D, bool kNonTemporal, bool kMaskBad, int kTerms, typename Lds>
 __device__ __forceinline__ void attend_chunks(
     Lds& lds, int32_t (&s_bad)[2][kWaves], const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t head_off,
@@ -105,9 +105,9 @@ __device__ __forceinline__ void attend_chunks(
   // kMaskBad: s_bad says which 16-key groups of each buffer's chunk have a block id outside the
   // cache (their keys are masked, as on the 16-row tiles and on the generic kernel that serves
   // unaligned 256-wide heads), and no slot past kfin is read.
-  // kSplitP: probabilities stay fp32: two 16-bit operands (pack8).  D 256 (as on the generic kernel; one
-  // 16-bit operand would be 16 % faster and moves the error against 64 bits from 2.8e-3 to
-  // 3.3e-3).  128 KiB of LDS: one workgroup per CU, a wave's accumulators in AGPRs.
+  // kTerms: the 16-bit operands that hold a probability (pack8).  Three, i.e. fp32, at D 256 (as
+  // on the generic kernel; one moves the error against 64 bits from 2.8e-3 to 3.3e-3), whose
+  // 128 KiB of LDS leave one workgroup per CU, a wave's accumulators in AGPRs.
   static_assert(LPW >= 1, "every wave loads part of a chunk");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -246,7 +246,9 @@ __device__ __forceinline__ void attend_chunks(
     mx = fmaxf(mx, dsp_shfl_xor(mx, 32)) * scale_log2;  // base-2 units; -inf stays -inf
     // Lazy rescale: the running max m only moves when some row's chunk max exceeds it by
     // more than 8 (so p <= 2^8); the result is exact either way, since l and acc share m.
-    if (__builtin_amdgcn_ballot_w64(mx > m + 8.f) != 0) {
+    // (Where pack8 takes p <= 1 at most, m is the exact maximum.)
+    constexpr float kLag = p_scale<Tag, kTerms>() == 1.f ? 8.f : 0.f;
+    if (__builtin_amdgcn_ballot_w64(mx > m + kLag) != 0) {
       const float m_new = fmaxf(m, mx);
       const float alpha = m_new == -INFINITY ? 1.f : dsp_exp2(m - m_new);
       m = m_new;
@@ -257,19 +259,20 @@ __device__ __forceinline__ void attend_chunks(
     const float neg_m = m == -INFINITY ? 0.f : -m;
     // P^T operands of the four 16-key steps: step ps = 2*mt + half takes registers
     // j = 8*half .. 8*half + 7, i.e. keys 16*ps + 4*hl + {0..3, 8..11}.
-    dsp_u32x4 pop[4], plo[4];
+    // Three terms are formed step by step in the loop below: all four steps' would take 48
+    // registers, the probabilities themselves 32.
+    dsp_u32x4 pop[4][kTerms];
+    float p8[4][8];
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+    for (int ps = 0; ps < 4; ++ps) {
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        float p8[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          p8[i] = dsp_exp2(fmaf(sc[mt][8 * half + i], scale_log2, neg_m));
-          lpart += p8[i];
-        }
-        pack8<Tag, kSplitP>(p8, pop[2 * mt + half], plo[2 * mt + half]);
+      for (int i = 0; i < 8; ++i) {
+        p8[ps][i] = dsp_exp2(fmaf(sc[ps >> 1][8 * (ps & 1) + i], scale_log2, neg_m)) *
+                    p_scale<Tag, kTerms>();
+        lpart += p8[ps][i];
       }
+      if constexpr (kTerms < 3) pack8<Tag, kTerms>(p8[ps], pop[ps]);
+    }
 
     // ---- O^T += V^T . P^T.  Per 16-key step ps the V^T operand is dim 32*dt + col, K index
     // 8*hl + i <-> key 16*ps + 8*(i/4) + 4*hl + i%4 (the P^T order).  In ds_read_b64_tr_b16,
@@ -278,6 +281,7 @@ __device__ __forceinline__ void attend_chunks(
     // 4*hl + (s%16)/4, dims 32*dt + 16*((s/16)%2) + 4*(s%4) .. +3, for inst = 0, 1.
 #pragma unroll
     for (int ps = 0; ps < 4; ++ps) {
+      if constexpr (kTerms == 3) pack8<Tag, kTerms>(p8[ps], pop[ps]);
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt) {
         v4i16 vh[2];
@@ -288,9 +292,9 @@ __device__ __forceinline__ void attend_chunks(
           vh[inst] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(
               vs_lds + kr * ROWB + 16 * ((dim0 >> 3) ^ vswz(kr)) + 2 * (dim0 & 7)));
         }
-        acc[dt] = mfma32x32<Tag>(__builtin_bit_cast(dsp_u32x4, vh), pop[ps], acc[dt]);
-        if constexpr (kSplitP)
-          acc[dt] = mfma32x32<Tag>(__builtin_bit_cast(dsp_u32x4, vh), plo[ps], acc[dt]);
+#pragma unroll
+        for (int k = 0; k < kTerms; ++k)
+          acc[dt] = mfma32x32<Tag>(__builtin_bit_cast(dsp_u32x4, vh), pop[ps][k], acc[dt]);
       }
     }
   }
@@ -438,7 +442,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
   for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[dt][j] = 0.f;
-  attend_chunks<Tag, D, kShared, (D > 128), (D > 128)>(lds, s_bad, kc, vc, num_slots, kvs_slot, head_off, bt, bt_row,
+  attend_chunks<Tag, D, kShared, (D > 128), (D > 128 ? 3 : 1)>(lds, s_bad, kc, vc, num_slots, kvs_slot, head_off, bt, bt_row,
                                  log2_bs, kbeg, kfin, lim, lim_min, wave_has_rows, qop, scale_log2,
                                  blk_first, blk_second, m, lpart, acc, any_bad);
 
@@ -601,10 +605,11 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
   return v;
 }
 
-// kSplitP: blocks below 128 rows (verify), which the 16-row tiles would serve: their running
-// maximum is exact, here it lags by up to 2^8, and one 16-bit probability would err 4 % more
-// (3.1e-3 -> 3.2e-3 against 64 bits, 32 verifies of 28 heads over 4).
-template <typename Tag, int D, bool kSplitP>
+// kTerms: the operands of a probability (attend_chunks).  Two for blocks below 128 rows
+// (verify), which the 16-row tiles would serve: their running maximum is exact, here it lags by
+// up to 2^8, and one 16-bit probability would err 4 % more (3.1e-3 -> 3.2e-3 against 64 bits, 32
+// verifies of 28 heads over 4).
+template <typename Tag, int D, int kTerms>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2))) void prefill_ragged_kernel(
     const uint16_t* __restrict__ q, int64_t qst, int64_t qsh, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
@@ -752,7 +757,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
 #pragma unroll
       for (int j = 0; j < 16; ++j) acc[dt][j] = 0.f;
     if (again) __syncthreads();  // every wave is done with the previous piece's buffers
-    attend_chunks<Tag, D, false, true, kSplitP>(lds, s_bad, kc, vc, num_slots, kvs_slot,
+    attend_chunks<Tag, D, false, true, kTerms>(lds, s_bad, kc, vc, num_slots, kvs_slot,
                                  int64_t(kvh) * kvs_head, bt, bt_row, log2_bs, kbeg, kfin, lim,
                                  lim_min, wave_has_rows, qop, scale_log2, blk0, blk1, m, lpart, acc,
                                  any_bad);
@@ -875,9 +880,9 @@ int launch_ragged(int W, hipStream_t s, const uint16_t* q, int64_t qst, int64_t 
                                   ws, ws_ml, ws_desc, out, ost, osh, err_count);
   };
   if (D > 128 || int64_t(max_q_len) * G < kRows)
-    launch(prefill_ragged_kernel<Tag, D, true>);
+    launch(prefill_ragged_kernel<Tag, D, (D > 128 ? 3 : 2)>);
   else
-    launch(prefill_ragged_kernel<Tag, D, (D > 128)>);
+    launch(prefill_ragged_kernel<Tag, D, (D > 128 ? 3 : 1)>);
   const int st = dsp_launch_status();
   if (st != DSP_OK) return st;
   prefill_ragged_merge_kernel<Tag, D><<<dim3(W, kRows / ragged_merge_rows(D)), 256, 0, s>>>(
