@@ -126,9 +126,9 @@ __device__ __forceinline__ int64_t active_workers(int64_t C, int num_workers) {
 // each 2 KiB slot row at D 128: the pool's DRAM pages are then read HG slices at a time).
 // kMode: kPlain; kWide, the shapes that the generic kernel serves otherwise (D 256 and G > 8),
 // whose probabilities are fp32: they enter P.V as three 16-bit operands (pack8), and keys of a
-// block id outside the cache are masked, as they are there; kSlots, decode by per-token slot
+// block id outside the cache are skipped, as they are there; kSlots, decode by per-token slot
 // table (`bt` is the slot table), which the VALU kernel serves otherwise: fp32 probabilities as
-// in kWide, bad slots masked and each counted, as they are there.  A slot-table window holds the
+// in kWide, bad slots skipped and each counted, as they are there.  A slot-table window holds the
 // slots of 64 keys, one per lane, the next window's loaded while it is in use; a lane takes the
 // slots of its K and V rows from it by permute (24 sequences of 200-3000 keys, 28 heads over 4:
 // kernel and merge 42 -> 26 us a layer).
@@ -354,7 +354,12 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
       }
       const int cur[2] = {kMode == kWide ? min(lim, vlim[0]) : lim,
                           kMode == kWide ? min(lim, vlim[1]) : lim};
-      const uint32_t ok_cur = okm;
+      // kWide and kSlots (decode: every row sees the same keys): the chunk's keys that count, i.e.
+      // inside the piece with an id inside the cache (uniform).
+      uint32_t keys = ~0u;
+      if constexpr (kMode == kWide)
+        keys = low_bits(min(min(ke, vlim[0]) - t0, 16)) | low_bits(min(ke, vlim[1]) - t0 - 16) << 16;
+      if constexpr (kMode == kSlots) keys = okm & low_bits(ke - t0);
       if (prefetch) {
         advance(tn);
         chunk_blocks(tn);
@@ -362,7 +367,7 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
         load_k(tn);
       }
       if constexpr (kMode == kSlots) {
-        const uint32_t bad = ~ok_cur & (ke - t0 < 32 ? (1u << (ke - t0)) - 1u : ~0u);
+        const uint32_t bad = ~keys & low_bits(ke - t0);
         bad_slots += __popc(bad);
         if (bad) {  // uniform, rare
 #pragma unroll
@@ -413,6 +418,7 @@ __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128
         __builtin_amdgcn_s_waitcnt(dsp_waitcnt_vm<2 * NKK>());
       else
         __builtin_amdgcn_s_waitcnt(dsp_waitcnt_vm<0>());
+      if (kMode != kPlain && keys != ~0u) zero_rows<CPR, VINS>(slab_l, keys);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");

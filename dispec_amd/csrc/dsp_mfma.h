@@ -78,4 +78,21 @@ __device__ __forceinline__ void pack8(const float* p, dsp_u32x4 (&t)[kTerms]) {
                      pack2(h[k][6], h[k][7])};
 }
 
+// The low n bits, n clamped to 0..32.
+__device__ __forceinline__ uint32_t low_bits(int n) {
+  return n >= 32 ? ~0u : (n <= 0 ? 0u : (1u << n) - 1u);
+}
+
+// Zeros the rows of a V slab (rows of CPR 16-byte chunks, the layout that kLoads 1-KiB DMA loads
+// wrote) whose bit of `keep` is not set: keys that count for no row, whose slab rows hold
+// another key's values or the pool's slot 0 and would get infinities past a probability of 0.
+template <int CPR, int kLoads>
+__device__ __forceinline__ void zero_rows(char* slab, uint32_t keep) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i)
+    if (!((keep >> (i * (64 / CPR) + lane / CPR)) & 1u))
+      *reinterpret_cast<dsp_u32x4*>(slab + i * 1024 + 16 * lane) = dsp_u32x4{0u, 0u, 0u, 0u};
+}
+
 }  // namespace dsp_mfma

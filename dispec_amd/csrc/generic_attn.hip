@@ -275,7 +275,7 @@ __global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu
   if (dec) ctx = ctx < 0 ? 0 : (ctx > max_ctx ? max_ctx : ctx);
   // keys visible to row r: its query's position + 1 (none for bad lengths or no context)
   auto visible = [&](int r) { return !dec && bad_len ? 0 : ctx - qlen + r / G + 1; };
-  const int kend = visible(min(r0 + 15, rows - 1));
+  const int kend = visible(min(r0 + 15, rows - 1)), vis0 = visible(r0);
   const int kbeg = part * P, kfin = min(kbeg + P, kend);
   if (kbeg >= kend && part > 0) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -354,6 +354,35 @@ __global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu
     for (int j = 0; j < 4; ++j) {
       p[j] = dsp_exp2(p[j] - mu);
       l += p[j];
+    }
+    if (t0 + 16 > vis0) {  // a chunk that the tile's first row does not see whole (uniform)
+      bool odd = false;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int h = 0; h < VH; ++h)
+#pragma unroll
+          for (int e = 0; e < VE; ++e) odd |= !(fabsf(vf[j][h][e]) < INFINITY);
+      if (__ballot(odd)) {  // rare
+        // Infinities and NaN of V go to the rows that see their keys only (0 * inf is NaN):
+        // kHuge * kHuge overflows to inf, -kHuge * kHuge to -inf, and NaN takes both.
+        constexpr float kHuge = 0x1p127f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float seen = t0 + 4 * grp + j < vis ? kHuge : 0.f;
+#pragma unroll
+          for (int h = 0; h < VH; ++h)
+#pragma unroll
+            for (int e = 0; e < VE; ++e) {
+              float& v = vf[j][h][e];
+              f32x4& a = acc[h * VE + e];
+              const bool nan = v != v;
+              a = __builtin_amdgcn_mfma_f32_16x16x4f32(nan || v == INFINITY ? kHuge : 0.f, seen, a, 0, 0, 0);
+              a = __builtin_amdgcn_mfma_f32_16x16x4f32(nan || v == -INFINITY ? -kHuge : 0.f, seen, a, 0, 0, 0);
+              v = fabsf(v) < INFINITY ? v : 0.f;
+            }
+        }
+      }
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j)

@@ -41,7 +41,7 @@ using namespace dsp_mfma;
 // combine kernel merges.
 // kSplitP: the shapes that the generic kernel serves otherwise (D 256, and decode with G > 8),
 // whose probabilities are fp32: they enter P.V as three 16-bit operands (pack8); and keys of a
-// block id outside the cache are masked, as they are there.
+// block id outside the cache are skipped, as they are there.
 template <typename Tag, int D, bool kDecode, bool kSplitP>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 128 ? 2 : 3))) void paged_mq_kernel(
     const uint16_t* __restrict__ q, int64_t qst, int64_t qsh, const uint16_t* __restrict__ kc,
@@ -199,6 +199,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
       for (int kk = 0; kk < NKK; ++kk) sc[st] = mfma32<Tag>(kop[st][kk], qop[kk], sc[st]);
     }
     const uint32_t cur_bad[2] = {bad_keys[0], bad_keys[1]};
+    // kSplitP: the chunk's keys that count, i.e. inside the partition with an id inside the cache
+    // (uniform)
+    const uint32_t keys = kSplitP ? low_bits(kfin - t0) & ~(cur_bad[0] | cur_bad[1] << 16) : ~0u;
     if (prefetch) load_k(tn);
     // Scale and causal mask; lane holds keys t0 + 16*st + 4*grp + j of packed row n.
     float s[2][4];
@@ -243,6 +246,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
       __builtin_amdgcn_s_waitcnt(dsp_waitcnt_vm<2 * NKK>());
     else
       __builtin_amdgcn_s_waitcnt(dsp_waitcnt_vm<0>());
+    if (kSplitP && keys != ~0u) zero_rows<CPR, VINS>(slab, keys);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");

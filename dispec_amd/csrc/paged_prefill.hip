@@ -103,8 +103,8 @@ __device__ __forceinline__ void attend_chunks(
   constexpr int RPI = 1024 / ROWB;               // rows per 1-KiB DMA load
   constexpr int LPW = SLAB / 1024 / kWaves;      // DMA loads per wave per slab
   // kMaskBad: s_bad says which 16-key groups of each buffer's chunk have a block id outside the
-  // cache (their keys are masked, as on the 16-row tiles and on the generic kernel that serves
-  // unaligned 256-wide heads), and no slot past kfin is read.
+  // cache (their keys are skipped, as on the 16-row tiles of 256-wide heads and on the generic
+  // kernel: scores masked, V zeroed), and no slot past kfin is read.
   // kTerms: the 16-bit operands that hold a probability (pack8).  Three, i.e. fp32, at D 256 (as
   // on the generic kernel; one moves the error against 64 bits from 2.8e-3 to 3.3e-3), whose
   // 128 KiB of LDS leave one workgroup per CU, a wave's accumulators in AGPRs.
@@ -141,6 +141,7 @@ __device__ __forceinline__ void attend_chunks(
   auto load_blk = [&](int t0) {
     return bt[bt_row + (min(t0 + 16 * wave, kfin - 1) >> log2_bs)];
   };
+  bool bad_rows = false;  // kMaskBad: the rows this wave loaded last have a bad block id (uniform)
   auto issue = [&](int buf, int t0, int32_t blk_v) {
     const int32_t blk = __builtin_amdgcn_readfirstlane(blk_v);
     // kMaskBad: rows past kfin repeat the last key's (a stale row there may hold anything)
@@ -149,10 +150,11 @@ __device__ __forceinline__ void attend_chunks(
     if (blk < 0 || (int64_t(blk) + 1) * (bmask + 1) > num_slots) {
       slot0 = 0;
       any_bad |= t0 + 16 * wave < kfin;
-      if constexpr (kMaskBad) s_bad[buf][wave] = 1;
-    } else if constexpr (kMaskBad) {
-      s_bad[buf][wave] = 0;
+      bad_rows = true;
+    } else {
+      bad_rows = false;
     }
+    if constexpr (kMaskBad) s_bad[buf][wave] = bad_rows;
     const int64_t e = slot0 * kvs_slot + head_off;
     const char* kb = reinterpret_cast<const char*>(kc + e);
     const char* vb = reinterpret_cast<const char*>(vc + e);
@@ -191,6 +193,7 @@ __device__ __forceinline__ void attend_chunks(
     // the next DMA overwrites
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(dsp_waitcnt_vm<0>());
+    if (kMaskBad && bad_rows) zero_rows<CPR, LPW>(&lds[c & 1][1][wave * LPW * 1024], 0);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
     if (c + 1 < nch) {

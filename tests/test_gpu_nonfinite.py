@@ -6,7 +6,8 @@ import numpy as np
 import pytest
 import torch
 
-from tests._util import randn
+from oracle import ref_cpu
+from tests._util import f64, gen, randn
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -48,3 +49,104 @@ def test_nan_queries_give_nan_rows(hip, dtype, G, D, ctx, q_len):
     assert bool(torch.isnan(got[q_len, G]).all())
     got[q_len, G] = want[q_len, G]
     assert torch.equal(got, want)
+
+
+# ---- ids outside the cache: no key of theirs is read, not even the pool's slot 0
+P_ERR = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}
+
+
+def _close(got, ref, vmax, dtype, what):
+    """The output's rounding (half a unit in its last place, at most 2 P_ERR of it) and, where the
+    kernel rounds probabilities to 16 bits, P_ERR of each: of max |v| at most."""
+    err = np.abs(f64(got) - ref) - 2 * P_ERR[dtype] * np.abs(ref)
+    assert np.isfinite(err).all() and err.max() <= P_ERR[dtype] * vmax, \
+        f"{what}: {err.max():.3g} over {P_ERR[dtype] * vmax:.3g}"
+
+
+def _ragged(q, kc, vc, bt, cu, lens, G, max_q, max_ctx, err=None, bs=16):
+    from dispec_amd import _lib
+    L, out = _lib.lib(), torch.empty_like(q)
+    (S, KVH, D), B = kc.shape, lens.numel()
+    need = L.dsp_paged_mq_ragged_workspace_bytes(B, G * KVH, KVH, D, max_q, max_ctx)
+    ws = torch.full((need // 4,), float("nan"), device=DEV)
+    _lib.check(L.dsp_paged_mq_attention_ragged(
+        q.data_ptr(), q.stride(0), q.stride(1), kc.data_ptr(), vc.data_ptr(), S, kc.stride(0),
+        kc.stride(1), bt.data_ptr(), bt.stride(0), bs, cu.data_ptr(), lens.data_ptr(), B, G * KVH,
+        KVH, D, D ** -0.5, max_q, max_ctx, ws.data_ptr(), need, out.data_ptr(), out.stride(0),
+        out.stride(1), _lib.dtype_code(q.dtype), _lib.ptr(err), _lib.stream_of(q)), "ragged")
+    return out
+
+
+def _spoiled(ctx, KVH, D, dtype, bad, seed=11):
+    """A pool whose block 0 is infinite and NaN, tables that never name it, the slots of every
+    sequence's keys in good blocks, and the table with ids outside the pool at `bad` = [(sequence,
+    block)]."""
+    bs = 16
+    need = [-(-n // bs) for n in ctx]
+    NB = sum(need) + 1
+    perm = (1 + torch.randperm(NB - 1, generator=gen(seed))).int()
+    kc, vc = (randn((NB * bs, KVH, D), seed + i, dtype).to(DEV) for i in (1, 2))
+    kc[:bs], vc[:8], vc[8:bs] = float("nan"), float("inf"), float("nan")
+    bt = torch.zeros((len(ctx), max(need)), dtype=torch.int32)
+    at = 0
+    for b, n in enumerate(need):
+        bt[b, :n] = perm[at:at + n]
+        at += n
+    keys = [(bt[b].long()[torch.arange(n) // bs] * bs + torch.arange(n) % bs).numpy()
+            for b, n in enumerate(ctx)]
+    for i, (b, j) in enumerate(bad):
+        bt[b, j] = (NB, -1, 2 ** 30)[i % 3]
+        keys[b][j * bs:(j + 1) * bs] = -1
+    return kc, vc, bt.to(DEV), [k[k >= 0] for k in keys]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("G,KVH,D", [(12, 2, 128), (9, 1, 64), (12, 1, 32), (4, 2, 256), (17, 1, 256)])
+@pytest.mark.parametrize("ctx,P", [([300, 77, 33], 0), ([1300, 2000, 40], 0), ([1300, 700, 40], 256)])
+def test_decode_skips_bad_blocks(hip, dtype, G, KVH, D, ctx, P):
+    from dispec_amd.engine.hip_attn import paged_decode_attention_blocks
+    bad = [(0, 0), (0, 5), (0, 18), (1, 1), (1, 4), (2, 2)]
+    kc, vc, bt, keys = _spoiled(ctx, KVH, D, dtype, bad)
+    q = randn((3, G * KVH, D), 5, dtype).to(DEV)
+    out = paged_decode_attention_blocks(q, kc, vc, bt, _i32(ctx), G, max_ctx=max(ctx),
+                                        partition_tokens=P)
+    ref = ref_cpu.decode_attention(f64(q), f64(kc), f64(vc), keys, [len(k) for k in keys], G)
+    _close(out, ref, 6, dtype, f"G={G} D={D} {ctx} P={P}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("G,KVH,D", [(7, 2, 128), (7, 2, 64), (1, 4, 32)])
+def test_slot_decode_skips_bad_slots(hip, dtype, G, KVH, D):
+    from dispec_amd.engine.hip_attn import batched_paged_decode_attention
+    ctx = [1500, 40, 33, 16] + [900] * 12
+    kc, vc, bt, keys = _spoiled(ctx, KVH, D, dtype, [])
+    st = torch.zeros((16, max(ctx)), dtype=torch.int32)
+    for b, k in enumerate(keys):
+        st[b, :len(k)] = torch.from_numpy(k).int()
+        for i, j in enumerate(sorted({0, 31, 32, len(k) // 2, len(k) - 1} & set(range(len(k))))):
+            st[b, j] = (kc.shape[0], -1, 2 ** 31 - 1)[i % 3]
+        keys[b] = k[(st[b, :len(k)] >= 0).numpy() & (st[b, :len(k)] < kc.shape[0]).numpy()]
+    q = randn((16, G * KVH, D), 5, dtype).to(DEV)
+    out = batched_paged_decode_attention(q, kc, vc, st.to(DEV), _i32(ctx), G)
+    ref = ref_cpu.decode_attention(f64(q), f64(kc), f64(vc), keys, [len(k) for k in keys], G)
+    _close(out, ref, 6, dtype, f"G={G} D={D}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("form,D", [("grid", 256), ("ragged", 64), ("ragged", 128), ("ragged", 256)])
+@pytest.mark.parametrize("q_lens", [[3, 1, 2], [70, 1, 9]])
+def test_multi_query_skips_bad_blocks(hip, dtype, form, D, q_lens):
+    """16-row and 128-row tiles (G 3), the grid and the equal shares; no bad block holds a query."""
+    from dispec_amd.engine.hip_attn import paged_mq_attention
+    ctx, G, KVH = [1000, 200, 63], 3, 2
+    kc, vc, bt, keys = _spoiled(ctx, KVH, D, dtype, [(0, 0), (0, 5), (0, 30), (1, 2), (2, 1)])
+    q = randn((sum(q_lens), G * KVH, D), 5, dtype).to(DEV)
+    cu = _i32([0] + list(np.cumsum(q_lens)))
+    if form == "ragged":
+        err = _i32([0])
+        out = _ragged(q, kc, vc, bt, cu, _i32(ctx), G, max(q_lens), 1008, err)
+        assert int(err.item()) > 0
+    else:
+        out = paged_mq_attention(q, kc, vc, bt, cu, _i32(ctx), G, max_q_len=max(q_lens))
+    ref = ref_cpu.mq_attention(f64(q), f64(kc), f64(vc), keys, q_lens, G)
+    _close(out, ref, 6, dtype, f"{form} D={D} {q_lens}")
