@@ -35,47 +35,64 @@ __device__ __forceinline__ uint16_t narrow(float f) {
     return dsp_f32_to_f16(f);
 }
 
-template <typename Tag>
-__device__ __forceinline__ float widen(uint16_t b) {
-  if constexpr (std::is_same<Tag, Bf16Tag>::value)
-    return dsp_bf16lo(b);
-  else
-    return dsp_f16lo(b);
-}
-
 __device__ __forceinline__ uint32_t pack2(uint16_t lo, uint16_t hi) {
   return uint32_t(lo) | (uint32_t(hi) << 16);
 }
 
-// Eight fp32 probabilities as kTerms 16-bit MFMA operands: the first is their rounding, each
-// further one the rounding of what the ones before it left over.  Three terms hold all 24 bits
-// of an fp32 value: P.V over them is P.V of fp32 probabilities, for the shapes whose
-// probabilities are fp32 (two hold 16 bits in bf16, 22 in fp16; the third costs the 256-wide
-// prefill tile 80 -> 91 us at 4 x 200 tokens over 1999, 24 slot-table decodes 20.7 -> 21.3).  bf16 has fp32's exponents.
-// fp16 ends at 2^-24, so three terms expect p * p_scale there, p <= 1: at 2^15 the last bit
-// kept is 2^-39, whatever p's size; the row sum takes the same factor, and the division by it
-// cancels the two.
+// Eight fp32 probabilities as kTerms 16-bit MFMA operands.  One: their rounding.  More: each
+// operand takes the leading bits of what the ones before it left over, the last one its
+// rounding.  Three hold all 24 bits of an fp32 value: P.V over them is P.V of fp32
+// probabilities, for the shapes whose probabilities are fp32 (two hold 16 bits in bf16, 22 in
+// fp16; the third costs the 256-wide prefill tile 80 -> 91 us at 4 x 200 tokens over 1999, 24
+// slot-table decodes 20.7 -> 21.3).
+// The leading bits are cut, not rounded, and an operand of a p above 0 is kept above 0 (by the
+// least number, 2^-100 or the last bit kept), so that an infinity in V meets positive factors
+// only: a 0 or a negative one would make NaN of it.
+// bf16 has fp32's exponents.  fp16 ends at 2^-24, so more than one term expects p * p_scale
+// there, at most 2^15: with three p <= 1 and the last bit kept is 2^-39, whatever p's size; with
+// two p <= 2^8 (a lagging maximum) and 2^-31.  The row sum takes the same factor, and the
+// division by it cancels the two.
 template <typename Tag, int kTerms>
 constexpr float p_scale() {
-  return kTerms == 3 && std::is_same<Tag, F16Tag>::value ? 32768.f : 1.f;
+  return kTerms == 1 || std::is_same<Tag, Bf16Tag>::value ? 1.f : kTerms == 2 ? 128.f : 32768.f;
 }
 
 template <typename Tag, int kTerms>
 __device__ __forceinline__ void pack8(const float* p, dsp_u32x4 (&t)[kTerms]) {
-  uint16_t h[kTerms][8];
+  if constexpr (kTerms == 1) {
+    uint16_t h[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    float rest = p[i];
+    for (int i = 0; i < 8; ++i) h[i] = narrow<Tag>(p[i]);
+    t[0] = dsp_u32x4{pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7])};
+    return;
+  }
+  constexpr bool kBf16 = std::is_same<Tag, Bf16Tag>::value;
+  constexpr float kLeast = kBf16 ? 0x1p-100f : 0x1p-24f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float rest[2] = {p[2 * i], p[2 * i + 1]};
+    const float least[2] = {fminf(rest[0], kLeast), fminf(rest[1], kLeast)};
 #pragma unroll
     for (int k = 0; k < kTerms; ++k) {
-      h[k][i] = narrow<Tag>(rest);
-      rest -= widen<Tag>(h[k][i]);
+      if (k + 1 == kTerms) {
+        t[k][i] = pack2(narrow<Tag>(rest[0]), narrow<Tag>(rest[1]));
+        break;
+      }
+      float cut[2];
+      if constexpr (kBf16) {
+        const uint32_t a = __float_as_uint(rest[0]), b = __float_as_uint(rest[1]);
+        t[k][i] = (a >> 16) | (b & 0xffff0000u);
+        cut[0] = __uint_as_float(a & 0xffff0000u);
+        cut[1] = __uint_as_float(b & 0xffff0000u);
+      } else {
+        t[k][i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(rest[0], rest[1]));
+        cut[0] = dsp_f16lo(t[k][i]);
+        cut[1] = dsp_f16hi(t[k][i]);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) rest[j] = fmaxf(rest[j] - cut[j], least[j]);
     }
   }
-#pragma unroll
-  for (int k = 0; k < kTerms; ++k)
-    t[k] = dsp_u32x4{pack2(h[k][0], h[k][1]), pack2(h[k][2], h[k][3]), pack2(h[k][4], h[k][5]),
-                     pack2(h[k][6], h[k][7])};
 }
 
 // The low n bits, n clamped to 0..32.

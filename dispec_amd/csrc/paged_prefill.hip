@@ -250,7 +250,7 @@ __device__ __forceinline__ void attend_chunks(
     // Lazy rescale: the running max m only moves when some row's chunk max exceeds it by
     // more than 8 (so p <= 2^8); the result is exact either way, since l and acc share m.
     // (Where pack8 takes p <= 1 at most, m is the exact maximum.)
-    constexpr float kLag = p_scale<Tag, kTerms>() == 1.f ? 8.f : 0.f;
+    constexpr float kLag = p_scale<Tag, kTerms>() > 128.f ? 0.f : 8.f;
     if (__builtin_amdgcn_ballot_w64(mx > m + kLag) != 0) {
       const float m_new = fmaxf(m, mx);
       const float alpha = m_new == -INFINITY ? 1.f : dsp_exp2(m - m_new);

@@ -150,3 +150,50 @@ def test_multi_query_skips_bad_blocks(hip, dtype, form, D, q_lens):
         out = paged_mq_attention(q, kc, vc, bt, cu, _i32(ctx), G, max_q_len=max(q_lens))
     ref = ref_cpu.mq_attention(f64(q), f64(kc), f64(vc), keys, q_lens, G)
     _close(out, ref, 6, dtype, f"{form} D={D} {q_lens}")
+
+
+
+# ---- infinities and NaN in V of keys that every row sees
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("form,G,KVH,D,q_lens,ctx", [
+    ("slots", 7, 2, 64, [1] * 16, [1100] * 15 + [40]), ("slots", 3, 2, 128, [1] * 16, [1100] * 16),
+    ("decode", 12, 2, 128, [1, 1], [300, 77]), ("decode", 12, 2, 128, [1, 1], [2000, 77]),
+    ("decode", 4, 2, 256, [1, 1], [300, 77]), ("decode", 4, 2, 256, [1, 1], [2000, 77]),
+    ("multi", 3, 2, 256, [5, 2], [900, 77]), ("multi", 3, 2, 256, [50, 2], [900, 77]),
+    ("ragged", 3, 2, 64, [5, 2], [900, 77]), ("ragged", 3, 2, 128, [5, 2], [900, 77]),
+    ("ragged", 3, 2, 256, [50, 2], [900, 77])])
+def test_infinite_values_stay_infinite(hip, dtype, form, G, KVH, D, q_lens, ctx):
+    """inf times a row's probability is inf, whatever the split of the probability into operands:
+    values at a sequence's keys 0, 20 and, for decode, the last."""
+    from dispec_amd.engine.hip_attn import (batched_paged_decode_attention,
+                                            paged_decode_attention_blocks, paged_mq_attention)
+    kc, vc, bt, keys = _spoiled(ctx, KVH, D, dtype, [])
+    clean = vc.clone()
+    for k, n in zip(keys, ctx):
+        at = torch.from_numpy(k)
+        vc[at[0], 0, 3], vc[at[20], 0, D - 1], vc[at[20], 1, 5] = float("inf"), -float("inf"), float("nan")
+        clean[at[0], 0, 3], clean[at[20], 0, D - 1], clean[at[20], 1, 5] = 0, 0, 0
+        if max(q_lens) == 1:
+            vc[at[-1], 1, 7], clean[at[-1], 1, 7] = float("inf"), 0
+    q = randn((sum(q_lens), G * KVH, D), 5, dtype).to(DEV)
+    lens = _i32(ctx)
+    if form == "slots":
+        st = torch.zeros((len(ctx), max(ctx)), dtype=torch.int32)
+        for b, k in enumerate(keys):
+            st[b, :len(k)] = torch.from_numpy(k).int()
+        out = batched_paged_decode_attention(q, kc, vc, st.to(DEV), lens, G)
+    elif form == "decode":
+        out = paged_decode_attention_blocks(q, kc, vc, bt, lens, G, max_ctx=max(ctx))
+    else:
+        cu = _i32([0] + list(np.cumsum(q_lens)))
+        if form == "ragged":
+            out = _ragged(q, kc, vc, bt, cu, lens, G, max(q_lens), bt.shape[1] * 16)
+        else:
+            out = paged_mq_attention(q, kc, vc, bt, cu, lens, G, max_q_len=max(q_lens))
+    want = ref_cpu.mq_attention(f64(q), f64(kc), f64(clean), keys, q_lens, G)
+    want[:, :G, 3], want[:, :G, D - 1], want[:, G:, 5] = np.inf, -np.inf, np.nan
+    if max(q_lens) == 1:
+        want[:, G:, 7] = np.inf
+    got, odd = f64(out), ~np.isfinite(want)
+    assert np.array_equal(got[odd], want[odd], equal_nan=True)
+    assert np.abs(got[~odd] - want[~odd]).max() <= 2 * P_ERR[dtype] * 6
