@@ -100,6 +100,13 @@ __device__ __forceinline__ uint32_t low_bits(int n) {
   return n >= 32 ? ~0u : (n <= 0 ? 0u : (1u << n) - 1u);
 }
 
+// Orders a wave's LDS accesses before and after it across its lanes.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Zeros the rows of a V slab (rows of CPR 16-byte chunks, the layout that kLoads 1-KiB DMA loads
 // wrote) whose bit of `keep` is not set: keys that count for no row, whose slab rows hold
 // another key's values or the pool's slot 0 and would get infinities past a probability of 0.
@@ -110,6 +117,63 @@ __device__ __forceinline__ void zero_rows(char* slab, uint32_t keep) {
   for (int i = 0; i < kLoads; ++i)
     if (!((keep >> (i * (64 / CPR) + lane / CPR)) & 1u))
       *reinterpret_cast<dsp_u32x4*>(slab + i * 1024 + 16 * lane) = dsp_u32x4{0u, 0u, 0u, 0u};
+}
+
+// ---- infinities and NaN of V on tiles whose rows see different keys.  A key that a row does not
+// see has probability 0, but 0 * inf is NaN.  So in chunks that some row does not see whole,
+// such values are found (any_nonfinite), added to the rows that see them (odd_operand against
+// kHuge for every key seen) and cleared in LDS (clear_nonfinite) before P.V.
+template <typename Tag>
+constexpr uint32_t exp_bits() {  // an infinity's bits; above it, NaN
+  return std::is_same<Tag, Bf16Tag>::value ? 0x7f80u : 0x7c00u;
+}
+constexpr uint32_t kHuge = 0x7f00u;  // 2^127 in bf16: its square overflows the accumulator
+
+// Whether any lane's part of the kLoads KiB at `slab` holds an infinity or NaN (wave-uniform).
+template <typename Tag, int kLoads>
+__device__ __forceinline__ bool any_nonfinite(const char* slab) {
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  u16x2 top = {0, 0};
+#pragma unroll 4
+  for (int i = 0; i < kLoads; ++i) {
+    const dsp_u32x4 v =
+        *reinterpret_cast<const dsp_u32x4*>(slab + i * 1024 + 16 * (threadIdx.x & 63));
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, v[j] & 0x7fff7fffu));
+  }
+  return __ballot(top[0] >= exp_bits<Tag>() || top[1] >= exp_bits<Tag>()) != 0;
+}
+
+template <typename Tag, int kLoads>
+__device__ __forceinline__ void clear_nonfinite(char* slab) {
+#pragma unroll 4
+  for (int i = 0; i < kLoads; ++i) {
+    dsp_u32x4* p = reinterpret_cast<dsp_u32x4*>(slab + i * 1024 + 16 * (threadIdx.x & 63));
+    dsp_u32x4 v = *p;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if ((v[j] & 0x7fffu) >= exp_bits<Tag>()) v[j] &= 0xffff0000u;
+      if ((v[j] & 0x7fff0000u) >= exp_bits<Tag>() << 16) v[j] &= 0xffffu;
+    }
+    *p = v;
+  }
+}
+
+// A bf16 operand (whatever the cache's type: the lane layouts are the same) of kHuge where v is
+// +inf or NaN (minus false), of -kHuge where it is -inf or NaN (minus true), 0 elsewhere.  The
+// MFMA of both with kHuge for the keys a row sees adds inf, -inf, or inf - inf = NaN to it (the
+// bf16 MFMA rounds a product to infinity before it adds it to an infinite sum).
+template <typename Tag>
+__device__ __forceinline__ dsp_u32x4 odd_operand(dsp_u32x4 v, bool minus) {
+  auto code = [minus](uint32_t h) {
+    const bool odd = minus ? (h & 0x7fffu) > exp_bits<Tag>() || h == (0x8000u | exp_bits<Tag>())
+                           : (h & 0x7fffu) > exp_bits<Tag>() || h == exp_bits<Tag>();
+    return odd ? kHuge | (minus ? 0x8000u : 0u) : 0u;
+  };
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = code(v[j] & 0xffffu) | code(v[j] >> 16) << 16;
+  return v;
 }
 
 }  // namespace dsp_mfma

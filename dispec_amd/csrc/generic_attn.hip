@@ -365,7 +365,9 @@ __global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu
           for (int e = 0; e < VE; ++e) odd |= !(fabsf(vf[j][h][e]) < INFINITY);
       if (__ballot(odd)) {  // rare
         // Infinities and NaN of V go to the rows that see their keys only (0 * inf is NaN):
-        // kHuge * kHuge overflows to inf, -kHuge * kHuge to -inf, and NaN takes both.
+        // kHuge * kHuge overflows to inf, -kHuge * kHuge to -inf, and NaN takes both (each
+        // from a sum of its own: products are not rounded before they are added, and inf - 2^254
+        // is inf).
         constexpr float kHuge = 0x1p127f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -377,8 +379,11 @@ __global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu
               float& v = vf[j][h][e];
               f32x4& a = acc[h * VE + e];
               const bool nan = v != v;
-              a = __builtin_amdgcn_mfma_f32_16x16x4f32(nan || v == INFINITY ? kHuge : 0.f, seen, a, 0, 0, 0);
-              a = __builtin_amdgcn_mfma_f32_16x16x4f32(nan || v == -INFINITY ? -kHuge : 0.f, seen, a, 0, 0, 0);
+              const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+              a += __builtin_amdgcn_mfma_f32_16x16x4f32(nan || v == INFINITY ? kHuge : 0.f, seen, none,
+                                                        0, 0, 0);
+              a += __builtin_amdgcn_mfma_f32_16x16x4f32(nan || v == -INFINITY ? -kHuge : 0.f, seen,
+                                                        none, 0, 0, 0);
               v = fabsf(v) < INFINITY ? v : 0.f;
             }
         }

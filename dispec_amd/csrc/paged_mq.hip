@@ -250,6 +250,37 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if constexpr (kSplitP && !kDecode) {
+      // a chunk that the tile's first row does not see whole (uniform): infinities and NaN in
+      // it go to the rows that see them only (V^T operands as below)
+      if (t0 + 31 > ctx - qlen + r0 / G && any_nonfinite<Tag, VINS>(slab)) {
+        dsp_u32x4 seen;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = t0 + 16 * (i >> 1) + 4 * grp + 2 * (i & 1);
+          seen[i] = (key <= pos_q ? kHuge : 0u) | (key < pos_q ? kHuge << 16 : 0u);
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          __builtin_amdgcn_sched_barrier(0);  // one tile's operands at a time: registers
+          const int d = 16 * nt + n;
+          uint16_t v[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const int kl = u < 4 ? 4 * grp + u : 16 + 4 * grp + (u - 4);
+            v[u] = *reinterpret_cast<const uint16_t*>(slab + kl * ROWB + 16 * swz(kl, d >> 3) +
+                                                      2 * (d & 7));
+          }
+          const dsp_u32x4 vop = dsp_u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]),
+                                          pack2(v[6], v[7])};
+          acc[nt] = mfma32<Bf16Tag>(odd_operand<Tag>(vop, false), seen, acc[nt]);
+          acc[nt] = mfma32<Bf16Tag>(odd_operand<Tag>(vop, true), seen, acc[nt]);
+        }
+        wave_lds_fence();
+        clear_nonfinite<Tag, VINS>(slab);
+        wave_lds_fence();
+      }
+    }
     // V^T operand: lane needs dim 16*nt + n of keys {4*grp+u} (u<4) and {16+4*grp+u-4}.
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {

@@ -82,17 +82,39 @@ __device__ __forceinline__ void dma16(const void* sbase, uint32_t voff, uint32_t
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4i16 lds_v4i16_t;
 
+// The V^T operand of 16-key step ps of a chunk in LDS: dim 32*dt + col, K index 8*hl + i <-> key
+// 16*ps + 8*(i/4) + 4*hl + i%4 (the P^T order; col and hl as in attend_chunks).  In
+// ds_read_b64_tr_b16, lane g + 4a + e of each 16-lane group g receives element e of the
+// 4-element segments addressed by lanes g + a + 4j (j = 0..3); so lane s addresses key 16*ps +
+// 8*inst + 4*hl + (s%16)/4, dims 32*dt + 16*((s/16)%2) + 4*(s%4) .. +3, for inst = 0, 1.
+template <int D>
+__device__ __forceinline__ dsp_u32x4 load_vt(const char* vs_lds, int ps, int dt) {
+  const int lane = threadIdx.x & 63, hl = lane >> 5;
+  v4i16 vh[2];
+#pragma unroll
+  for (int inst = 0; inst < 2; ++inst) {
+    const int kr = 16 * ps + 8 * inst + 4 * hl + ((lane & 15) >> 2);
+    const int dim0 = 32 * dt + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    const int swz = D >= 128 ? 4 * (kr & 3) : 4 * ((kr >> 1) & 1);
+    vh[inst] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(
+        vs_lds + kr * 2 * D + 16 * ((dim0 >> 3) ^ swz) + 2 * (dim0 & 7)));
+  }
+  return __builtin_bit_cast(dsp_u32x4, vh);
+}
+
 // One workgroup's keys [kbeg, kfin) of one (sequence, KV head), in 64-key chunks, for the rows
 // whose Q^T operands are in qop: the running (max, sum, accumulator) of each row is updated.
-// lim: the last key this lane's row sees; lim_min: the least of them in the wave (uniform).
+// lim: the last key this lane's row sees; lim_min: the least of them in the wave, tile_lim in the
+// workgroup (uniform).
 // blk_first / blk_second: this wave's block ids of the first two chunks, loaded early and
 // unclamped.  Every wave of the workgroup calls it (it has barriers).
 template <typename Tag, int D, bool kNonTemporal, bool kMaskBad, int kTerms, typename Lds>
 __device__ __forceinline__ void attend_chunks(
-    Lds& lds, int32_t (&s_bad)[2][kWaves], const uint16_t* __restrict__ kc,
+    Lds& lds, int32_t (&s_bad)[2][kWaves], int32_t (&s_odd)[2][kWaves],
+    const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t head_off,
     const int32_t* __restrict__ bt, int64_t bt_row, int32_t log2_bs, int kbeg, int kfin, int lim,
-    int lim_min, bool wave_has_rows, const dsp_u32x4 (&qop)[D / 16], float scale_log2,
+    int lim_min, int tile_lim, bool wave_has_rows, const dsp_u32x4 (&qop)[D / 16], float scale_log2,
     int32_t blk_first, int32_t blk_second, float& m, float& lpart, f32x16 (&acc)[D / 32],
     bool& any_bad) {
   constexpr int NKS = D / 16;        // 16-dim steps of the score MFMA
@@ -104,7 +126,9 @@ __device__ __forceinline__ void attend_chunks(
   constexpr int LPW = SLAB / 1024 / kWaves;      // DMA loads per wave per slab
   // kMaskBad: s_bad says which 16-key groups of each buffer's chunk have a block id outside the
   // cache (their keys are skipped, as on the 16-row tiles of 256-wide heads and on the generic
-  // kernel: scores masked, V zeroed), and no slot past kfin is read.
+  // kernel: scores masked, V zeroed), no slot past kfin is read, and infinities and NaN of V reach
+  // the rows that see their keys only: s_odd says which groups of a chunk that some row of the tile
+  // does not see whole hold any.
   // kTerms: the 16-bit operands that hold a probability (pack8).  Three, i.e. fp32, at D 256 (as
   // on the generic kernel; one moves the error against 64 bits from 2.8e-3 to 3.3e-3), whose
   // 128 KiB of LDS leave one workgroup per CU, a wave's accumulators in AGPRs.
@@ -193,16 +217,34 @@ __device__ __forceinline__ void attend_chunks(
     // the next DMA overwrites
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(dsp_waitcnt_vm<0>());
-    if (kMaskBad && bad_rows) zero_rows<CPR, LPW>(&lds[c & 1][1][wave * LPW * 1024], 0);
+    char* const my_v = &lds[c & 1][1][wave * LPW * 1024];  // the V rows this wave loaded
+    const bool edge = kMaskBad && t0 + kChunk - 1 > tile_lim;
+    if (kMaskBad && bad_rows) zero_rows<CPR, LPW>(my_v, 0);
+    if (edge) {
+      __builtin_amdgcn_sched_barrier(0);
+      s_odd[c & 1][wave] = any_nonfinite<Tag, LPW>(my_v);
+    }
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
+    bool odd = false;  // rare: see below (uniform in the workgroup)
+    if (edge)
+      odd = __builtin_amdgcn_readfirstlane(s_odd[c & 1][0] | s_odd[c & 1][1] | s_odd[c & 1][2] |
+                                           s_odd[c & 1][3]) != 0;
+    auto clear_odd = [&] {
+      __syncthreads();  // every wave has taken the chunk's infinities and NaN
+      clear_nonfinite<Tag, LPW>(my_v);
+      __syncthreads();
+    };
     if (c + 1 < nch) {
       issue((c + 1) & 1, t0 + kChunk, blk);
       if (c + 2 < nch) blk = load_blk(t0 + 2 * kChunk);
     }
     // A wave whose 32 rows all lie past the tile's rows (a short query block: a verify
     // tile of 10 rows leaves three of four waves empty) only loads its share of each chunk.
-    if (!wave_has_rows) continue;
+    if (!wave_has_rows) {
+      if (odd) clear_odd();
+      continue;
+    }
     const char* ks_lds = &lds[c & 1][0][0];
     const char* vs_lds = &lds[c & 1][1][0];
 
@@ -277,27 +319,51 @@ __device__ __forceinline__ void attend_chunks(
       if constexpr (kTerms < 3) pack8<Tag, kTerms>(p8[ps], pop[ps]);
     }
 
-    // ---- O^T += V^T . P^T.  Per 16-key step ps the V^T operand is dim 32*dt + col, K index
-    // 8*hl + i <-> key 16*ps + 8*(i/4) + 4*hl + i%4 (the P^T order).  In ds_read_b64_tr_b16,
-    // lane g + 4a + e of each 16-lane group g receives element e of the 4-element segments
-    // addressed by lanes g + a + 4j (j = 0..3); so lane s addresses key 16*ps + 8*inst +
-    // 4*hl + (s%16)/4, dims 32*dt + 16*((s/16)%2) + 4*(s%4) .. +3, for inst = 0, 1.
+    // (rare) infinities and NaN of V to the rows that see them
+    if (kMaskBad && odd) {
+#pragma unroll 1
+      for (int ps = 0; ps < 4; ++ps) {
+        dsp_u32x4 seen;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = t0 + 16 * ps + 8 * (i >> 1) + 4 * hl + 2 * (i & 1);
+          seen[i] = (key <= lim ? kHuge : 0u) | (key < lim ? kHuge << 16 : 0u);
+        }
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) {
+          __builtin_amdgcn_sched_barrier(0);  // one tile's operands at a time: registers
+          const dsp_u32x4 v = load_vt<D>(vs_lds, ps, dt);
+          acc[dt] = mfma32x32<Bf16Tag>(odd_operand<Tag>(v, false), seen, acc[dt]);
+          acc[dt] = mfma32x32<Bf16Tag>(odd_operand<Tag>(v, true), seen, acc[dt]);
+        }
+      }
+      clear_odd();
+    }
+    // ---- O^T += V^T . P^T
 #pragma unroll
     for (int ps = 0; ps < 4; ++ps) {
       if constexpr (kTerms == 3) pack8<Tag, kTerms>(p8[ps], pop[ps]);
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt) {
-        v4i16 vh[2];
+        if constexpr (D > 128) {
+          const dsp_u32x4 vop = load_vt<D>(vs_lds, ps, dt);
 #pragma unroll
-        for (int inst = 0; inst < 2; ++inst) {
-          const int kr = 16 * ps + 8 * inst + 4 * hl + ((lane & 15) >> 2);
-          const int dim0 = 32 * dt + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-          vh[inst] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(
-              vs_lds + kr * ROWB + 16 * ((dim0 >> 3) ^ vswz(kr)) + 2 * (dim0 & 7)));
+          for (int k = 0; k < kTerms; ++k) acc[dt] = mfma32x32<Tag>(vop, pop[ps][k], acc[dt]);
+        } else {
+          // load_vt written out: as a call the compiler keeps fewer addresses in registers, which
+          // costs D 128 5 % (4 x 512 tokens over 4096: 154 -> 161 us) and saves D 256 6 %
+          v4i16 vh[2];
+#pragma unroll
+          for (int inst = 0; inst < 2; ++inst) {
+            const int kr = 16 * ps + 8 * inst + 4 * hl + ((lane & 15) >> 2);
+            const int dim0 = 32 * dt + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+            vh[inst] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(
+                vs_lds + kr * ROWB + 16 * ((dim0 >> 3) ^ vswz(kr)) + 2 * (dim0 & 7)));
+          }
+#pragma unroll
+          for (int k = 0; k < kTerms; ++k)
+            acc[dt] = mfma32x32<Tag>(__builtin_bit_cast(dsp_u32x4, vh), pop[ps][k], acc[dt]);
         }
-#pragma unroll
-        for (int k = 0; k < kTerms; ++k)
-          acc[dt] = mfma32x32<Tag>(__builtin_bit_cast(dsp_u32x4, vh), pop[ps][k], acc[dt]);
       }
     }
   }
@@ -328,7 +394,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
   constexpr int SLAB = kChunk * 2 * D;  // one K (or V) chunk
   __shared__ __attribute__((aligned(1024))) char lds[2][2][SLAB];  // [buffer][K | V]
   __shared__ int32_t s_cu[kShared ? kMaxSharedSeqs + 1 : 1];         // cu_q, prefix pass
-  __shared__ int32_t s_bad[2][kWaves];
+  __shared__ int32_t s_bad[2][kWaves], s_odd[2][kWaves];
 
   // XCD-aware order: the dispatcher hands workgroup `lin` to XCD lin % 8.  Each XCD gets a
   // contiguous range of logical ids, so the tiles of one (sequence, KV head) -- which read
@@ -427,6 +493,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
   // `rows` have q = 0: finite scores, never stored.
   const int lim = min(ctx - qlen + qi, kfin - 1);
   const int lim_min = min(ctx - qlen + (r0 + 32 * wave) / G, kfin - 1);
+  const int tile_lim = min(ctx - qlen + r0 / G, kfin - 1);
   const int64_t bt_row = int64_t(b) * bt_stride;
   const int64_t head_off = int64_t(kvh) * kvs_head;
 
@@ -445,8 +512,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
   for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[dt][j] = 0.f;
-  attend_chunks<Tag, D, kShared, (D > 128), (D > 128 ? 3 : 1)>(lds, s_bad, kc, vc, num_slots, kvs_slot, head_off, bt, bt_row,
-                                 log2_bs, kbeg, kfin, lim, lim_min, wave_has_rows, qop, scale_log2,
+  attend_chunks<Tag, D, kShared, (D > 128), (D > 128 ? 3 : 1)>(lds, s_bad, s_odd, kc, vc, num_slots, kvs_slot, head_off, bt, bt_row,
+                                 log2_bs, kbeg, kfin, lim, lim_min, tile_lim, wave_has_rows, qop, scale_log2,
                                  blk_first, blk_second, m, lpart, acc, any_bad);
 
   if (err_count && any_bad && lane == 0) atomicAdd(err_count, 1);  // once per wave
@@ -613,7 +680,7 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
 // up to 2^8, and one 16-bit probability would err 4 % more (3.1e-3 -> 3.2e-3 against 64 bits, 32
 // verifies of 28 heads over 4).
 template <typename Tag, int D, int kTerms>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2))) void prefill_ragged_kernel(
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : D > 64 ? 2 : 3))) void prefill_ragged_kernel(
     const uint16_t* __restrict__ q, int64_t qst, int64_t qsh, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int64_t num_slots, int64_t kvs_slot, int64_t kvs_head,
     const int32_t* __restrict__ bt, int64_t bt_stride, int32_t log2_bs,
@@ -623,7 +690,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
     int64_t ost, int64_t osh, int32_t* __restrict__ err_count) {
   constexpr int NKS = D / 16, NDT = D / 32, SLAB = kChunk * 2 * D;
   __shared__ __attribute__((aligned(1024))) char lds[2][2][SLAB];
-  __shared__ int32_t s_bad[2][kWaves];
+  __shared__ int32_t s_bad[2][kWaves], s_odd[2][kWaves];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hl = lane >> 5, col = lane & 31;
@@ -747,6 +814,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
     const int h = kvh * G + (row_ok ? r % G : 0);
     const int lim = min(sq.ctx - sq.qlen + qi, kfin - 1);
     const int lim_min = min(sq.ctx - sq.qlen + (r0 + 32 * wave) / G, kfin - 1);
+    const int tile_lim = min(sq.ctx - sq.qlen + r0 / G, kfin - 1);
     dsp_u32x4 qop[NKS];
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks)
@@ -760,9 +828,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
 #pragma unroll
       for (int j = 0; j < 16; ++j) acc[dt][j] = 0.f;
     if (again) __syncthreads();  // every wave is done with the previous piece's buffers
-    attend_chunks<Tag, D, false, true, kTerms>(lds, s_bad, kc, vc, num_slots, kvs_slot,
+    attend_chunks<Tag, D, false, true, kTerms>(lds, s_bad, s_odd, kc, vc, num_slots, kvs_slot,
                                  int64_t(kvh) * kvs_head, bt, bt_row, log2_bs, kbeg, kfin, lim,
-                                 lim_min, wave_has_rows, qop, scale_log2, blk0, blk1, m, lpart, acc,
+                                 lim_min, tile_lim, wave_has_rows, qop, scale_log2, blk0, blk1, m, lpart, acc,
                                  any_bad);
     lpart += dsp_shfl_xor(lpart, 32);
     if (c0 == 0 && c1 == nch) {

@@ -197,3 +197,54 @@ def test_infinite_values_stay_infinite(hip, dtype, form, G, KVH, D, q_lens, ctx)
     got, odd = f64(out), ~np.isfinite(want)
     assert np.array_equal(got[odd], want[odd], equal_nan=True)
     assert np.abs(got[~odd] - want[~odd]).max() <= 2 * P_ERR[dtype] * 6
+
+# ---- infinities and NaN in a token's V and K: only the rows that see the token get them
+@pytest.mark.parametrize("form,dtype,D", [
+    ("grid", torch.float32, 8), ("grid", torch.float32, 16), ("grid", torch.float32, 64),
+    ("grid", torch.float32, 256), ("grid", torch.bfloat16, 256), ("grid", torch.float16, 256),
+    ("ragged", torch.bfloat16, 64), ("ragged", torch.float16, 64), ("ragged", torch.bfloat16, 128),
+    ("ragged", torch.float16, 128), ("ragged", torch.bfloat16, 256), ("ragged", torch.float16, 256)])
+@pytest.mark.parametrize("q_lens,ctx", [([9, 1, 4], [300, 64, 4]), ([150, 70, 1], [900, 70, 129]),
+                                        ([70, 3], [70, 1000])])
+@pytest.mark.parametrize("G", [1, 3])
+def test_a_token_spoils_the_rows_that_see_it(hip, form, dtype, D, q_lens, ctx, G):
+    """Two of each sequence's new tokens (its only one where it has one) hold NaN, inf and -inf in
+    some dims of V: the later rows have them there, the earlier ones are as if they were zeros."""
+    from dispec_amd.engine.hip_attn import paged_mq_attention
+    KVH, bs = 2, 16
+    kc, vc, bt, keys = _spoiled(ctx, KVH, D, dtype, [])
+    clean = vc.clone()
+    first = {}                          # row -> tokens of its sequence that are spoilt and seen
+    at = 0
+    for n, c, slots in zip(q_lens, ctx, keys):
+        spoilt = sorted({n // 2, n - 1})
+        for i in spoilt:
+            s = int(slots[c - n + i])
+            vc[s, 0, 1], vc[s, 0, 3], vc[s, 0, D - 1] = float("nan"), float("inf"), -float("inf")
+            vc[s, 1, 2] = float("inf") if i == n - 1 else -float("inf")
+            vc[s, 1, 0] = float("inf")
+            clean[s, 0, [1, 3, D - 1]], clean[s, 1, :3:2] = 0, 0
+        for i in range(n):
+            first[at + i] = [t for t in spoilt if t <= i]
+        at += n
+    q = randn((sum(q_lens), G * KVH, D), 5, dtype).to(DEV)
+    cu = _i32([0] + list(np.cumsum(q_lens)))
+    if form == "ragged":
+        out = _ragged(q, kc, vc, bt, cu, _i32(ctx), G, max(q_lens), bt.shape[1] * bs)
+    else:
+        out = paged_mq_attention(q, kc, vc, bt, cu, _i32(ctx), G, max_q_len=max(q_lens))
+    want = ref_cpu.mq_attention(f64(q), f64(kc), f64(clean), keys, q_lens, G)
+    inf = np.inf
+    ends = {a - 1 for a in np.cumsum(q_lens)}
+    for t, seen in first.items():
+        if seen:
+            want[t, :G, 1], want[t, :G, 3], want[t, :G, D - 1] = np.nan, inf, -inf
+            want[t, G:, 0] = inf
+            # the sequence's last token has inf where an earlier one has -inf
+            want[t, G:, 2] = -inf if t not in ends else (inf if len(seen) == 1 else np.nan)
+    got = f64(out)
+    odd = ~np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[odd & ~np.isnan(want)], want[odd & ~np.isnan(want)])
+    err = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11 if dtype == torch.float16 else 1e-6
+    assert np.abs(got[~odd] - want[~odd]).max() <= err * 6
