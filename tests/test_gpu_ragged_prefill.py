@@ -173,3 +173,51 @@ def test_the_rule_and_its_refusals(hip, monkeypatch):
     assert call([4] * 32, [1000] * 32) == [("", 0)]
     assert call([5] * 32, [1000] * 32, slots=1032) == [("", 0)]
     assert call(*mixed, G=2, D=256, slots=1016) == [("_ragged", _lib.DSP_EUNSUPPORTED), ("", 0)]
+
+
+# ---- a lost, doubled or misplaced chunk shows whatever the length of the row
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("q_lens,ctx,G,KVH,D", [
+    *[(*b, 7, 2, 128) for b in BATCHES], *[(*b, 3, 3, 64) for b in BATCHES[:1] + BATCHES[3:5]],
+    (*BATCHES[0], 4, 2, 256), ([5] * 33, [200 + 61 * i for i in range(33)], 7, 4, 128),
+    ([9, 18, 1], [4000, 18, 3000], 7, 2, 64),
+    ([1] * 24 + [1300], [100 + 90 * i for i in range(24)] + [1377], 7, 2, 128),   # 72 tiles
+    ([1, 7900, 3], [5000, 8000, 64], 7, 1, 128),                                  # 432 tiles
+    ([4000, 1], [4096, 2000], 1, 2, 64)])
+def test_every_chunk_counts_once(hip, dtype, q_lens, ctx, G, KVH, D):
+    """All scores 0, V the number of the key's chunk as a unit vector: output d of a row is the
+    share of its keys that lie in chunk d (turned by the KV head), to half a unit in the last
+    place of the type and, against a row sum of 1, that of a probability."""
+    from dispec_amd import _lib
+    bs, B, T, Hq = 16, len(ctx), sum(q_lens), G * KVH
+    need = [-(-c // bs) for c in ctx]
+    perm = torch.randperm(sum(need) + 1, generator=torch.Generator().manual_seed(4)).int()
+    bt = torch.zeros((B, max(need)), dtype=torch.int32)
+    vc = torch.zeros(((sum(need) + 1) * bs, KVH, D), dtype=dtype)
+    at = 0
+    for b, n in enumerate(need):
+        bt[b, :n] = perm[at:at + n]
+        at += n
+        j = torch.arange(ctx[b])
+        for h in range(KVH):
+            vc[bt[b].long()[j // bs] * bs + j % bs, h, (j // 64 + 17 * h) % D] = 1
+    assert max(ctx) <= 64 * D
+    q, kc = torch.zeros((T, Hq, D), dtype=dtype, device=DEV), torch.zeros_like(vc).to(DEV)
+    vc, bt = vc.to(DEV), bt.to(DEV)
+    cu, lens = (torch.tensor(x, dtype=torch.int32, device=DEV)
+                for x in ([0] + list(np.cumsum(q_lens)), ctx))
+    L, mq, mc = _lib.lib(), max(q_lens), bt.shape[1] * bs
+    size = L.dsp_paged_mq_ragged_workspace_bytes(B, Hq, KVH, D, mq, mc)
+    ws = torch.full((size // 4,), float("nan"), device=DEV)
+    out = torch.full_like(q, 7.0)
+    _lib.check(L.dsp_paged_mq_attention_ragged(
+        q.data_ptr(), q.stride(0), q.stride(1), kc.data_ptr(), vc.data_ptr(), kc.shape[0],
+        kc.stride(0), kc.stride(1), bt.data_ptr(), bt.stride(0), bs, cu.data_ptr(), lens.data_ptr(),
+        B, Hq, KVH, D, 1.0, mq, mc, ws.data_ptr(), size, out.data_ptr(), out.stride(0),
+        out.stride(1), _lib.dtype_code(dtype), None, _lib.stream_of(q)), "ragged")
+    seen = torch.cat([torch.arange(c - n + 1, c + 1) for n, c in zip(q_lens, ctx)]).to(DEV)
+    chunk = (seen[:, None] - 64 * torch.arange(D, device=DEV)).clamp(0, 64)
+    want = torch.stack([chunk.roll(17 * h, 1) for h in range(KVH)], 1).double() / seen[:, None, None]
+    want = want.repeat_interleave(G, 1)
+    half = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert bool(((out.double() - want).abs() <= want * (2 * half) + 2.0 ** -25).all())
