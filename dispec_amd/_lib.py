@@ -98,7 +98,8 @@ _CALLS = None
 # binds them with METH_FASTCALL functions that take the same arguments as the ctypes
 # functions and skip ctypes' per-argument conversion (~4-5 us a call).
 FAST_CALLS = ("dsp_paged_decode", "dsp_kv_append", "dsp_paged_mq_attention",
-              "dsp_paged_mq_attention_shared_prefix", "dsp_qk_norm_rope_append")
+              "dsp_paged_mq_attention_ragged", "dsp_paged_mq_attention_shared_prefix",
+              "dsp_qk_norm_rope_append")
 
 
 class HipLibraryError(RuntimeError):

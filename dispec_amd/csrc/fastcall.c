@@ -69,6 +69,10 @@ typedef int (*mq_fn)(void*, int64_t, int64_t, void*, void*, int64_t, int64_t, in
                      int64_t, int32_t, void*, void*, int32_t, int32_t, int32_t, int32_t, float,
                      int32_t, int32_t, int32_t, void*, size_t, void*, int64_t, int64_t, int32_t,
                      void*, void*);
+typedef int (*mq_ragged_fn)(void*, int64_t, int64_t, void*, void*, int64_t, int64_t, int64_t,
+                            void*, int64_t, int32_t, void*, void*, int32_t, int32_t, int32_t,
+                            int32_t, float, int32_t, int32_t, void*, size_t, void*, int64_t,
+                            int64_t, int32_t, void*, void*);
 typedef int (*mq_sp_fn)(void*, int64_t, int64_t, void*, void*, int64_t, int64_t, int64_t, void*,
                         int64_t, int32_t, void*, void*, int32_t, int32_t, int32_t, int32_t,
                         float, int32_t, int32_t, int32_t, int32_t, void*, size_t, void*,
@@ -81,6 +85,7 @@ typedef int (*prologue_fn)(void*, int64_t, int64_t, void*, int64_t, int64_t, voi
 static decode_fn p_decode;
 static append_fn p_append;
 static mq_fn p_mq;
+static mq_ragged_fn p_mq_ragged;
 static mq_sp_fn p_mq_sp;
 static prologue_fn p_prologue;
 
@@ -134,6 +139,21 @@ static PyObject* w_mq(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   return PyLong_FromLong(st);
 }
 
+static const char kMqRaggedSig[] = "PqqPPqqqPqiPPiiiifiiPzPqqiPP";
+static PyObject* w_mq_ragged(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+  arg_t v[32];
+  UNBOUND(p_mq_ragged, "dsp_paged_mq_attention_ragged");
+  if (!convert("dsp_paged_mq_attention_ragged", kMqRaggedSig, a, n, v)) return NULL;
+  int st;
+  Py_BEGIN_ALLOW_THREADS
+  st = p_mq_ragged(v[0].p, v[1].q, v[2].q, v[3].p, v[4].p, v[5].q, v[6].q, v[7].q,
+                   v[8].p, v[9].q, v[10].i, v[11].p, v[12].p, v[13].i, v[14].i,
+                   v[15].i, v[16].i, v[17].f, v[18].i, v[19].i, v[20].p, v[21].z,
+                   v[22].p, v[23].q, v[24].q, v[25].i, v[26].p, v[27].p);
+  Py_END_ALLOW_THREADS
+  return PyLong_FromLong(st);
+}
+
 static const char kMqSpSig[] = "PqqPPqqqPqiPPiiiifiiiiPzPqqiPP";
 static PyObject* w_mq_sp(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   arg_t v[32];
@@ -175,6 +195,7 @@ static PyObject* w_bind(PyObject* self, PyObject* args) {
   if (!strcmp(name, "dsp_paged_decode")) p_decode = (decode_fn)p;
   else if (!strcmp(name, "dsp_kv_append")) p_append = (append_fn)p;
   else if (!strcmp(name, "dsp_paged_mq_attention")) p_mq = (mq_fn)p;
+  else if (!strcmp(name, "dsp_paged_mq_attention_ragged")) p_mq_ragged = (mq_ragged_fn)p;
   else if (!strcmp(name, "dsp_paged_mq_attention_shared_prefix")) p_mq_sp = (mq_sp_fn)p;
   else if (!strcmp(name, "dsp_qk_norm_rope_append")) p_prologue = (prologue_fn)p;
   else {
@@ -189,6 +210,8 @@ static PyMethodDef kMethods[] = {
     {"dsp_paged_decode", (PyCFunction)(void (*)(void))w_decode, METH_FASTCALL, NULL},
     {"dsp_kv_append", (PyCFunction)(void (*)(void))w_append, METH_FASTCALL, NULL},
     {"dsp_paged_mq_attention", (PyCFunction)(void (*)(void))w_mq, METH_FASTCALL, NULL},
+    {"dsp_paged_mq_attention_ragged", (PyCFunction)(void (*)(void))w_mq_ragged, METH_FASTCALL,
+     NULL},
     {"dsp_paged_mq_attention_shared_prefix", (PyCFunction)(void (*)(void))w_mq_sp,
      METH_FASTCALL, NULL},
     {"dsp_qk_norm_rope_append", (PyCFunction)(void (*)(void))w_prologue, METH_FASTCALL, NULL},
@@ -206,6 +229,7 @@ PyMODINIT_FUNC PyInit__fastcall(void) {
   } kSigs[] = {{"dsp_paged_decode", kDecodeSig},
                {"dsp_kv_append", kAppendSig},
                {"dsp_paged_mq_attention", kMqSig},
+               {"dsp_paged_mq_attention_ragged", kMqRaggedSig},
                {"dsp_paged_mq_attention_shared_prefix", kMqSpSig},
                {"dsp_qk_norm_rope_append", kPrologueSig}};
   PyObject* m = PyModule_Create(&kModule);

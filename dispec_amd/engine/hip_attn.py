@@ -39,6 +39,7 @@ def _ragged_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx) -> int:
     return _lib.lib().dsp_paged_mq_ragged_workspace_bytes(B, Hq, KVH, D, max_q_len, max_ctx)
 
 
+@functools.lru_cache(maxsize=1024)
 def _prefer_ragged(T, B, KVH, G, D, max_q_len, max_ctx) -> bool:
     """Whether a batch runs on 128-row tiles with their chunks dealt out in equal shares
     (dsp_paged_mq_attention_ragged) rather than as a grid of the longest block's tiles for
@@ -271,34 +272,52 @@ def paged_mq_attention(q, k_cache, v_cache, block_table, cu_q, ctx_lens, kv_grou
     else:
         P = int(partition_tokens)   # 0: the library picks the partition
     stream = _lib.stream_of(q)
-    max_q_len, max_ctx, rows = int(max_q_len), int(max_ctx), int(max_q_len) * kv_groups
-    ragged = 0
-    if (rows > 16 and not sp and not P and q.dtype != torch.float32 and D in (64, 128, 256)
-            and block_size >= 16 and (rows >= 128 or S % block_size == 0)
-            and _prefer_ragged(T, B, KVH, kv_groups, D, max_q_len, max_ctx)):
-        ragged = _ragged_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx)
-    head = (q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(), S,
-            k_cache.stride(0), k_cache.stride(1), block_table.data_ptr(), block_table.stride(0),
-            block_size, cu_q.data_ptr(), ctx_lens.data_ptr(), B, Hq, KVH, D, float(scale),
-            max_q_len, max_ctx)
-    tail = (out.data_ptr(), out.stride(0), out.stride(1), _lib.dtype_code(q.dtype),
-            _lib.ptr(err), stream)
-    if ragged:
-        # up to 67 MB whatever the batch: taken from torch's stream-ordered allocator per call
-        parts = torch.empty(ragged // 4, dtype=torch.float32, device=q.device)
-        st = L.dsp_paged_mq_attention_ragged(*head, parts.data_ptr(), ragged, *tail)
-        # a pool or rows it does not take: the grid of fixed partitions below
-        if st not in (_lib.DSP_EUNSUPPORTED, _lib.DSP_EALIGN):
-            _lib.check(st, "dsp_paged_mq_attention_ragged")
-            return out
+    max_q_len, max_ctx = int(max_q_len), int(max_ctx)
+    # (calls of up to 16 rows, verify and decode of forks, pay one comparison for the ragged launch)
+    if (max_q_len * kv_groups > 16 and not P and not sp
+            and _ragged(q, k_cache, v_cache, block_table, cu_q, ctx_lens, block_size, scale,
+                        max_q_len, max_ctx, out, err, stream)):
+        return out
     need = _mq_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx, P)
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = _workspace(need, q.device, stream)
     ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    tail = (_lib.ptr(workspace), ws_bytes, *tail)
+    head = (q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(), S,
+            k_cache.stride(0), k_cache.stride(1), block_table.data_ptr(), block_table.stride(0),
+            block_size, cu_q.data_ptr(), ctx_lens.data_ptr(), B, Hq, KVH, D, float(scale),
+            max_q_len, max_ctx)
+    tail = (_lib.ptr(workspace), ws_bytes, out.data_ptr(), out.stride(0), out.stride(1),
+            _lib.dtype_code(q.dtype), _lib.ptr(err), stream)
     if sp:
         _lib.check(L.dsp_paged_mq_attention_shared_prefix(*head, sp, int(P), *tail),
                    "dsp_paged_mq_attention_shared_prefix")
     else:
         _lib.check(L.dsp_paged_mq_attention(*head, int(P), *tail), "dsp_paged_mq_attention")
     return out
+
+
+def _ragged(q, k_cache, v_cache, block_table, cu_q, ctx_lens, block_size, scale, max_q_len, max_ctx,
+            out, err, stream) -> bool:
+    """dsp_paged_mq_attention_ragged where it is the better launch (_prefer_ragged) and takes the
+    call; False, having done nothing, otherwise."""
+    (T, Hq, D), (S, KVH, _), B = q.shape, k_cache.shape, ctx_lens.numel()
+    rows = max_q_len * (Hq // KVH)
+    if (q.dtype == torch.float32 or D not in (64, 128, 256) or block_size < 16
+            or rows < 128 and S % block_size
+            or not _prefer_ragged(T, B, KVH, Hq // KVH, D, max_q_len, max_ctx)):
+        return False
+    need = _ragged_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx)
+    if not need:
+        return False
+    # up to 67 MB whatever the batch: taken from torch's stream-ordered allocator per call
+    parts = torch.empty(need // 4, dtype=torch.float32, device=q.device)
+    st = _lib.calls().dsp_paged_mq_attention_ragged(
+        q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(), S,
+        k_cache.stride(0), k_cache.stride(1), block_table.data_ptr(), block_table.stride(0),
+        block_size, cu_q.data_ptr(), ctx_lens.data_ptr(), B, Hq, KVH, D, float(scale), max_q_len,
+        max_ctx, parts.data_ptr(), need, out.data_ptr(), out.stride(0), out.stride(1),
+        _lib.dtype_code(q.dtype), _lib.ptr(err), stream)
+    if st in (_lib.DSP_EUNSUPPORTED, _lib.DSP_EALIGN):   # a pool or rows it does not take
+        return False
+    _lib.check(st, "dsp_paged_mq_attention_ragged")
+    return True

@@ -87,6 +87,17 @@ def test_multi_query_statuses_match():
             assert slow(*a) == fast(*a) == st, (name, B)
 
 
+def test_ragged_statuses_match():
+    slow, fast = _both("dsp_paged_mq_attention_ragged")
+    p = 4096
+    head = (p, 1024, 128, p, p, 4096, 256, 128, p, 64, 16, p, p)
+    for B, dtype, st in ((0, _lib.DSP_BF16, _lib.DSP_OK), (-3, _lib.DSP_BF16, _lib.DSP_EINVAL),
+                         (2, _lib.DSP_F32, _lib.DSP_EUNSUPPORTED),
+                         (2, _lib.DSP_BF16, _lib.DSP_EWORKSPACE)):
+        a = head + (B, 8, 2, 128, 0.088, 5, 1024, None, 0, p, 1024, 128, dtype, None, None)
+        assert slow(*a) == fast(*a) == st, (B, dtype)
+
+
 def test_prologue_statuses_match():
     slow, fast = _both("dsp_qk_norm_rope_append")
     p = 4096
