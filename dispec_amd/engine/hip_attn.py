@@ -43,29 +43,55 @@ def _ragged_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx) -> int:
 def _prefer_ragged(T, B, KVH, G, D, max_q_len, max_ctx) -> bool:
     """Whether a batch runs on 128-row tiles with their chunks dealt out in equal shares
     (dsp_paged_mq_attention_ragged) rather than as a grid of the longest block's tiles for
-    every sequence.
+    every sequence.  The lengths are on the device, so the rule knows their bounds and the number
+    of tokens only: it takes the shapes whose batches gain nearly whatever their lengths are.
+    The lines were drawn on 16000 random batches of nine head shapes (2 to 8 KV heads of 64 to 256)
+    and checked on 10000 others, with contexts of 20 to 32768 tokens, alike or with one or two
+    long ones (figures: grid / shares, us a layer).
 
-    Blocks of 17 to 127 rows (verify): the grid's 16-row tiles read the keys once each, the
-    128-row tile once for all of them, which pays for its start-up and merge from about
-    256K keys of 128 (sequences times KV heads times max_ctx).  A long context over few KV
-    heads would be cut into more than 64 pieces for one merge, so it stays on the grid.
-    (us, grid / shares: 28 heads over 4, 32 verifies of 5 over 500-4000 keys 86/41; 12 over 2,
-    64 of 3-8 83/40; 32 over 8, 24 of 5 95/57; 14 over 2 of 64, 64 of 2-9 50/34; 16 over 8, 32
-    of 2-9 79/69.  Below the line: 32 over 8, 5 of 1-7 over 1109-5647 26/30; 14 over 2 of 64, 26
-    of 1-4 25/30; one of 6000 keys among 19 of 50-400, 12 over 2, 24/32, among 39 39/33.  One
-    of 30000 among 7, 12 over 2, 41/90.)
+    W: workgroups that fit the chip, each of which gets a share.
 
-    Longer blocks: when that grid has at least three times the tiles that the T query tokens
-    can fill, and is not small.  (us, grid / shares, heads 14 over 2 of 64, 28 over 4 and 32
-    over 8 of 128: 24 decodes and a 700-token chunk 52/36, 118/56, 153/69; 30 decodes and two
-    1000-token chunks 155/56, 498/135, 605/165; but 2 decodes and a 1000-token prompt, 2.9
-    times the tiles, 27/27, 41/46, 46/52, and four equal chunks 54/67, 128/155, 135/161.)"""
-    if max_q_len * G < 128:
-        return (max_q_len * G > 16 and B * KVH * max_ctx * D >= 128 * (256 << 10)
-                and (max_ctx <= 6144 or KVH >= 8 and D >= 128))
-    grid = KVH * B * (-(-max_q_len * G // 128))
+    Blocks of 17 to 127 rows (verify).  The grid's 16-row tiles read the keys once each, the 128-row
+    tile once for all of them, which pays for its start-up and merge from about 256K keys of 128
+    (sequences times KV heads times max_ctx), and where
+    * at least W / 4 (sequence, KV head) pairs share the work: one long context among fewer would
+      be cut into many pieces for one merge (one of 11360 among 3, 16 heads over 8: 25 / 42; one of
+      30000 among 7, 12 over 2: 41 / 90);
+    * the table is not so wide that few KV heads give a merge more than 64 pieces;
+    * a third of the queries that B blocks of max_q_len would have are there: not one chunk beside
+      decodes (one of 46 beside 66, 16 over 8: 101 / 163), unless contexts reach 6144 tokens;
+    * heads are at most 128 wide (below 12288 tokens: 256-wide verifies lost every second time).
+    Of the batches checked, 1.9 times as fast at the median; 1 in 80 slower by more than 3 %, 1 in
+    160 by more than 10 %.  (28 heads over 4, 32 verifies of 5 over 500-4000 keys 86 / 41; 32 over
+    8, 24 of 5 95 / 57.)
+
+    Longer blocks.  The grid has at least 256 tiles and several times those that the T query tokens
+    can fill, and
+    * filled tiles times the longest context give every worker seven chunks or more (31 decodes of
+      600 keys and a 159-token chunk, 14 over 2 of 64: 20 / 26);
+    * from half a filled tile per worker to about one, where a share cuts nearly every tile in two
+      for the merge and contexts of similar length need no shares (58 decodes of about 1200 keys and
+      a 148-token chunk, 32 over 8: 52 / 93), the grid has to be 9 or 14 times too large; elsewhere,
+      and for heads wider than 128, 5 times; 3 times from 8192 tokens on.
+    Of the batches checked, 2.8 times as fast at the median; 1 in 100 slower by more than 3 %, 1 in
+    200 by more than 10 %.  (24 decodes and a 700-token chunk, 28 over 4: 118 / 56.)"""
+    workers = _ragged_ws_bytes(B, KVH * G, KVH, D, max_q_len, max_ctx) // (4 * (256 * (D + 2) + 4))
+    if not workers:
+        return False
+    rows = max_q_len * G
+    if rows < 128:
+        return (rows > 16 and B * KVH * max_ctx * D >= 128 * (256 << 10)
+                and (max_ctx <= 6144 or KVH >= 8 and D >= 128)
+                and 4 * B * KVH >= workers
+                and (max_ctx >= 6144 or T >= 0.35 * B * max_q_len)
+                and (D <= 128 or max_ctx >= 12288))
+    grid = KVH * B * (-(-rows // 128))
     filled = KVH * (B + (T - B) * G / 128)
-    return grid >= 256 and grid >= 3 * filled
+    if grid < 256 or max_ctx >= 8192:
+        return grid >= 256 and grid >= 3 * filled
+    load = filled / workers
+    spare = 5 if D > 128 or load <= 0.45 or load >= 1.3 else 9 if load < 0.7 else 14
+    return grid >= spare * filled and load * max_ctx >= 7 * 64
 
 
 # Split-K workspaces of calls that bring none, one per (device, stream): kernels on one
