@@ -6,8 +6,10 @@ same argument meaning, the per-token int32 slot table, `scale = scale or D ** -0
 an output allocated like `torch.empty_like(q)`.  They call `dsp_paged_decode`, a
 GQA-packed split-K kernel with a log-sum-exp combine, instead of one Triton program per
 (sequence, query head).  Like the Triton kernel they take any power-of-two head_dim from 8
-to 256 and fp32 caches as well as bf16 / fp16: shapes outside the tuned kernels (fp32, head
-dims 8 and 256, more than 8 query heads per KV head) run on a generic wave-per-row kernel.
+to 256 and fp32 caches as well as bf16 / fp16: fp32 runs on 16-row tiles of the fp32 matrix
+cores, and the 16-bit shapes that the tuned kernels leave out (head_dim 8; slot tables or rows
+off 16-byte alignment with 256-wide heads or more than 8 query heads per KV head) on a generic
+wave-per-row kernel.
 
 `paged_decode_attention_blocks` is the block-table form (the table is
 [B, max_blocks] int32 instead of [B, max_ctx] slots), the one `ModelRunner` uses.
@@ -217,8 +219,9 @@ def decode_workspace(batch, num_heads, num_kv_heads, head_dim, max_ctx, device):
 def mq_workspace(batch, num_heads, num_kv_heads, head_dim, max_q_len, max_ctx, device,
                  shared_prefix_tokens=0, balanced=False):
     """A float32 split-K workspace for every `paged_mq_attention` launch of this shape with
-    the automatic partition (or the balanced split), or None when it needs none.  One
-    buffer serves all layers of a forward: the launches run in stream order."""
+    the automatic partition (or the balanced split), whichever of its launches the call takes,
+    or None when it needs none.  One buffer serves all layers of a forward: the launches run in
+    stream order."""
     L = _lib.calls()
     if shared_prefix_tokens:
         P = L.dsp_paged_mq_shared_prefix_partition_tokens(
@@ -227,6 +230,14 @@ def mq_workspace(batch, num_heads, num_kv_heads, head_dim, max_q_len, max_ctx, d
         P = _lib.DSP_SPLIT_BALANCED if balanced else 0
     need = L.dsp_paged_mq_workspace_bytes(batch, num_heads, num_kv_heads, head_dim, max_q_len,
                                           max_ctx, P)
+    G = num_heads // num_kv_heads
+    if not P and max_q_len * G > 16 and any(
+            _prefer_ragged(batch + full * (max_q_len - 1), batch, num_kv_heads, G, head_dim,
+                           max_q_len, max_ctx)
+            for full in (batch >> i for i in range(batch.bit_length()))):
+        # (the number of tokens is not known here: 1, 2, 4, ... blocks of max_q_len, others of 1)
+        need = max(need, _ragged_ws_bytes(batch, num_heads, num_kv_heads, head_dim, max_q_len,
+                                          max_ctx))
     return torch.empty(need // 4 + 1, dtype=torch.float32, device=device) if need else None
 
 
@@ -302,7 +313,7 @@ def paged_mq_attention(q, k_cache, v_cache, block_table, cu_q, ctx_lens, kv_grou
     # (calls of up to 16 rows, verify and decode of forks, pay one comparison for the ragged launch)
     if (max_q_len * kv_groups > 16 and not P and not sp
             and _ragged(q, k_cache, v_cache, block_table, cu_q, ctx_lens, block_size, scale,
-                        max_q_len, max_ctx, out, err, stream)):
+                        max_q_len, max_ctx, workspace, out, err, stream)):
         return out
     need = _mq_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx, P)
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
@@ -323,7 +334,7 @@ def paged_mq_attention(q, k_cache, v_cache, block_table, cu_q, ctx_lens, kv_grou
 
 
 def _ragged(q, k_cache, v_cache, block_table, cu_q, ctx_lens, block_size, scale, max_q_len, max_ctx,
-            out, err, stream) -> bool:
+            workspace, out, err, stream) -> bool:
     """dsp_paged_mq_attention_ragged where it is the better launch (_prefer_ragged) and takes the
     call; False, having done nothing, otherwise."""
     (T, Hq, D), (S, KVH, _), B = q.shape, k_cache.shape, ctx_lens.numel()
@@ -335,13 +346,14 @@ def _ragged(q, k_cache, v_cache, block_table, cu_q, ctx_lens, block_size, scale,
     need = _ragged_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx)
     if not need:
         return False
-    # up to 67 MB whatever the batch: taken from torch's stream-ordered allocator per call
-    parts = torch.empty(need // 4, dtype=torch.float32, device=q.device)
+    if workspace is None or workspace.numel() * workspace.element_size() < need:
+        # up to 67 MB whatever the batch: taken from torch's stream-ordered allocator per call
+        workspace = torch.empty(need // 4, dtype=torch.float32, device=q.device)
     st = _lib.calls().dsp_paged_mq_attention_ragged(
         q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(), S,
         k_cache.stride(0), k_cache.stride(1), block_table.data_ptr(), block_table.stride(0),
         block_size, cu_q.data_ptr(), ctx_lens.data_ptr(), B, Hq, KVH, D, float(scale), max_q_len,
-        max_ctx, parts.data_ptr(), need, out.data_ptr(), out.stride(0), out.stride(1),
+        max_ctx, workspace.data_ptr(), need, out.data_ptr(), out.stride(0), out.stride(1),
         _lib.dtype_code(q.dtype), _lib.ptr(err), stream)
     if st in (_lib.DSP_EUNSUPPORTED, _lib.DSP_EALIGN):   # a pool or rows it does not take
         return False

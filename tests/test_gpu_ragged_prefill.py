@@ -221,3 +221,35 @@ def test_every_chunk_counts_once(hip, dtype, q_lens, ctx, G, KVH, D):
     want = want.repeat_interleave(G, 1)
     half = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     assert bool(((out.double() - want).abs() <= want * (2 * half) + 2.0 ** -25).all())
+
+
+@pytest.mark.parametrize("q_lens,ctx", [([1] * 24 + [700], [100 + 90 * i for i in range(24)] + [1501]),
+                                        ([5] * 40, [3000] * 40)])
+def test_a_callers_workspace_serves_the_ragged_launch(hip, q_lens, ctx):
+    """mq_workspace covers it, and a call that is handed the buffer allocates nothing."""
+    from dispec_amd.engine.hip_attn import _prefer_ragged, mq_workspace, paged_mq_attention
+    G, KVH, D, bs = 7, 4, 128, 16
+    B, T, mq = len(ctx), sum(q_lens), max(q_lens)
+    width = -(-max(ctx) // bs)
+    assert _prefer_ragged(T, B, KVH, G, D, mq, width * bs)
+    kc, vc = (randn((width * bs, KVH, D), s, torch.bfloat16).to(DEV) for s in (1, 2))
+    bt = torch.arange(width, dtype=torch.int32, device=DEV).repeat(B, 1)
+    q = randn((T, G * KVH, D), 3, torch.bfloat16).to(DEV)
+    cu, lens = (torch.tensor(x, dtype=torch.int32, device=DEV)
+                for x in ([0] + list(np.cumsum(q_lens)), ctx))
+    ws = mq_workspace(B, G * KVH, KVH, D, mq, width * bs, DEV)
+    out, want = torch.empty_like(q), torch.empty_like(q)
+
+    def call(o, w):
+        paged_mq_attention(q, kc, vc, bt, cu, lens, G, block_size=bs, max_q_len=mq,
+                           max_ctx=width * bs, out=o, workspace=w)
+
+    call(want, None)
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    call(out, ws)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
+    assert torch.equal(out, want)
+    small = torch.empty(16, device=DEV)     # too small: the call brings its own
+    out.zero_()
+    call(out, small)
+    assert torch.equal(out, want)
