@@ -338,8 +338,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
     }
     if (nparts == 1) {
       const int qrow = q0 + row / G, hh = kvh * G + row % G;
-      // (no keys: 0 * 0; a NaN score makes L and A NaN, and the row with them)
-      out[int64_t(qrow) * ost + int64_t(hh) * osh + d] = narrow<Tag>(L > 0.f ? A / L : A * 0.f);
+      // (L 0: no keys; a NaN score makes L and A NaN, and the row with them)
+      out[int64_t(qrow) * ost + int64_t(hh) * osh + d] = narrow<Tag>(L == 0.f ? 0.f : A / L);
     } else if (kDecode) {
       const int64_t wrow = (int64_t(b) * KVH * G + kvh * G + row) * num_parts + part;
       ws_acc[wrow * D + d] = A;
