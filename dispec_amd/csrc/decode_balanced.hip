@@ -670,7 +670,9 @@ int launch_balanced(int D, A... args) {
     case 32: return launch_balanced_d<Tag, 32, kMode>(args...);
     case 64: return launch_balanced_d<Tag, 64, kMode>(args...);
     case 128: return launch_balanced_d<Tag, 128, kMode>(args...);
-    case 256: return launch_balanced_d<Tag, 256, kMode == kPlain ? kWide : kMode>(args...);
+    case 256:  // block tables only (balanced_decode_applies: no slot tables of 256-wide heads)
+      if constexpr (kMode != kSlots) return launch_balanced_d<Tag, 256, kWide>(args...);
+      return DSP_EUNSUPPORTED;
     default: return DSP_EUNSUPPORTED;
   }
 }

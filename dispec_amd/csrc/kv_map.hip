@@ -311,7 +311,7 @@ __device__ __forceinline__ void map_tile(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   // This wave's loads: instruction j covers tile rows 8 * (wave * kLPW + j) .. +7 (A rows
-  // for waves 0-3, Bt rows for waves 4-7); lane l fills slot l % 8 of row l / 8, i.e.
+  // for the first half of the waves, Bt rows for the second); lane l fills slot l % 8 of row l / 8, i.e.
   // chunk (l % 8) ^ (row & 7).  Rows past M / N are clamped to the last row (their outputs are
   // never stored).  Element offsets fit 32 bits (checked on the host).
   const bool loads_a = wave * TL::kLPW * 64 < TL::kBM * big::kCPR;
@@ -547,7 +547,7 @@ __global__ __launch_bounds__(big::kNT) void map_gemm_big_kernel(
 }
 
 // Many maps in one launch (dsp_kv_map_group): the layers' key and value maps of one prompt.
-constexpr int kMaxGroup = 80;  // 40 bytes an entry: the kernel arguments stay below 4 KiB
+constexpr int kMaxGroup = 80;  // the kernel arguments stay below 4 KiB (checked below)
 struct GroupEntry {
   const uint16_t* bt;
   const uint16_t* bias;
@@ -560,6 +560,8 @@ struct GroupArgs {
   uint16_t* c[2];              // target layers
   int64_t a_layer_stride, c_layer_stride;
 };
+static_assert(sizeof(GroupArgs) + sizeof(PoolOut) + 5 * sizeof(int64_t) <= 4096,
+              "map_group_kernel's arguments");
 
 // 1-D grid over (map, m tile, n tile), n fastest: a prompt of a few hundred tokens has 4 to 16
 // tiles per map, so one map alone leaves most of the chip idle.  72 maps of 1023 tokens: 2420

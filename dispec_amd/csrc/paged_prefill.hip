@@ -144,15 +144,14 @@ __device__ __forceinline__ void attend_chunks(
   // swizzled by (row & (CPR-1)) for the A-operand reads (32 rows, one 16-byte chunk each);
   // V rows by whole 64-byte groups (4 chunks): 4*(row & 3) at D 128 and 4*((row >> 1) & 1)
   // at D 64, so each half-wave of a transposing read (4 consecutive rows x 64 bytes) covers
-  // all 64 banks once.  Rows past kfin repeat the last key's row (finite data, masked);
-  // an out-of-range slot reads slot 0.
+  // all 64 banks once.
   auto kswz = [](int row) { return row & (CPR - 1); };
   auto vswz = [](int row) { return D >= 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1); };
   // Wave w loads rows 16*w .. 16*w + 15 of each chunk.  Chunks start at multiples of 64
   // keys and blocks hold a multiple of 16 tokens, so those rows lie in one block: its id
   // is wave-uniform and the addresses are a scalar base plus per-lane constants.  Rows past
-  // kfin read other slots of the same block (finite data, masked); an out-of-range block
-  // reads slots 0..15.
+  // kfin, masked, read other slots of the same block, with kMaskBad the last key's again; an
+  // out-of-range block reads slots 0..15 (with kMaskBad its V is zeroed then).
   static_assert(LPW * RPI == 16, "16 rows per wave per chunk");
   uint32_t koff[LPW], voff[LPW];
 #pragma unroll

@@ -200,24 +200,27 @@ int dsp_kv_scatter_ordered(void* k_pool, void* v_pool, int64_t num_layers,
  *                  asks for the balanced split whatever the size (block tables, D in {32,
  *                  64, 128}, G <= 8, B <= 512; else DSP_EUNSUPPORTED).  0 with a slot table
  *                  of 16 to 512 sequences, more than 512 wide and of 16384 entries or
- *                  more: the balanced split too (probabilities kept to fp32 accuracy,
- *                  bad slots masked and counted once per KV head).  Otherwise fixed partitions of partition_tokens keys (0: chosen by
- *                  dsp_paged_decode_partition_tokens) per (sequence, KV head), merged by
- *                  the combine kernel when a sequence spans more than one.  `workspace`
+ *                  more: the balanced split too (probabilities in fp32, bad slots skipped
+ *                  and counted once per KV head).  Otherwise fixed partitions of
+ *                  partition_tokens keys (0: chosen by dsp_paged_decode_partition_tokens)
+ *                  per (sequence, KV head), merged by the combine kernel when a sequence
+ *                  spans more than one.  `workspace`
  *                  must hold dsp_paged_decode_workspace_bytes(..., partition_tokens)
  *                  bytes (16-byte aligned) for the same arguments, on the same device.
  * dtype: DSP_BF16, DSP_F16 or DSP_F32 (caches, q and out all of it).  The tuned kernels
  * serve bf16 / fp16 with D in {16, 32, 64, 128} and G = Hq / KVH in 1..8, and on block tables
- * with 16-byte-aligned rows D 256 and any G too (probabilities kept to fp32 accuracy there,
- * in P.V as well); every other shape with D a power of two from 8 to 256 (fp32, D 8, slot
+ * with 16-byte-aligned rows D 256 and any G too (probabilities in fp32 there, in P.V as
+ * well); every other shape with D a power of two from 8 to 256 (fp32, D 8, slot
  * tables or unaligned rows with D 256 or G above 8) runs on a generic kernel -- fp32 on 16-row
  * tiles of the fp32 matrix cores, 16-bit one wave per (sequence, query head, partition); fp32
- * accumulation, element-aligned pointers -- whose automatic partition is dsp_paged_decode_partition_tokens
- * and whose workspace is covered by dsp_paged_decode_workspace_bytes.  Other D:
- * DSP_EUNSUPPORTED.
+ * accumulation, element-aligned pointers -- whose automatic partition is
+ * dsp_paged_decode_partition_tokens and whose workspace is covered by
+ * dsp_paged_decode_workspace_bytes.  Other D: DSP_EUNSUPPORTED.
  * err_count (optional) is incremented for a context length outside [0, max_ctx]
  * (clamped) and, on block tables and the generic kernel, once per wave (fp32: per
- * query row and partition) that met a block id whose slots lie outside the cache (those keys are skipped). */
+ * query row and partition) that met a block id whose slots lie outside the cache.  Its slots
+ * are never read; its keys are skipped by slot table, at D 256, with G above 8 and on the
+ * generic kernel, and elsewhere count as keys of unspecified values. */
 size_t dsp_paged_decode_workspace_bytes(int32_t B, int32_t Hq, int32_t KVH, int32_t D,
                                         int32_t max_ctx, int32_t partition_tokens);
 int dsp_paged_decode_partition_tokens(int32_t B, int32_t KVH, int32_t D, int32_t max_ctx);
@@ -287,14 +290,16 @@ int dsp_paged_decode_noalloc(const void* q, int64_t q_stride_b, int64_t q_stride
  *                tokens, B <= 512, D in {32, 64, 128} (else DSP_EUNSUPPORTED) and always
  *                `workspace` (dsp_paged_mq_workspace_bytes with DSP_SPLIT_BALANCED).
  * dtype DSP_BF16 / DSP_F16 with D in {32, 64, 128}, or 256 with 16-byte-aligned rows, on the
- * tuned kernels; DSP_F32, or D 8 or 16 (or 256 unaligned), on a generic kernel (one wave per query row, head and key partition; fixed
- * partitions only -- DSP_SPLIT_BALANCED and the shared-prefix entry return
+ * tuned kernels; DSP_F32 on 16-row tiles of the fp32 matrix cores and D 8 or 16 (or 256
+ * unaligned) on a generic kernel, one wave per query row, head and key partition (both on
+ * fixed partitions only -- DSP_SPLIT_BALANCED and the shared-prefix entry return
  * DSP_EUNSUPPORTED for them); any G = Hq / KVH.  A sequence with q_len > ctx or
  * ctx > max_ctx is counted in err_count and its rows written as zeros.  A block id whose
  * slots lie outside the cache is never dereferenced: it is counted once per wave that met
- * it, and its keys are masked out on the 16-row tiles and the balanced split, read from
- * slots 0..15 on the 128-row tile (that sequence's result is then unspecified).
- * Batches with max_q_len * G >= 128 (D 64 or 128, blocks of >= 16 tokens) run on a
+ * it (fp32: per query row and partition).  Its keys are skipped with fp32 caches, at D 256 and
+ * on the generic kernel; at D 32 to 128 they count as keys of unspecified values (zeros or
+ * slots 0..15).  (With dsp_paged_mq_attention_ragged they are skipped at every D.)
+ * Batches with max_q_len * G >= 128 (D 64, 128 or 256, blocks of >= 16 tokens) run on a
  * 128-row tile built for chunked prefill; shorter ones (verify) on 16-row tiles.  The
  * automatic partition is sized for whichever runs. */
 int dsp_paged_mq_partition_tokens(int32_t B, int32_t Hq, int32_t KVH, int32_t D,
@@ -319,8 +324,9 @@ int dsp_paged_mq_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
  * tokens, B <= 512 and at most 4096 tiles of 128 rows per KV head in a sequence (else
  * DSP_EUNSUPPORTED; the workspace size is then 0, or the pool smaller than 16 slots or, at D
  * 256, not whole blocks).  workspace: dsp_paged_mq_ragged_workspace_bytes bytes, always needed,
- * 16-byte aligned.  Bad lengths as for dsp_paged_mq_attention on its 128-row tile, keys of bad
- * block ids counted and masked out (of a sequence with more than max_q_len queries the first max_q_len are computed). */
+ * 16-byte aligned.  Bad lengths as for dsp_paged_mq_attention on its 128-row tile; keys of bad
+ * block ids are counted and skipped, a block that lies partly outside the cache whole (of a
+ * sequence with more than max_q_len queries the first max_q_len are computed). */
 size_t dsp_paged_mq_ragged_workspace_bytes(int32_t B, int32_t Hq, int32_t KVH, int32_t D,
                                            int32_t max_q_len, int32_t max_ctx);
 int dsp_paged_mq_attention_ragged(const void* q, int64_t q_stride_t, int64_t q_stride_h,
