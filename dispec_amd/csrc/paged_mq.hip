@@ -169,6 +169,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
                                        16, 0, 2);
     }
   };
+  // kSplitP: the V^T operand's LDS offsets as one per nt & 3 and constants (rows 4 * grp + u and 16
+  // + 4 * grp + u all swizzle by 2 * grp, see decode_balanced.hip), where registers are short
+  int vbase[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    vbase[j] = 4 * grp * ROWB + 32 * (j ^ (((2 * grp) & (CPR - 1)) >> 1)) + 16 * (n >> 3) + 2 * (n & 7);
   // Software pipeline: once a chunk's K has fed the score MFMAs and its V sits in LDS, the
   // same registers take the loads of this wave's chunk of the next round, which then
   // overlap the softmax and P.V of the current one.  (Not across a window boundary: the
@@ -199,9 +205,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
       for (int kk = 0; kk < NKK; ++kk) sc[st] = mfma32<Tag>(kop[st][kk], qop[kk], sc[st]);
     }
     const uint32_t cur_bad[2] = {bad_keys[0], bad_keys[1]};
-    // kSplitP: the chunk's keys that count, i.e. inside the partition with an id inside the cache
-    // (uniform)
-    const uint32_t keys = kSplitP ? low_bits(kfin - t0) & ~(cur_bad[0] | cur_bad[1] << 16) : ~0u;
+    // kSplitP: the chunk's keys that count, i.e. with an id inside the cache and, for decode, inside
+    // the partition (uniform; other rows past the partition are not seen, below)
+    const uint32_t keys = kSplitP ? ~(cur_bad[0] | cur_bad[1] << 16) &
+                                        (kDecode ? low_bits(kfin - t0) : ~0u)
+                                  : ~0u;
     if (prefetch) load_k(tn);
     // Scale and causal mask; lane holds keys t0 + 16*st + 4*grp + j of packed row n.
     float s[2][4];
@@ -253,7 +261,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
     if constexpr (kSplitP && !kDecode) {
       // a chunk that the tile's first row does not see whole (uniform): infinities and NaN in
       // it go to the rows that see them only (V^T operands as below)
-      if (t0 + 31 > ctx - qlen + r0 / G && any_nonfinite<Tag, VINS>(slab)) {
+      if (t0 + 31 > ctx - qlen + r0 / G && __builtin_expect(any_nonfinite<Tag, VINS>(slab), 0)) {
         dsp_u32x4 seen;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -263,14 +271,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
           __builtin_amdgcn_sched_barrier(0);  // one tile's operands at a time: registers
-          const int d = 16 * nt + n;
           uint16_t v[8];
 #pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            const int kl = u < 4 ? 4 * grp + u : 16 + 4 * grp + (u - 4);
-            v[u] = *reinterpret_cast<const uint16_t*>(slab + kl * ROWB + 16 * swz(kl, d >> 3) +
-                                                      2 * (d & 7));
-          }
+          for (int u = 0; u < 8; ++u)
+            v[u] = *reinterpret_cast<const uint16_t*>(slab + vbase[nt & 3] +
+                                                      (u < 4 ? u : 12 + u) * ROWB + 32 * (nt & ~3));
           const dsp_u32x4 vop = dsp_u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]),
                                           pack2(v[6], v[7])};
           acc[nt] = mfma32<Bf16Tag>(odd_operand<Tag>(vop, false), seen, acc[nt]);
@@ -289,8 +294,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int kl = u < 4 ? 4 * grp + u : 16 + 4 * grp + (u - 4);
-        v[u] = *reinterpret_cast<const uint16_t*>(slab + kl * ROWB + 16 * swz(kl, d >> 3) +
-                                                  2 * (d & 7));
+        v[u] = kSplitP ? *reinterpret_cast<const uint16_t*>(
+                             slab + vbase[nt & 3] + (kl - 4 * grp) * ROWB + 32 * (nt & ~3))
+                       : *reinterpret_cast<const uint16_t*>(slab + kl * ROWB + 16 * swz(kl, d >> 3) +
+                                                            2 * (d & 7));
       }
       const dsp_u32x4 vop = dsp_u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]),
                                    pack2(v[6], v[7])};
