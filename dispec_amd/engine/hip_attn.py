@@ -312,6 +312,7 @@ def paged_mq_attention(q, k_cache, v_cache, block_table, cu_q, ctx_lens, kv_grou
     max_q_len, max_ctx = int(max_q_len), int(max_ctx)
     # (calls of up to 16 rows, verify and decode of forks, pay one comparison for the ragged launch)
     if (max_q_len * kv_groups > 16 and not P and not sp
+            and _prefer_ragged(T, B, KVH, kv_groups, D, max_q_len, max_ctx)
             and _ragged(q, k_cache, v_cache, block_table, cu_q, ctx_lens, block_size, scale,
                         max_q_len, max_ctx, workspace, out, err, stream)):
         return out
@@ -335,17 +336,13 @@ def paged_mq_attention(q, k_cache, v_cache, block_table, cu_q, ctx_lens, kv_grou
 
 def _ragged(q, k_cache, v_cache, block_table, cu_q, ctx_lens, block_size, scale, max_q_len, max_ctx,
             workspace, out, err, stream) -> bool:
-    """dsp_paged_mq_attention_ragged where it is the better launch (_prefer_ragged) and takes the
-    call; False, having done nothing, otherwise."""
-    (T, Hq, D), (S, KVH, _), B = q.shape, k_cache.shape, ctx_lens.numel()
-    rows = max_q_len * (Hq // KVH)
-    if (q.dtype == torch.float32 or D not in (64, 128, 256) or block_size < 16
-            or rows < 128 and S % block_size
-            or not _prefer_ragged(T, B, KVH, Hq // KVH, D, max_q_len, max_ctx)):
+    """dsp_paged_mq_attention_ragged, where it takes the call; False, having done nothing,
+    otherwise."""
+    (_, Hq, D), (S, KVH, _), B = q.shape, k_cache.shape, ctx_lens.numel()
+    if (q.dtype == torch.float32 or block_size < 16
+            or max_q_len * (Hq // KVH) < 128 and S % block_size):
         return False
     need = _ragged_ws_bytes(B, Hq, KVH, D, max_q_len, max_ctx)
-    if not need:
-        return False
     if workspace is None or workspace.numel() * workspace.element_size() < need:
         # up to 67 MB whatever the batch: taken from torch's stream-ordered allocator per call
         workspace = torch.empty(need // 4, dtype=torch.float32, device=q.device)
