@@ -131,7 +131,7 @@ __device__ __forceinline__ int64_t active_workers(int64_t C, int num_workers) {
 // in kWide, bad slots skipped and each counted, as they are there.  A slot-table window holds the
 // slots of 64 keys, one per lane, the next window's loaded while it is in use; a lane takes the
 // slots of its K and V rows from it by permute (24 sequences of 200-3000 keys, 28 heads over 4:
-// kernel and merge 42 -> 26 us a layer).
+// kernel and merge 42 -> 27 us a layer).
 enum Mode { kPlain, kWide, kSlots };
 template <typename Tag, int D, bool kOff32, int HG, int kMode>
 __global__ __launch_bounds__(64 * HG) __attribute__((amdgpu_waves_per_eu(D > 128 ? 2 : kOcc))) void decode_balanced_kernel(

@@ -43,8 +43,8 @@ __device__ __forceinline__ uint32_t pack2(uint16_t lo, uint16_t hi) {
 // operand takes the leading bits of what the ones before it left over, the last one its
 // rounding.  Three hold all 24 bits of an fp32 value: P.V over them is P.V of fp32
 // probabilities, for the shapes whose probabilities are fp32 (two hold 16 bits in bf16, 22 in
-// fp16; the third costs the 256-wide prefill tile 80 -> 91 us at 4 x 200 tokens over 1999, 24
-// slot-table decodes 20.7 -> 21.3).
+// fp16; with the third the 256-wide prefill tile takes 91 us instead of 82 at 4 x 200 tokens over
+// 1999, 24 slot-table decodes 21.9 instead of 20.9).
 // The leading bits are cut, not rounded, and an operand of a p above 0 is kept above 0 (by the
 // least number, 2^-100 or the last bit kept), so that an infinity in V meets positive factors
 // only: a 0 or a negative one would make NaN of it.

@@ -606,7 +606,7 @@ int mq_attention_impl(const void* q, int64_t q_stride_t, int64_t q_stride_h,
   DSP_HOST_CHECK(dsp_is_pow2(block_size), DSP_EINVAL);
   DSP_HOST_CHECK(bt_stride * block_size >= max_ctx, DSP_EINVAL);
   // 256-wide 16-bit heads run on the same tiles where the 16-byte vectors they load are
-  // aligned (4 x 200-token chunks of 16 heads over ~2000 keys: 85 us a layer, 13.1 ms on the
+  // aligned (4 x 200-token chunks of 16 heads over ~2000 keys: 103 us a layer, 13.1 ms on the
   // generic kernel, which re-reads the keys for every row and head); the generic kernel, which
   // needs element alignment only, keeps the rest.
   const bool wide = D == 256 && dtype != DSP_F32 && prefix_tokens == 0 &&

@@ -575,10 +575,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D > 12
 // workspace: slot 2w for worker w's first piece when it continues a tile, 2w + 1 for its last
 // when it begins one; the merge kernel's workgroup w folds the tile that worker w began.
 // Verifies of 17 to 127 rows, whose 16-row tiles would each read the keys: 32 of 5 over 500-4000
-// keys 86 -> 41 us (28 heads over 4).
-// 24 decodes of 100-2860 keys beside a 700-token chunk over 1501 keys: 118 -> 55 us a layer with
-// the merge (28 heads over 4 of 128), 52 -> 32 (14 over 2 of 64), 151 -> 70 (32 over 8).  The
-// merge is 8-12 us of it: a partial is 64 KiB a tile at D 128.
+// keys 93 -> 48 us (28 heads over 4).
+// 24 decodes of 100-2860 keys beside a 700-token chunk over 1501 keys: 117 -> 58 us a layer with
+// the merge (28 heads over 4 of 128), 46 -> 31 (14 over 2 of 64), 150 -> 71 (32 over 8).  The
+// merge is 8-13 us of it: a partial is 64 KiB a tile at D 128.
 constexpr int kMinChunks = 2;       // a worker gets at least this many chunks
 // Run ends this many chunks from a tile's end or less move onto it: 2 decodes and a 1000-token
 // prompt 45 -> 41 us at 2, 42 at 4, where batches of short contexts lose (4 decodes and 64

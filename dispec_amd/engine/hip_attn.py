@@ -64,8 +64,8 @@ def _prefer_ragged(T, B, KVH, G, D, max_q_len, max_ctx) -> bool:
       decodes (one of 46 beside 66, 16 over 8: 101 / 163), unless contexts reach 6144 tokens;
     * heads are at most 128 wide (below 12288 tokens: 256-wide verifies lost every second time).
     Of the batches checked, 1.9 times as fast at the median; 1 in 80 slower by more than 3 %, 1 in
-    160 by more than 10 %.  (28 heads over 4, 32 verifies of 5 over 500-4000 keys 86 / 41; 32 over
-    8, 24 of 5 95 / 57.)
+    160 by more than 10 %.  (28 heads over 4, 32 verifies of 5 over 500-4000 keys 93 / 48; 32 over
+    8, 24 of 5 92 / 48.)
 
     Longer blocks.  The grid has at least 256 tiles and several times those that the T query tokens
     can fill, and
@@ -76,7 +76,7 @@ def _prefer_ragged(T, B, KVH, G, D, max_q_len, max_ctx) -> bool:
       a 148-token chunk, 32 over 8: 52 / 93), the grid has to be 9 or 14 times too large; elsewhere,
       and for heads wider than 128, 5 times; 3 times from 8192 tokens on.
     Of the batches checked, 2.8 times as fast at the median; 1 in 100 slower by more than 3 %, 1 in
-    200 by more than 10 %.  (24 decodes and a 700-token chunk, 28 over 4: 118 / 56.)"""
+    200 by more than 10 %.  (24 decodes and a 700-token chunk, 28 over 4: 117 / 58.)"""
     workers = _ragged_ws_bytes(B, KVH * G, KVH, D, max_q_len, max_ctx) // (4 * (256 * (D + 2) + 4))
     if not workers:
         return False

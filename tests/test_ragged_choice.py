@@ -38,12 +38,12 @@ SLOWER = [
     ((16, 8, 256), [(32, 10)], 1500, "every second one"),
 ]
 FASTER = [
-    ((28, 4, 128), [(24, 1), (1, 700)], 2864, "118 / 56"),
-    ((14, 2, 64), [(24, 1), (1, 700)], 3008, "52 / 36"),
-    ((32, 8, 128), [(30, 1), (2, 1000)], 3008, "605 / 165"),
-    ((28, 4, 128), [(32, 5)], 4000, "86 / 41"),
-    ((12, 2, 128), [(64, 6)], 4000, "83 / 40"),
-    ((32, 8, 128), [(24, 5)], 4000, "95 / 57"),
+    ((28, 4, 128), [(24, 1), (1, 700)], 2864, "117 / 58"),
+    ((14, 2, 64), [(24, 1), (1, 700)], 3008, "46 / 31"),
+    ((32, 8, 128), [(30, 1), (2, 1000)], 3008, "318 / 114"),
+    ((28, 4, 128), [(32, 5)], 4000, "93 / 48"),
+    ((12, 2, 128), [(64, 6)], 4000, "87 / 47"),
+    ((32, 8, 128), [(24, 5)], 4000, "92 / 48"),
 ]
 
 
